@@ -235,7 +235,10 @@ int hpcgx_problem_info(const hpcgx_problem *p, int level, hpcgx_level_info *info
 }
 
 double hpcgx_optimize_problem_memory_use(const hpcgx_problem *p) {
-  return p ? p->P.arena.bytes : 0.0;
+  if (!p) return 0.0;
+  double b = p->P.arena.bytes;
+  for (int l = 0; l < p->P.nlevels; ++l) b += p->P.L[l].lex.mem.bytes;
+  return b;
 }
 
 int hpcgx_problem_vectors(hpcgx_problem *p, double *b, double *x, double *xexact,
@@ -280,6 +283,7 @@ int hpcgx_replace_diagonal(hpcgx_problem *p, int level, const double *diag, void
     hpcgx::Level &L = level_of(p, level);
     hpcgx::launch_replace_diag(L, diag, S(stream));
     hpcgx::replace_diag32(L, diag, S(stream));
+    hpcgx::lex_replace_diag(L, diag, S(stream));
   });
 }
 
@@ -426,6 +430,10 @@ int hpcgx_tune(hpcgx_problem *p, const char *key, double value) {
     }
     if (k == "resid_fused") {
       P.resid_fused = value != 0.0;
+      return;
+    }
+    if (k == "lex_panels") {
+      P.use_lex = value != 0.0;
       return;
     }
     if (k == "hc_pairs") {

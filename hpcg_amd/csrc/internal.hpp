@@ -102,9 +102,45 @@ struct DeviceArena {
         return;
       }
   }
-  ~DeviceArena() {
+  void clear() {
     for (void *p : ptrs)
       if (p) (void)hipFree(p);
+    ptrs.clear();
+    bytes = 0.0;
+  }
+  ~DeviceArena() { clear(); }
+};
+
+// A level's copy in the order of its reference-order sweeps (lex.hip), built
+// at the first such sweep.  One LexRec per wavefront and step: rows
+// [start, start + cnt) of the copy; the steps its panel's neighbour must have
+// finished first ([0] forward, [1] backward sweep); slot j's column of row q
+// is base[j] / 8 + q (byte offsets of x), or, with general set, LexPlan::col's.
+struct LexRec {
+  int32_t start, cnt;
+  int32_t need[2];
+  uint32_t general;
+  uint32_t base[kSlots];
+};
+static_assert(sizeof(LexRec) == 128, "one cache line");
+struct LexPlan {
+  bool tried = false, ready = false;
+  int npanels = 0, waves = 0;
+  int64_t nrec = 0, nprog = 0;
+  LexRec *recs = nullptr;     // [steps][waves]
+  int32_t *sptr = nullptr;    // [npanels + 1] steps of a panel
+  int64_t *pstart = nullptr;  // [npanels + 1] rows of a panel
+  int32_t *row = nullptr;     // [n] device row of a position
+  int32_t *pos = nullptr;     // [n] position of a device row
+  double *val = nullptr;      // [28 n] chunk by chunk, two slots side by side; then the diagonal
+  int32_t *col = nullptr;     // [27 n] positions
+  int32_t *dpos = nullptr;    // [n] slot of the diagonal
+  double *x = nullptr, *r = nullptr;  // [n] x and r in this order
+  unsigned *prog = nullptr;   // ticket and progress counters, forward then backward
+  hipEvent_t done = nullptr;  // the last sweep's end (its scratch is free again)
+  DeviceArena mem;
+  ~LexPlan() {
+    if (done) (void)hipEventDestroy(done);
   }
 };
 
@@ -207,6 +243,7 @@ struct Level {
   int32_t *ftile = nullptr;  // per kTile transfer rows: fine row / kTile
   int32_t *rperm = nullptr;
   double *rc = nullptr, *xc = nullptr;  // next level's residual and correction
+  LexPlan lex;
 };
 
 struct Problem {
@@ -252,6 +289,8 @@ struct Problem {
   // non-temporal multivector loads and stores in the block CG's vector
   // kernels ("block_nt")
   bool block_nt = true;
+  // reference-order FP64 sweeps by panels of rows (lex.hip; "lex_panels")
+  bool use_lex = true;
   // block PCG finest colour steps: slot 3m + 2's x rows from slot 3m's by
   // W-lane moves on affine tiles ("block_pairs")
   bool block_pairs = false;
@@ -407,6 +446,10 @@ void launch_spmv(const Problem &P, const Level &L, const double *x, double *y,
 // path only).
 void launch_symgs_rows(const Problem &P, const Level &L, int64_t begin, int64_t end,
                        const double *r, double *x, hipStream_t s, double *dpart = nullptr);
+// Reference-order symmetric sweep by panels (lex.hip); false (nothing
+// launched) where it does not apply.
+bool launch_symgs_lex(Problem &P, int l, const double *r, double *x, hipStream_t s);
+void lex_replace_diag(Level &L, const double *d, hipStream_t s);
 void launch_symgs_list(const Level &L, const int32_t *rows, int64_t count,
                        const double *r, double *x, hipStream_t s);
 // The colour step of a forward sweep whose x was zero when the sweep began
@@ -510,6 +553,11 @@ void link_levels(Problem &P, int l, const NaturalLevel &Nf, hipStream_t s);
 void build_wave(Problem &P, Level &L, int slab_factor, int rows, hipStream_t s);
 void build_chunks(Problem &P, Level &L, bool interleave);
 void drop_wave(Problem &P, Level &L);
+// Stable sort of row ids by a small non-negative integer key (< nbins):
+// rows_out = rows ordered by (key, row); returns the bin pointers
+// ptr[0..nbins], bin k owning rows_out[ptr[k] .. ptr[k+1]).
+std::vector<int64_t> sort_rows_by_key(int64_t n, const int32_t *key, int nbins,
+                                      int32_t *rows_out, hipStream_t s);
 void problem_vectors(const Problem &P, double *b, double *x, double *xexact,
                      hipStream_t s);
 // The grids level l's rows come from (empty when unknown).

@@ -1,0 +1,699 @@
+// lex.hip -- the reference-order (lexicographic) Gauss-Seidel sweeps as two
+// launches per symmetric sweep.
+//
+// The level schedule (rows of hyperplane s of the dependency DAG depend only
+// on lower hyperplanes) run as one launch per hyperplane is bound by the
+// launches and by memory latency: at 256^3 a V-cycle is 13400 launches of a
+// few thousand rows each, whose entries lie scattered over the colour-ordered
+// ELL (one 64-byte sector per 8-byte value): 438 ms.
+//
+// Here natural rows are cut into panels of consecutive rows (one grid plane,
+// or as many rows as the matrix is wide), so that a row couples only to its
+// own panel and the two next to it.  One workgroup owns one panel and walks
+// its hyperplanes in order, with a workgroup barrier between them; it waits
+// for the panel before it (after it in the backward sweep) only until that
+// panel has finished the lower (higher) hyperplanes.  That wait goes one way,
+// so the panels form a pipeline: the cross-workgroup latency is paid once per
+// panel, not once per hyperplane.  In the forward sweep a row of hyperplane s
+// reads updated x only from rows of lower hyperplanes, all of them finished,
+// and old x only from rows of higher ones, which wait for it (the pattern is
+// symmetric); the backward sweep mirrors this.  So every row meets exactly
+// the values the sequential sweep gives it.
+//
+// The matrix is copied once into that order (LexPlan): rows by panel,
+// hyperplane and natural row; entries of a chunk of at most 64 rows (one
+// wavefront) stored slot by slot, the chunk's slots aligned by natural column
+// offset, so that both the stored entries and the gathered x of a wavefront
+// are consecutive.  x and r are permuted into the same order for the sweep.
+//
+// Measured (MI355X, one V-cycle in reference order): 256^3 439.2 -> 23.9 ms,
+// 64x48x32 21.7 -> 2.56 ms.  What bounds it now is the chain of hyperplanes:
+// about 1.1 us a step (one wavefront a panel) to 1.5 us (two), for gathers
+// behind the barrier, 27 dependent subtractions and a division, over
+// (hyperplanes of a panel) + 7 (panels - 1) steps: each panel starts four
+// hyperplanes, two steps of publishing and one of look-ahead after the last.
+// Joining several planes into one panel (fewer hops, more wavefronts sharing a
+// CU's L1) measured slower, 30 ms (two planes) and 33 ms (four) against 24.5
+// at 256^3, as did matrix loads two or three steps ahead instead of one
+// (24.5 against 23.8 ms; the 63 loads a wavefront may have in flight cap it).
+#include <algorithm>
+#include <climits>
+
+#include "internal.hpp"
+
+namespace hpcgx {
+namespace {
+
+constexpr int kLexWaves = 4;               // wavefronts per workgroup, at most
+constexpr int kLexPad = 32;                // progress counters 128 bytes apart
+constexpr unsigned kLexSpins = 1u << 22;   // polls before a wait gives up (seconds)
+constexpr int64_t kLexRows = 256;          // see build_lex
+constexpr int kLexAhead = 1;               // steps the matrix loads run ahead
+constexpr int kLexIn = 4, kLexOut = 9;     // slots of the own and of a neighbour panel
+static_assert(2 * kLexOut + 2 * kLexIn + 1 == kSlots, "slot groups");
+constexpr int kLexStore = kSlots + 1;      // values stored per row
+constexpr int kLexEdge = 64;               // rows of 0 before and after the copy of x
+constexpr int kLexRing = 2048;             // fresh x values held in LDS
+constexpr int kLexReach = kLexRing - 64 * kLexWaves - 64;  // furthest fresh row
+
+inline unsigned grid_for(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
+__device__ inline int64_t gtid() { return (int64_t)blockIdx.x * blockDim.x + threadIdx.x; }
+
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+
+template <bool STREAM, class T>
+__device__ inline T mload(const T *p) {
+  if (STREAM) return __builtin_nontemporal_load(p);
+  return *p;
+}
+// x of another workgroup's rows: device-coherent, as in the wavefront sweep
+// (kernels.hip): served past the per-XCD L2.
+__device__ inline double xload(const double *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void xstore(double *p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline unsigned pload(const unsigned *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// key[natural row] = panel * nsched + hyperplane; panel p holds the natural
+// rows [bound[p], bound[p + 1])
+__global__ __launch_bounds__(kBlock) void k_lex_key(int64_t n, int nsched, int npanels,
+                                                    const int64_t *__restrict__ bound,
+                                                    const int64_t *__restrict__ level_ptr,
+                                                    const int32_t *__restrict__ level_rows,
+                                                    const int32_t *__restrict__ iperm,
+                                                    int32_t *__restrict__ key) {
+  const int64_t k = gtid();
+  if (k >= n) return;
+  int lo = 0, hi = nsched - 1;  // last hyperplane with level_ptr <= k
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) / 2;
+    if (level_ptr[mid] <= k) lo = mid; else hi = mid - 1;
+  }
+  const int64_t g = iperm[level_rows[k]];
+  int a = 0, b = npanels - 1;
+  while (a < b) {
+    const int mid = (a + b + 1) / 2;
+    if (bound[mid] <= g) a = mid; else b = mid - 1;
+  }
+  key[g] = a * nsched + lo;
+}
+
+// row[k] = device row of position k, pos[device row] = k
+__global__ __launch_bounds__(kBlock) void k_lex_rows(int64_t n, const int32_t *__restrict__ order,
+                                                     const int32_t *__restrict__ perm,
+                                                     int32_t *__restrict__ row,
+                                                     int32_t *__restrict__ pos) {
+  const int64_t k = gtid();
+  if (k >= n) return;
+  const int32_t i = perm[order[k]];
+  row[k] = i;
+  pos[i] = (int32_t)k;
+}
+
+__device__ inline int wave_min(int v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
+  return v;
+}
+
+// Slot j of row q of a chunk of cnt rows from `start`: two slots side by side
+// per row (16-byte loads), the diagonal again in slot kSlots.
+__device__ inline int64_t lex_at(int32_t start, int cnt, int j, int q) {
+  return (int64_t)start * kLexStore + ((int64_t)(j / 2) * cnt + q) * 2 + j % 2;
+}
+
+__device__ inline int wave_max(int v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
+  return v;
+}
+
+// Copies one chunk's rows (one wavefront).  Where it can, the chunk's slots
+// are aligned by natural column offset (repeated wavefront minimum of each
+// row's next offset, as k_tile_layout does) into five groups that keep the
+// ascending order: kLexOut slots for the panel before, kLexIn for lower rows
+// of its own panel, the diagonal, kLexIn for upper rows, kLexOut for the panel
+// after; a slot's column must be one base plus the row's place in the chunk
+// (rows of a hyperplane and their neighbours are consecutive in this order).  A row without the slot's offset gets the value 0 there.  Chunks
+// that do not fit (offsets that do not ascend, stored zeros, more offsets or
+// other couplings, rows further back than the ring of fresh x holds) keep the
+// device slots and 32-bit columns.  *bad is set when a column lies further
+// away than the next panel.
+__global__ __launch_bounds__(kBlock) void k_lex_fill(
+    int64_t nrec, int64_t n, LexRec *recs, const int32_t *__restrict__ panel_of,
+    const int64_t *__restrict__ pstart, int npanels, const int32_t *__restrict__ row,
+    const int32_t *__restrict__ pos, const int32_t *__restrict__ iperm,
+    const int32_t *__restrict__ col, const double *__restrict__ val,
+    const double *__restrict__ diag, const uint8_t *__restrict__ nnz_row,
+    double *__restrict__ lval, int32_t *__restrict__ lcol, int32_t *__restrict__ ldpos,
+    int *bad) {
+  const int64_t q = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  if (q >= nrec) return;  // whole wavefronts
+  const int cnt = recs[q].cnt;
+  const int lane = threadIdx.x & 63;
+  const int32_t start = recs[q].start;
+  if (lane < kSlots) recs[q].base[lane] = (uint32_t)(start + kLexEdge) << 3;
+  if (cnt == 0) return;
+  const int pn = panel_of[q];
+  const int32_t pb = (int32_t)pstart[pn], pe = (int32_t)pstart[pn + 1];
+  const int32_t lo = pn > 0 ? (int32_t)pstart[pn - 1] : pb;
+  const int32_t hi = pn + 1 < npanels ? (int32_t)pstart[pn + 2] : pe;
+  const bool live = lane < cnt;
+  const int32_t k = start + (live ? lane : 0);
+  const int64_t i = row[k];
+  const int32_t g = iperm[i];
+  const int64_t at0 = (int64_t)start * kSlots + lane;
+  // the row's entries, in slot order: ascending offsets and no stored zeros?
+  int m = 0, last = INT_MIN, ds = 0;
+  bool plain = true, far = false;
+  for (int j = 0; j < kSlots; ++j) {
+    if (val[(int64_t)j * n + i] == 0.0) continue;
+    const int32_t cd = col[(int64_t)j * n + i];
+    const int o = iperm[cd] - g;
+    const int32_t c = pos[cd];
+    plain = plain && (m == 0 || o > last);
+    far = far || c < lo || c >= hi;
+    last = o;
+    ++m;
+  }
+  if (live && far) atomicOr(bad, 1);
+  plain = plain && m == nnz_row[i];
+  bool fits = __ballot(live && !plain) == 0ull;
+  // two passes over the chunk's distinct offsets: count each group's, then
+  // place them
+  const int first[6] = {0, kLexOut, kLexOut + kLexIn, kLexOut + kLexIn + 1,
+                        kLexOut + 2 * kLexIn + 1, kSlots};
+  int used[5] = {0, 0, 0, 0, 0}, place[5];
+  if (fits && live)
+    for (int u = 0; u < kSlots; ++u) lval[lex_at(start, cnt, u, lane)] = 0.0;
+  for (int pass = 0; pass < 2 && fits; ++pass) {
+    int e = 0;
+    for (;;) {
+      while (e < kSlots && val[(int64_t)e * n + i] == 0.0) ++e;
+      const int32_t cd = e < kSlots ? col[(int64_t)e * n + i] : 0;
+      const int head = live && e < kSlots ? iperm[cd] - g : INT_MAX;
+      const int mn = wave_min(head);
+      if (mn == INT_MAX) break;
+      const bool has = head == mn;
+      const int32_t c = has ? pos[cd] : 0;
+      const int grp = !has ? 0 : c < pb ? 0 : c >= pe ? 4 : c < k ? 1 : c > k ? 3 : 2;
+      // one group and one base for all rows that have the offset; fresh x of
+      // the own panel (groups 1 and 3) near enough for the ring
+      const int g0 = wave_min(has ? grp : INT_MAX), g1 = wave_max(has ? grp : INT_MIN);
+      const int b0 = wave_min(has ? c - lane : INT_MAX), b1 = wave_max(has ? c - lane : INT_MIN);
+      const int away = wave_max(has && (grp == 1 || grp == 3) ? abs(c - k) : 0);
+      fits = g0 == g1 && b0 == b1 && away <= kLexReach;
+      if (!fits) break;
+      if (pass == 0) {
+        ++used[g0];
+      } else {
+        const int slot = place[g0]++;
+        if (has) {
+          lval[lex_at(start, cnt, slot, lane)] = val[(int64_t)e * n + i];
+          if (grp == 2) ds = slot;
+        }
+        if (lane == 0) recs[q].base[slot] = (uint32_t)(b0 + kLexEdge) << 3;
+      }
+      if (has) ++e;
+    }
+    if (pass == 0 && fits) {
+      for (int u = 0; u < 5; ++u) {
+        place[u] = first[u];
+        fits = fits && used[u] <= first[u + 1] - first[u];
+      }
+    }
+  }
+  if (!fits && live) {
+    for (int u = 0; u < kSlots; ++u) {
+      const double v = val[(int64_t)u * n + i];
+      int32_t c = pos[col[(int64_t)u * n + i]];
+      // an unused slot's column need not be near: the row's own x there
+      if (v == 0.0 && (c < lo || c >= hi)) c = k;
+      if (c == k && v != 0.0) ds = u;
+      lval[lex_at(start, cnt, u, lane)] = v;
+      lcol[at0 + (int64_t)u * cnt] = c;
+    }
+  }
+  if (live) {
+    lval[lex_at(start, cnt, kSlots, lane)] = diag[i];
+    ldpos[k] = ds;
+  }
+  if (lane == 0) recs[q].general = fits ? 0u : 1u;
+}
+
+// A new diagonal (device order) into the copy: slot ldpos of each row and the
+// diagonal's own.
+__global__ __launch_bounds__(kBlock) void k_lex_diag(int64_t nrec,
+                                                     const LexRec *__restrict__ recs,
+                                                     const int32_t *__restrict__ row,
+                                                     const int32_t *__restrict__ ldpos,
+                                                     const double *__restrict__ d, double *lval) {
+  const int64_t q = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  if (q >= nrec) return;
+  const int lane = threadIdx.x & 63, cnt = recs[q].cnt;
+  if (lane >= cnt) return;
+  const int32_t start = recs[q].start, k = start + lane;
+  const double v = d[row[k]];
+  lval[lex_at(start, cnt, ldpos[k], lane)] = v;
+  lval[lex_at(start, cnt, kSlots, lane)] = v;
+}
+
+__global__ __launch_bounds__(kBlock) void k_lex_zero(int64_t n, double *x) {
+  const int64_t i = gtid();
+  if (i < n) x[i] = 0.0;
+}
+
+// x and r into the sweep's order; clears both sweeps' progress counters.
+__global__ __launch_bounds__(kBlock) void k_lex_in(int64_t n, const int32_t *__restrict__ row,
+                                                   const double *__restrict__ r,
+                                                   const double *__restrict__ x,
+                                                   double *__restrict__ lr,
+                                                   double *__restrict__ lx, unsigned *prog,
+                                                   int64_t nprog) {
+  const int64_t k = gtid();
+  if (k < nprog) prog[k] = 0u;
+  if (k >= n) return;
+  const int32_t i = row[k];
+  lr[k] = r[i];
+  lx[k] = x[i];
+}
+
+__global__ __launch_bounds__(kBlock) void k_lex_out(int64_t n, const int32_t *__restrict__ pos,
+                                                    const double *__restrict__ lx,
+                                                    double *__restrict__ x) {
+  const int64_t i = gtid();
+  if (i < n) x[i] = lx[pos[i]];
+}
+
+// One sweep direction.  Workgroup order comes from a ticket, so a workgroup
+// only ever waits for panels whose workgroups have already started; a wait
+// that exceeds kLexSpins polls sets *err and gives up, as all later ones do,
+// and the sweep ends with wrong values instead of hanging.
+//
+// A step's loads run ahead of it, so that between two barriers only the chain
+// through the rows just finished remains: values, right-hand side, diagonal
+// and old x kLexAhead steps ahead; x of the other panels and of rows not yet
+// reached (neither changes before the step) one step ahead, after the wait
+// for the neighbour panel; x of the own panel's fresh rows from a ring in LDS.
+//
+// Progress: counter p holds the steps of panel p whose x stores have
+// completed.  Vector memory operations of a wavefront complete in order.  Its
+// stores of step k are followed by the gathers for step k + 2, so once step
+// k + 2 has used those, the stores have been acknowledged; after the barrier
+// that ends step k + 2 this holds for every wavefront and step k is
+// published: no wait for a store stands in the chain of steps.
+template <bool STREAM, int DIR>
+__global__ __launch_bounds__(64 * kLexWaves) void k_lex_sweep(
+    int npanels, int waves, const LexRec *__restrict__ recs, const int32_t *__restrict__ sptr,
+    const int64_t *__restrict__ pstart, const double *__restrict__ lval,
+    const int32_t *__restrict__ lcol, const double *__restrict__ r, double *x, unsigned *prog,
+    int *err) {
+  __shared__ double ring[kLexRing];
+  __shared__ int s_ticket;
+  // rows without an entry in a fresh slot read the ring too (times 0)
+  for (int k = threadIdx.x; k < kLexRing; k += blockDim.x) ring[k] = 0.0;
+  if (threadIdx.x == 0) s_ticket = (int)atomicAdd(prog, 1u);
+  __syncthreads();
+  const int q = __builtin_amdgcn_readfirstlane(s_ticket);
+  if (q >= npanels) return;
+  const int p = DIR == 0 ? q : npanels - 1 - q;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t lane = threadIdx.x & 63, lane8 = lane * 8u;
+  const int s0 = sptr[p], nsteps = sptr[p + 1] - s0;
+  const uint32_t pb = ((uint32_t)pstart[p] + kLexEdge) << 3,
+                 pe = ((uint32_t)pstart[p + 1] + kLexEdge) << 3;
+  unsigned *mine = prog + (int64_t)(1 + p) * kLexPad;
+  const unsigned *nbr = q > 0 ? (DIR == 0 ? mine - kLexPad : mine + kLexPad) : mine;
+  unsigned seen = q > 0 ? 0u : ~0u;
+
+  struct Mat { f64x2 v[kLexStore / 2]; double r, o; };  // values and diagonal; b, old x
+  struct Gat { double x[kSlots]; uint32_t f[kLexIn], general; };  // x by slot; ring offsets
+  constexpr int kFresh = DIR == 0 ? kLexOut : kLexOut + kLexIn + 1;  // first fresh slot
+  constexpr int kDiag = kLexOut + kLexIn;
+  constexpr int kOther = DIR == 0 ? 0 : kSlots - kLexOut;  // first slot of the neighbour panel
+  // byte offsets of x count from kLexEdge rows before its first
+  auto xat = [&](uint32_t off) {
+    return reinterpret_cast<double *>(reinterpret_cast<char *>(x - kLexEdge) + off);
+  };
+  auto rec = [&](int k) -> const LexRec & {  // step k of the sweep, this wavefront's chunk
+    const int kk = k < nsteps ? k : nsteps - 1;
+    const int st = DIR == 0 ? s0 + kk : s0 + nsteps - 1 - kk;
+    return recs[(int64_t)st * waves + w];
+  };
+  // rows of a step: first row and their number, read kLexAhead + 2 steps ahead
+  // (with both ends of the record, so that all of it is in the scalar cache
+  // when the gathers need it)
+  struct Span { int start, cnt; uint32_t tail; };
+  auto span = [&](int k) {
+    const LexRec &C = rec(k);
+    return Span{C.start, k < nsteps ? C.cnt : 0, C.base[kSlots - 1]};
+  };
+  // Loads are issued whether or not the wavefront has rows in the step (from
+  // rows it may read): a load under a condition would make every later wait
+  // count on its absence.
+  auto lane_of = [&](const Span &S) { return min(lane, (uint32_t)max(S.cnt, 1) - 1u); };
+  auto load = [&](Mat &M, const Span &S) {
+    const uint32_t ln = lane_of(S);
+    const f64x2 *vp = reinterpret_cast<const f64x2 *>(lval + (int64_t)S.start * kLexStore);
+#pragma unroll
+    for (int j = 0; j < kLexStore / 2; ++j) {
+      M.v[j] = mload<STREAM>(vp + ln);
+      vp += S.cnt;
+    }
+    M.r = (r + S.start)[ln];
+    M.o = (x + S.start)[ln];
+  };
+  unsigned polled = 0;  // progress of the neighbour, asked for a step earlier
+  // x of step k that is not fresh, after the wait for the neighbour panel
+  auto gather = [&](Gat &G, const Span &S, int k) {
+    const LexRec &C = rec(k);
+    const unsigned need = (unsigned)C.need[DIR];
+    if (seen < need) {
+      seen = max(seen, (unsigned)__builtin_amdgcn_readfirstlane(polled));
+      unsigned spins = 0;
+      while (seen < need) {
+        seen = __builtin_amdgcn_readfirstlane(pload(nbr));
+        if (++spins > kLexSpins ||
+            ((spins & 1023u) == 0u &&
+             __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+          if (lane == 0) atomicOr(err, 1);
+          seen = ~0u;
+        }
+      }
+    }
+    // x loads stay behind the poll (the compiler; the wavefront itself issues
+    // in order and the poll's branch holds it)
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    polled = pload(nbr);
+#pragma unroll
+    for (int j = 0; j < kSlots; ++j) {
+      const uint32_t off = (j == kSlots - 1 ? S.tail : C.base[j]) + lane8;
+      if (j >= kFresh && j < kFresh + kLexIn)
+        G.f[j - kFresh] = off & (kLexRing * 8u - 1u);
+      else if (j != kDiag)  // the diagonal slot takes the old x
+        G.x[j] = j >= kOther && j < kOther + kLexOut ? xload(xat(off)) : *xat(off);
+    }
+    G.general = C.general;
+  };
+  auto finish = [&](const Span &S, double sum, double o, double d) {
+    sum += o * d;
+    const double z = sum / d;
+    if (lane < (uint32_t)S.cnt) {
+      ring[(S.start + kLexEdge + lane) & (kLexRing - 1)] = z;
+      xstore(x + S.start + lane, z);
+    }
+  };
+  auto step = [&](Mat &M, Gat &G, const Span &S) {
+    // a wavefront without rows in the step goes through it as well (and stores
+    // nothing): its earlier stores are acknowledged as the others' are
+    if (!G.general) {
+      double fresh[kLexIn];
+#pragma unroll
+      for (int j = 0; j < kLexIn; ++j)
+        fresh[j] = *reinterpret_cast<const double *>(reinterpret_cast<const char *>(ring) +
+                                                     G.f[j]);
+      double sum = M.r;
+#pragma unroll
+      for (int j = 0; j < kSlots; ++j)
+        sum -= M.v[j / 2][j % 2] * (j >= kFresh && j < kFresh + kLexIn ? fresh[j - kFresh]
+                         : j == kDiag                       ? M.o
+                                                            : G.x[j]);
+      finish(S, sum, M.o, M.v[kSlots / 2][1]);
+    } else {
+      const uint32_t ln = lane_of(S);
+      const int32_t *cp = lcol + (int64_t)S.start * kSlots;
+      double sum = (r + S.start)[ln];
+      uint32_t c[kSlots];
+#pragma unroll
+      for (int j = 0; j < kSlots; ++j) {
+        c[j] = ((uint32_t)cp[ln] + kLexEdge) << 3;
+        cp += S.cnt;
+      }
+#pragma unroll
+      for (int j = 0; j < kSlots; ++j) {
+        const bool other = DIR == 0 ? c[j] < pb : c[j] >= pe;
+        const double xc = other ? xload(xat(c[j])) : *xat(c[j]);
+        sum -= lval[lex_at(S.start, S.cnt, j, ln)] * xc;
+      }
+      finish(S, sum, (x + S.start)[ln], lval[lex_at(S.start, S.cnt, kSlots, ln)]);
+      __builtin_amdgcn_s_waitcnt(0);
+    }
+  };
+
+  Mat M[kLexAhead + 1];
+  Gat G[2];
+  Span S[kLexAhead + 2];  // of steps k .. k + kLexAhead + 1
+#pragma unroll
+  for (int a = 0; a < kLexAhead + 2; ++a) S[a] = span(a);
+#pragma unroll
+  for (int a = 0; a < kLexAhead; ++a) load(M[a], S[a]);
+  gather(G[0], S[0], 0);
+  constexpr int kUnroll = 2 * (kLexAhead + 1);
+  for (int k = 0; k < nsteps; k += kUnroll) {
+#pragma unroll
+    for (int a = 0; a < kUnroll; ++a) {
+      if (k + a >= nsteps) break;
+      load(M[(a + kLexAhead) % (kLexAhead + 1)], S[kLexAhead]);
+      gather(G[(a + 1) & 1], S[1], k + a + 1);
+      const Span next = span(k + a + kLexAhead + 2);
+      step(M[a % (kLexAhead + 1)], G[a & 1], S[0]);
+      __syncthreads();
+      if (threadIdx.x == 0 && k + a >= 2)
+        __hip_atomic_store(mine, (unsigned)(k + a - 1), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int b = 0; b < kLexAhead + 1; ++b) S[b] = S[b + 1];
+      S[kLexAhead + 1] = next;
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // this wavefront's x stores are complete
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(mine, (unsigned)nsteps, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+struct Buf {  // device buffer freed on scope exit
+  void *p = nullptr;
+  explicit Buf(size_t bytes) { HPCGX_HIP(hipMalloc(&p, bytes ? bytes : 1)); }
+  ~Buf() { (void)hipFree(p); }
+  template <class T> T *as() const { return static_cast<T *>(p); }
+};
+
+// The plan with panels of natural rows [bound[p], bound[p + 1]); false when
+// some row couples further than to the next panel.
+bool try_lex(Problem &P, Level &L, LexPlan &X, const std::vector<int64_t> &bound,
+             hipStream_t s) {
+  const int64_t n = L.n;
+  const int64_t np = (int64_t)bound.size() - 1;
+  if (np * L.nsched >= (int64_t)1 << 30) return false;
+  std::vector<int64_t> kp;  // positions of (panel, hyperplane) keys
+  X.row = X.mem.alloc<int32_t>(n);
+  X.pos = X.mem.alloc<int32_t>(n);
+  {
+    Buf key(sizeof(int32_t) * n), order(sizeof(int32_t) * n),
+        lptr(sizeof(int64_t) * (L.nsched + 1)), bnd(sizeof(int64_t) * bound.size());
+    HPCGX_HIP(hipMemcpyAsync(bnd.p, bound.data(), sizeof(int64_t) * bound.size(),
+                             hipMemcpyHostToDevice, s));
+    HPCGX_HIP(hipMemcpyAsync(lptr.p, L.level_ptr.data(), sizeof(int64_t) * (L.nsched + 1),
+                             hipMemcpyHostToDevice, s));
+    k_lex_key<<<grid_for(n), kBlock, 0, s>>>(n, L.nsched, (int)np, bnd.as<int64_t>(),
+                                             lptr.as<int64_t>(), L.level_rows, L.iperm,
+                                             key.as<int32_t>());
+    HPCGX_LAUNCHED();
+    kp = sort_rows_by_key(n, key.as<int32_t>(), (int)(np * L.nsched), order.as<int32_t>(), s);
+    k_lex_rows<<<grid_for(n), kBlock, 0, s>>>(n, order.as<int32_t>(), L.perm, X.row, X.pos);
+    HPCGX_LAUNCHED();
+    HPCGX_HIP(hipStreamSynchronize(s));
+  }
+  // steps: at most W chunks of one hyperplane of one panel
+  int64_t widest = 0;
+  for (size_t b = 0; b + 1 < kp.size(); ++b) widest = std::max(widest, kp[b + 1] - kp[b]);
+  const int W = (int)std::min<int64_t>(kLexWaves, (widest + 63) / 64);
+  std::vector<int32_t> sptr{0}, level, panel_of;
+  std::vector<int64_t> pstart;
+  std::vector<LexRec> recs;
+  for (int64_t p = 0; p < np; ++p) {
+    pstart.push_back(kp[p * L.nsched]);
+    for (int lv = 0; lv < L.nsched; ++lv) {
+      const int64_t e = kp[p * L.nsched + lv + 1];
+      for (int64_t b = kp[p * L.nsched + lv]; b < e;) {
+        level.push_back(lv);
+        for (int w = 0; w < W; ++w) {
+          LexRec r = {};
+          r.start = (int32_t)std::min<int64_t>(b, n - 1);
+          r.cnt = (int32_t)std::min<int64_t>(64, e - b);
+          b += r.cnt;
+          recs.push_back(r);
+          panel_of.push_back((int32_t)p);
+        }
+      }
+    }
+    sptr.push_back((int32_t)level.size());
+  }
+  pstart.push_back(n);
+  // steps of the panel before below a step's hyperplane, of the one after above it
+  for (int64_t p = 0; p < np; ++p) {
+    int64_t f = p > 0 ? sptr[p - 1] : 0, b = p + 1 < np ? sptr[p + 2] : 0;
+    for (int64_t st = sptr[p]; st < sptr[p + 1]; ++st) {
+      if (p > 0)
+        while (f < sptr[p] && level[f] < level[st]) ++f;
+      for (int w = 0; w < W; ++w) recs[st * W + w].need[0] = p > 0 ? (int32_t)(f - sptr[p - 1]) : 0;
+    }
+    for (int64_t st = (int64_t)sptr[p + 1] - 1; st >= sptr[p]; --st) {
+      if (p + 1 < np)
+        while (b > sptr[p + 1] && level[b - 1] > level[st]) --b;
+      for (int w = 0; w < W; ++w)
+        recs[st * W + w].need[1] = p + 1 < np ? (int32_t)(sptr[p + 2] - b) : 0;
+    }
+  }
+  X.npanels = (int)np;
+  X.waves = W;
+  X.nrec = (int64_t)recs.size();
+  X.recs = X.mem.alloc<LexRec>(recs.size());
+  X.sptr = X.mem.alloc<int32_t>(sptr.size());
+  X.pstart = X.mem.alloc<int64_t>(pstart.size());
+  X.val = X.mem.alloc<double>((size_t)kLexStore * n);
+  X.col = X.mem.alloc<int32_t>((size_t)kSlots * n);
+  X.dpos = X.mem.alloc<int32_t>(n);
+  X.x = X.mem.alloc<double>(n + 2 * kLexEdge) + kLexEdge;
+  k_lex_zero<<<grid_for(n + 2 * kLexEdge), kBlock, 0, s>>>(n + 2 * kLexEdge, X.x - kLexEdge);
+  HPCGX_LAUNCHED();
+  X.r = X.mem.alloc<double>(n);
+  X.nprog = (int64_t)kLexPad * (np + 1);
+  X.prog = X.mem.alloc<unsigned>(2 * X.nprog);
+  HPCGX_HIP(hipMemcpyAsync(X.recs, recs.data(), sizeof(LexRec) * recs.size(),
+                           hipMemcpyHostToDevice, s));
+  HPCGX_HIP(hipMemcpyAsync(X.sptr, sptr.data(), sizeof(int32_t) * sptr.size(),
+                           hipMemcpyHostToDevice, s));
+  HPCGX_HIP(hipMemcpyAsync(X.pstart, pstart.data(), sizeof(int64_t) * pstart.size(),
+                           hipMemcpyHostToDevice, s));
+  Buf pof(sizeof(int32_t) * panel_of.size()), bad(sizeof(int));
+  HPCGX_HIP(hipMemcpyAsync(pof.p, panel_of.data(), sizeof(int32_t) * panel_of.size(),
+                           hipMemcpyHostToDevice, s));
+  HPCGX_HIP(hipMemsetAsync(bad.p, 0, sizeof(int), s));
+  const int64_t wpb = kBlock / 64;
+  k_lex_fill<<<(unsigned)((X.nrec + wpb - 1) / wpb), kBlock, 0, s>>>(
+      X.nrec, n, X.recs, pof.as<int32_t>(), X.pstart, X.npanels, X.row, X.pos, L.iperm, L.col,
+      L.val, L.diag, L.nnz_row, X.val, X.col, X.dpos, bad.as<int>());
+  HPCGX_LAUNCHED();
+  int far = 0;
+  HPCGX_HIP(hipMemcpyAsync(&far, bad.p, sizeof far, hipMemcpyDeviceToHost, s));
+  HPCGX_HIP(hipStreamSynchronize(s));
+  return far == 0;
+}
+
+// Panels: the planes of the grids the rows come from, where known.  Else one
+// panel for the whole level where a hyperplane holds few rows on average
+// (kLexRows: one workgroup keeps up, and no wait crosses workgroups), or as
+// many rows as the matrix is wide.  Any choice is only used if every row is
+// found to couple to its neighbour panels at most; levels without one keep
+// one launch per hyperplane.
+void build_lex(Problem &P, int l, hipStream_t s) {
+  Level &L = P.L[l];
+  LexPlan &X = L.lex;
+  X.tried = true;
+  const int64_t n = L.n;
+  // a copy takes 27 * 12 + 32 bytes a row; at most half of what is free
+  size_t avail = 0, total = 0;
+  if (hipMemGetInfo(&avail, &total) != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
+  if ((double)n * (12.0 * kSlots + 48.0) > 0.5 * (double)avail) return;
+  std::vector<std::vector<int64_t>> tries;
+  std::vector<int64_t> planes{0};
+  for (const GridPart &g : grid_parts(P, l))
+    for (int z = 1; z <= g.nz; ++z) planes.push_back(g.off + (int64_t)g.nx * g.ny * z);
+  bool rising = planes.back() == n;
+  for (size_t k = 1; k < planes.size(); ++k) rising = rising && planes[k] > planes[k - 1];
+  if (rising) tries.push_back(planes);
+  if (n / std::max(1, L.nsched) <= kLexRows) {
+    tries.push_back({0, n});
+  } else if (L.bandwidth > 0 && 2 * L.bandwidth <= n) {
+    std::vector<int64_t> even;
+    for (int64_t b = 0; b < n; b += L.bandwidth) even.push_back(b);
+    even.push_back(n);
+    tries.push_back(even);
+  }
+  for (const auto &bound : tries) {
+    try {
+      if (try_lex(P, L, X, bound, s)) {
+        X.ready = true;
+        return;
+      }
+      X.mem.clear();
+    } catch (const std::exception &) {  // no room for the copy: one launch per hyperplane
+      (void)hipGetLastError();
+      X.mem.clear();
+      return;
+    }
+  }
+}
+
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
+}  // namespace
+
+bool launch_symgs_lex(Problem &P, int l, const double *r, double *x, hipStream_t s) {
+  Level &L = P.L[l];
+  LexPlan &X = L.lex;
+  if (!P.use_lex || L.n < 2 || L.n >= ((int64_t)1 << 29) - 2 * kLexEdge)
+    return false;
+  // Under a caller's capture the copy cannot be built, and its scratch would
+  // be used at replays this call cannot order; the problem's own captured
+  // iterations run inside calls that own the problem's vectors anyway.
+  const bool own = s && (s == P.graph.cap || s == P.fleet.graph.cap);
+  if (!own && capturing(s)) return false;
+  if (!X.tried && !own) build_lex(P, l, s);
+  if (!X.ready) return false;
+  // one scratch per level: a sweep on another stream follows the last one
+  if (!own) {
+    if (!X.done)
+      HPCGX_HIP(hipEventCreateWithFlags(&X.done, hipEventDisableTiming));
+    else
+      HPCGX_HIP(hipStreamWaitEvent(s, X.done, 0));
+  }
+  const int64_t n = L.n;
+  k_lex_in<<<grid_for(std::max(n, 2 * X.nprog)), kBlock, 0, s>>>(n, X.row, r, x, X.r, X.x, X.prog,
+                                                                 2 * X.nprog);
+  HPCGX_LAUNCHED();
+  const dim3 g(X.npanels), b(64 * X.waves);
+#define HPCGX_LEX(ST, DIR)                                                                       \
+  k_lex_sweep<ST, DIR><<<g, b, 0, s>>>(X.npanels, X.waves, X.recs, X.sptr, X.pstart, X.val,      \
+                                       X.col, X.r, X.x, X.prog + DIR * X.nprog, P.wave_err)
+  if (L.stream) {
+    HPCGX_LEX(true, 0);
+    HPCGX_LEX(true, 1);
+  } else {
+    HPCGX_LEX(false, 0);
+    HPCGX_LEX(false, 1);
+  }
+#undef HPCGX_LEX
+  HPCGX_LAUNCHED();
+  k_lex_out<<<grid_for(n), kBlock, 0, s>>>(n, X.pos, X.x, x);
+  HPCGX_LAUNCHED();
+  if (!own) HPCGX_HIP(hipEventRecord(X.done, s));
+  return true;
+}
+
+void lex_replace_diag(Level &L, const double *d, hipStream_t s) {
+  LexPlan &X = L.lex;
+  if (!X.ready) return;
+  const int64_t wpb = kBlock / 64;
+  k_lex_diag<<<(unsigned)((X.nrec + wpb - 1) / wpb), kBlock, 0, s>>>(X.nrec, X.recs, X.row, X.dpos,
+                                                                     d, X.val);
+  HPCGX_LAUNCHED();
+}
+
+}  // namespace hpcgx

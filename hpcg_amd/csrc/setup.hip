@@ -517,9 +517,8 @@ __global__ __launch_bounds__(kBlock) void k_colour_rank(int64_t n, const int32_t
   key[i] = rank.r[color[i]];
 }
 
-// Stable sort of row ids by a small non-negative integer key (< nbins):
-// rows_out = rows ordered by (key, row); returns the bin pointers
-// ptr[0..nbins], bin k owning rows_out[ptr[k] .. ptr[k+1]).
+}  // namespace
+
 std::vector<int64_t> sort_rows_by_key(int64_t n, const int32_t *key,
                                       int nbins, int32_t *rows_out,
                                       hipStream_t s) {
@@ -556,6 +555,8 @@ std::vector<int64_t> sort_rows_by_key(int64_t n, const int32_t *key,
   for (int b = nbins - 1; b >= 0; --b) ptr[b] = std::min(ptr[b], ptr[b + 1]);
   return ptr;
 }
+
+namespace {
 
 // tile_ptr[c*(S+1) + s] = first device row of colour c whose natural row is
 // >= s*W (binary search: a colour block lists its natural rows in order).

@@ -12,7 +12,8 @@ namespace hpcgx {
 // ComputeSYMGS_ref.cpp:67-100: forward sweep, then backward sweep.
 //  * lexicographic ordering: levels of the row DAG in increasing order, then
 //    in decreasing order; rows of a level are independent, so this is the
-//    reference's sequential sweep, row for row;
+//    reference's sequential sweep, row for row (by panels of rows, lex.hip;
+//    else one launch per level);
 //  * multicolour ordering: colours 0..C-1, then C-1..0.
 namespace {
 // Event pair around a launch on the finest level (hpcgx_kernel_timing), so
@@ -98,7 +99,7 @@ void symgs(Problem &P, int l, int ordering, const double *r, double *x,
       colour_step(P, L, c, r, x, s, rz ? rz + off : nullptr);
       off += rz_slots(L.color_ptr[c + 1] - L.color_ptr[c]);
     }
-  } else {
+  } else if (!launch_symgs_lex(P, l, r, x, s)) {
     for (int t = 0; t < L.nsched; ++t)
       launch_symgs_list(L, L.level_rows + L.level_ptr[t],
                         L.level_ptr[t + 1] - L.level_ptr[t], r, x, s);

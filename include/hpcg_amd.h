@@ -394,6 +394,13 @@ int hpcgx_cg_fleet(hpcgx_problem *p, int ordering, const double *b, double *x, i
  *                      and x values of colours already updated in that
  *                      sweep (default 1; the same x as a zero fill followed
  *                      by the full sweep)
+ *   "lex_panels"       1/0: FP64 sweeps in the reference's row order run as
+ *                      one launch per direction over panels of rows, from a
+ *                      copy of the level's matrix in that order built at
+ *                      the first such sweep (about 360 bytes a row; only
+ *                      where at most half of the free memory holds it), or
+ *                      one launch per hyperplane of the schedule
+ *                      (default 1; the same bits)
  *   "block_nt"         1/0: the block PCG's vector kernels (r.z, the p and
  *                      r updates) use non-temporal loads and stores on
  *                      multivectors of 2^24 or more values (default 1; the
