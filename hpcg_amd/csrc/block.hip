@@ -120,9 +120,6 @@ __device__ inline void block_finish_s(double v, int s, double *partials, unsigne
 // narrow column ids where the level has them).  A wavefront's rows lie in
 // one tile.  Per column the arithmetic is the single-vector kernels'
 // (mixed.hip, kernels.hip), term for term.
-__device__ inline int tile_of(int64_t i) {
-  return __builtin_amdgcn_readfirstlane((int)(i / kTile));
-}
 __device__ inline half_t vc_val(uint32_t w) {
   return __builtin_bit_cast(half_t, (uint16_t)(w & 0xffffu));
 }
@@ -167,9 +164,9 @@ template <bool STREAM, bool C16, class F>
 __device__ inline void slots32(const Col16 &C, const uint32_t *__restrict__ vc,
                                const int32_t *__restrict__ col,
                                const half_t *__restrict__ val16, int64_t n, int64_t i, F &&f) {
-  const int t = C16 ? tile_of(i) : 0;
-  if (C16 && C.info[t] != kTile32) {
-    const int32_t *__restrict__ base = C.tbase + (int64_t)t * kBaseStride;
+  const int t = C16 ? C.tile(i) : 0;
+  if (C16 && (C.flags(t) & 3u) != kTile32) {
+    const int32_t *__restrict__ base = C.bases(t);
 #pragma unroll
     for (int j = 0; j < kSlots; ++j) {
       const uint32_t w = mload<STREAM>(vc + (int64_t)j * n + i);
@@ -211,7 +208,7 @@ __device__ __attribute__((always_inline)) inline void bgs32_row(int64_t i, int o
 
 // ---- the first forward sweep of a block V-cycle level from X = 0 ----------
 // kernels.hip's zero-x colour step for W lanes per row: the slots that
-// Level::zmask leaves out of the tile, and the X rows at or beyond `begin`
+// kRecLive leaves out of the tile, and the X rows at or beyond `begin`
 // (colours not yet updated in this sweep), are read through buffer views
 // whose range check returns 0 without a memory access, so every row's loads
 // still go out together and X needs no fill.  Skipped terms are a * 0.
@@ -240,9 +237,9 @@ __device__ __attribute__((always_inline)) inline void bgs32_row_zero(
     const half_t *__restrict__ val16, const float *__restrict__ diag32,
     const float *__restrict__ R, float *X) {
   constexpr int V = 4;
-  const int t = tile_of(i);
-  const int64_t tb = (int64_t)t * kTile;
-  const uint32_t row = (uint32_t)(i - tb);
+  const int t = C.tile(i);
+  const uint32_t row = (uint32_t)C.place(i);
+  const int64_t tb = __builtin_amdgcn_readfirstlane((int)(i - row));
   const uint32_t xlim = (uint32_t)(begin * S * 4);
   float sum[V];
   ldv<V>(R + i * S + o, sum);
@@ -253,8 +250,8 @@ __device__ __attribute__((always_inline)) inline void bgs32_row_zero(
     sum[2] -= a * xv.z;
     sum[3] -= a * xv.w;
   };
-  if (C.info[t] != kTile32) {
-    const int32_t *__restrict__ base = C.tbase + (int64_t)t * kBaseStride;
+  if ((C.flags(t) & 3u) != kTile32) {
+    const int32_t *__restrict__ base = C.bases(t);
 #pragma unroll
     for (int j = 0; j < kSlots; ++j) {
       const bool live = (zm >> j) & 1u;
@@ -280,8 +277,8 @@ __device__ __attribute__((always_inline)) inline void bgs32_row_zero(
   stv<V>(X + i * S + o, sum);
 }
 
-// bgs32_row_zero over the live slots only (tune key "zero_live"): Level::
-// zmask's set bits in ascending slot order, CH per chunk, the chunk's
+// bgs32_row_zero over the live slots only (tune key "zero_live"): kRecLive's
+// set bits in ascending slot order, CH per chunk, the chunk's
 // unused entries read through empty views (0 * 0), so the loads of dead
 // slots are not issued.  NARROW: packed words (else 32-bit ids), decided
 // once per tile outside the loop.
@@ -290,7 +287,7 @@ __device__ __attribute__((always_inline)) inline void bzero_live_sum(
     uint32_t zm, int t, int64_t tb, uint32_t row, uint32_t xlim, int o, int64_t n,
     const Col16 &C, const uint32_t *__restrict__ vc, const int32_t *__restrict__ col,
     const half_t *__restrict__ val16, const float *X, float *sum) {
-  const int32_t *__restrict__ base = C.tbase + (int64_t)t * kBaseStride;
+  const int32_t *__restrict__ base = C.bases(t);
   uint32_t mm = zm;
   while (mm) {
     int js[CH];
@@ -341,22 +338,22 @@ __device__ __attribute__((always_inline)) inline void bzero_live_sum(
 
 template <bool STREAM, int S, int CH>
 __device__ __attribute__((always_inline)) inline void bgs32_row_zero_live(
-    uint32_t zm, int64_t begin, int64_t i, int o, int64_t n, const Col16 &C,
+    int64_t begin, int64_t i, int o, int64_t n, const Col16 &C,
     const uint32_t *__restrict__ vc, const int32_t *__restrict__ col,
     const half_t *__restrict__ val16, const float *__restrict__ diag32,
     const float *__restrict__ R, float *X) {
   constexpr int V = 4;
-  // a wavefront's 64 / W rows lie in one tile (begin is a multiple of
-  // kTile), so the tile and its mask are uniform: the slot loop runs on
-  // scalar registers
-  const int t = __builtin_amdgcn_readfirstlane(tile_of(i));
-  zm = __builtin_amdgcn_readfirstlane(zm);
-  const int64_t tb = (int64_t)t * kTile;
-  const uint32_t row = (uint32_t)(i - tb);
+  // a wavefront's 64 / W rows lie in one tile (begin is a colour's first
+  // row), so the tile and its mask are uniform: the slot loop runs on scalar
+  // registers
+  const int t = C.tile(i);
+  const uint32_t zm = C.live(t);
+  const uint32_t row = (uint32_t)C.place(i);
+  const int64_t tb = __builtin_amdgcn_readfirstlane((int)(i - row));
   const uint32_t xlim = (uint32_t)(begin * S * 4);
   float sum[V];
   ldv<V>(R + i * S + o, sum);
-  if (C.info[t] != kTile32)
+  if ((C.flags(t) & 3u) != kTile32)
     bzero_live_sum<STREAM, S, true, CH>(zm, t, tb, row, xlim, o, n, C, vc, col, val16, X, sum);
   else
     bzero_live_sum<STREAM, S, false, CH>(zm, t, tb, row, xlim, o, n, C, vc, col, val16, X, sum);
@@ -367,12 +364,11 @@ __device__ __attribute__((always_inline)) inline void bgs32_row_zero_live(
 }
 
 // A colour step of the first forward sweep from X = 0, rows [begin, end)
-// (begin a multiple of kTile).
+// (begin a colour's first row).
 // LIVE: the live slots only (bgs32_row_zero_live), else every slot (bgs32_row_zero)
 template <bool STREAM, int S, bool LIVE = false>
 __global__ __launch_bounds__(kBlock) void k_bgs32_rows_zero(
-    int64_t begin, int64_t end, int64_t n, Col16 C, const uint32_t *__restrict__ zmask,
-    const uint32_t *__restrict__ vc, const int32_t *__restrict__ col,
+    int64_t begin, int64_t end, int64_t n, Col16 C, const uint32_t *__restrict__ vc, const int32_t *__restrict__ col,
     const half_t *__restrict__ val16, const float *__restrict__ diag32,
     const float *__restrict__ R, float *X) {
   constexpr int W = S / 4;
@@ -380,25 +376,18 @@ __global__ __launch_bounds__(kBlock) void k_bgs32_rows_zero(
   const int64_t i = begin + g / W;
   if (i >= end) return;
   if (LIVE)
-    bgs32_row_zero_live<STREAM, S, 8>(zmask[tile_of(i)], begin, i, (int)(g % W) * 4, n, C, vc,
-                                      col, val16, diag32, R, X);
+    bgs32_row_zero_live<STREAM, S, 8>(begin, i, (int)(g % W) * 4, n, C, vc, col, val16, diag32,
+                                      R, X);
   else
-    bgs32_row_zero<STREAM, S>(zmask[tile_of(i)], begin, i, (int)(g % W) * 4, n, C, vc, col,
+    bgs32_row_zero<STREAM, S>(C.live(C.tile(i)), begin, i, (int)(g % W) * 4, n, C, vc, col,
                               val16, diag32, R, X);
 }
 
 // Whether tile t has all its offset words affine (slot j's column is its
-// base plus the row's position in the tile) and slot 3m + 2's base one
-// above slot 3m's for every m: on the 27-point grid the x - 1 and x + 1
+// base plus the row's place in the tile) and slot 3m + 2's base one above
+// slot 3m's for every m: on the 27-point grid the x - 1 and x + 1
 // neighbours, consecutive rows of one colour block (uniform per tile).
-__device__ inline bool bpairs_tile(const Col16 &C, int t) {
-  if (C.info[t] != kTile8 || !C.amask || C.amask[t] != (1u << kSlotWords) - 1u) return false;
-  const int32_t *__restrict__ base = C.tbase + (int64_t)t * kBaseStride;
-  bool ok = true;
-#pragma unroll
-  for (int m = 0; m < kSlots / 3; ++m) ok = ok && base[3 * m + 2] == base[3 * m] + 1;
-  return ok;
-}
+__device__ inline bool bpairs_tile(const Col16 &C, int t) { return C.pairs(C.flags(t)); }
 
 // bgs32_row on a wavefront whose 64 / W rows are all present and whose tile
 // passes bpairs_tile: slot 3m + 2's x rows are slot 3m's one row (W lanes)
@@ -413,12 +402,12 @@ __device__ __attribute__((always_inline)) inline void bgs32_row_pairs(int64_t i,
                                        const float *__restrict__ diag32,
                                        const float *__restrict__ R, float *X) {
   constexpr int V = 4, W = S / 4, ROWS = 64 / W;
-  const int t = tile_of(i);
-  const int32_t *__restrict__ base = C.tbase + (int64_t)t * kBaseStride;
+  const int t = C.tile(i);
+  const int32_t *__restrict__ base = C.bases(t);
   const int lane = (int)(threadIdx.x & 63);
   const bool last = lane >= 64 - W;
   const int64_t i0 = i - lane / W;  // the wavefront's first row
-  const int32_t plast = (int32_t)(__builtin_amdgcn_readfirstlane((int)(i0 % kTile)) + ROWS - 1);
+  const int32_t plast = (int32_t)(__builtin_amdgcn_readfirstlane(C.place(i0)) + ROWS - 1);
   float sum[V];
   ldv<V>(R + i * S + o, sum);
 #pragma unroll 1
@@ -449,7 +438,7 @@ __device__ __attribute__((always_inline)) inline void bgs32_row_pairs(int64_t i,
   stv<V>(X + i * S + o, sum);
 }
 
-// One colour step, rows [begin, end) (begin a multiple of kTile when C16).
+// One colour step, rows [begin, end) (begin a colour's first row when C16).
 // PAIRS: bgs32_row_pairs on the wavefronts where it applies.
 template <bool STREAM, int S, bool C16, bool PAIRS = false>
 __global__ __launch_bounds__(kBlock) void k_bgs32_rows(int64_t begin, int64_t end, int64_t n,
@@ -464,7 +453,7 @@ __global__ __launch_bounds__(kBlock) void k_bgs32_rows(int64_t begin, int64_t en
   if (PAIRS) {
     // the wavefront's first row; all its 64 / W rows present (uniform)
     const int64_t i0 = begin + ((int64_t)blockIdx.x * kBlock + (threadIdx.x & ~63u)) / W;
-    if (i0 + 64 / W <= end && bpairs_tile(C, tile_of(i0))) {
+    if (i0 + 64 / W <= end && bpairs_tile(C, C.tile(i0))) {
       bgs32_row_pairs<STREAM, S>(i, (int)(g % W) * 4, n, C, vc, diag32, R, X);
       return;
     }
@@ -486,7 +475,7 @@ __global__ __launch_bounds__(kBlock) void k_bresid_restrict32_rows(
   const int64_t t = g / W;
   const int o = (int)(g % W) * V;
   if (t >= nc) return;
-  const int64_t f = fine_row(ftile, t);
+  const int64_t f = C.transfer(ftile, t);
   float a[V], xv[V];
 #pragma unroll
   for (int k = 0; k < V; ++k) a[k] = 0.0f;
@@ -544,9 +533,9 @@ __device__ inline void bspmv_row(int64_t i, int o, int64_t n, const Col16 &C,
   double xv[V];
 #pragma unroll
   for (int k = 0; k < V; ++k) y[k] = 0.0;
-  const int t = H ? tile_of(i) : 0;
-  if (H && C.info[t] != kTile32) {
-    const int32_t *__restrict__ base = C.tbase + (int64_t)t * kBaseStride;
+  const int t = H ? C.tile(i) : 0;
+  if (H && (C.flags(t) & 3u) != kTile32) {
+    const int32_t *__restrict__ base = C.bases(t);
     const int ds = dslot[i];
     const double di = diag[i];
 #pragma unroll
@@ -631,6 +620,7 @@ __global__ __launch_bounds__(kBlock) void k_bspmv_chunks(
     const double *__restrict__ X, double *__restrict__ Y, bool dot, double *__restrict__ cpart) {
   constexpr int V = 2, W = S / V;
   const int64_t q = blockIdx.x, b = q / W;
+  if (H) C.chunk(chunks, b);
   const int64_t i = chunks[2 * b] + (q % W) * (kBlock / W) + threadIdx.x / W;
   const int o = (int)(threadIdx.x % W) * V;
   double acc[V] = {0.0, 0.0};
@@ -662,6 +652,7 @@ __global__ __launch_bounds__(kBlock) void k_bspmv_resid_chunks(
     float *__restrict__ R32, double *__restrict__ cpart) {
   constexpr int V = 2, W = S / V;
   const int64_t q = blockIdx.x, b = q / W;
+  if (H) C.chunk(chunks, b);
   const int64_t i = chunks[2 * b] + (q % W) * (kBlock / W) + threadIdx.x / W;
   const int o = (int)(threadIdx.x % W) * V;
   double acc[V] = {0.0, 0.0};
@@ -1014,8 +1005,8 @@ bool rows_kernels(int s) { return s == 4 || s == 8 || s == 16; }
 template <int S>
 void gs_rows_s(const Problem &P, const Level &L, int64_t b, int64_t e, const float *R, float *X,
                hipStream_t st) {
-  const Col16 C = col16_of(P, L);
-  const bool c16 = L.vc && use_col16(P, L, b);
+  const Col16 C = col16_of(P, L, b);
+  const bool c16 = L.vc && use_col16(P, L);
   const unsigned g = grid_for((e - b) * (S / 4));
   // the shared neighbour rows: 16.22 -> 15.63 ms per block iteration at s = 8
   // (256^3), 30.05 -> 30.79 ms at s = 16 (same job), so s = 8 only
@@ -1043,10 +1034,10 @@ void gs_rows_s(const Problem &P, const Level &L, int64_t b, int64_t e, const flo
 template <int S>
 void gs_rows_zero_s(const Problem &P, const Level &L, int64_t b, int64_t e, const float *R,
                     float *X, hipStream_t st) {
-  const Col16 C = col16_of(P, L);
+  const Col16 C = col16_of(P, L, b);
   const unsigned g = grid_for((e - b) * (S / 4));
 #define HPCGX_BZ(ST, LI)                                                                      \
-  k_bgs32_rows_zero<ST, S, LI><<<g, kBlock, 0, st>>>(b, e, L.n, C, L.zmask, L.vc, L.col,        \
+  k_bgs32_rows_zero<ST, S, LI><<<g, kBlock, 0, st>>>(b, e, L.n, C, L.vc, L.col,        \
                                                      L.val16, L.diag32, R, X)
   const bool live = P.zero_live & 8;
   if (L.stream && live) HPCGX_BZ(true, true);
@@ -1077,7 +1068,7 @@ template <int S>
 void restrict_rows_s(const Problem &P, const Level &L, const float *RF, const float *XF,
                      float *RC, hipStream_t st) {
   const Col16 C = col16_of(P, L);
-  const bool c16 = L.vc && use_col16(P, L, 0);
+  const bool c16 = L.vc && use_col16(P, L);
   const unsigned g = grid_for(L.nc * (S / 4));
   if (L.stream && c16)
     k_bresid_restrict32_rows<true, S, true><<<g, kBlock, 0, st>>>(
@@ -1116,7 +1107,7 @@ template <int S>
 void spmv_rows_s(const Problem &P, const Level &L, const double *X, double *Y, bool dot,
                  unsigned g, hipStream_t st) {
   const Col16 C = col16_of(P, L);
-  const bool h = L.vc && P.half_exact && use_col16(P, L, 0);
+  bool h = L.vc && P.half_exact && use_col16(P, L);
   auto &B = P.blk;
   constexpr int W = S / 2;
   if (P.spmv_dot_chunked && B.cpart && B.ncpart >= L.nchunks * W * S) {
@@ -1139,6 +1130,7 @@ void spmv_rows_s(const Problem &P, const Level &L, const double *X, double *Y, b
     }
     return;
   }
+  h = h && L.aligned;  // these walk all rows: tiles at multiples of kTile
   if (L.stream && h)
     k_bspmv_rows<true, S, true><<<g, kBlock, 0, st>>>(L.n, C, L.vc, L.dslot, L.diag, L.col,
                                                       L.val, X, Y, dot, B.partials, B.ticket,
@@ -1169,12 +1161,8 @@ void spmv_rows(const Problem &P, const Level &L, int s, const double *X, double 
 // unfilled X (every colour step through gs_rows_zero).
 bool zero_guess_block(const Problem &P, int l, int ordering, int s) {
   const Level &L = P.L[l];
-  if (!P.zero_guess || ordering != HPCGX_ORDER_MULTICOLOR || !rows_kernels(s) || !L.zmask ||
-      !L.vc || !L.tbase || !use_col16(P, L, 0) || L.n * s * 4 >= ((int64_t)1 << 32))
-    return false;
-  for (int c = 0; c < L.ncolors; ++c)
-    if (L.color_ptr[c] % kTile) return false;
-  return true;
+  return P.zero_guess && ordering == HPCGX_ORDER_MULTICOLOR && rows_kernels(s) && L.vc &&
+         use_col16(P, L) && L.n * s * 4 < ((int64_t)1 << 32);
 }
 
 // zero_x: X was zero when the sweep began (only with zero_guess_block).
@@ -1365,7 +1353,7 @@ void block_residual_fused_s(Problem &P, const double *Bv, const double *X, hipSt
   auto &B = P.blk;
   const Level &L = P.L[0];
   const Col16 C = col16_of(P, L);
-  const bool h = L.vc && P.half_exact && use_col16(P, L, 0);
+  const bool h = L.vc && P.half_exact && use_col16(P, L);
   constexpr int W = S / 2;
   const unsigned G = (unsigned)(L.nchunks * W);
 #define HPCGX_BRC(ST, HH)                                                                    \

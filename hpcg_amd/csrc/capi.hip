@@ -228,7 +228,7 @@ int hpcgx_problem_info(const hpcgx_problem *p, int level, hpcgx_level_info *info
     info->ncoarse = L.nc;
     info->wave = (L.wave && p->P.use_wave) ? 1 : 0;
     info->nslabs = L.nslabs;
-    info->col16 = L.c16 ? 1 : 0;
+    info->col16 = L.c16 && L.aligned ? 1 : 0;
     info->wide_tiles = L.wide_tiles;
     info->byte_tiles = L.byte_tiles;
   });

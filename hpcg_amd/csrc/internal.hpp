@@ -30,8 +30,11 @@ constexpr int kWaveRows = 2;               // rows per thread of a wavefront tas
 constexpr int kTile = 64;  // rows sharing narrow column bases (one wavefront)
 constexpr int kSlotWords = (kSlots + 3) / 4;  // 8-bit offsets of 4 slots per word
 constexpr int kPairWords = (kSlots + 1) / 2;  // FP16 values of 2 slots per word
-constexpr int kBaseStride = 32;  // ints per tile in Level::tbase (128 bytes)
+constexpr int kBaseStride = 32;  // ints per tile record (Level::trec, 128 bytes)
 enum TileClass { kTile8 = 0, kTile32 = 1, kTile16 = 2 };
+enum TileRecord { kRecFlags = 27, kRecLive = 28 };  // fields of a tile record after the bases
+constexpr int kMidSlot = kSlots / 2;  // the diagonal's slot on a tile with every offset
+constexpr unsigned kAllAffine = (1u << kSlotWords) - 1u;
 constexpr int kBandLines = 1;  // grid lines per band of the in-colour order (1 = natural)
 
 struct Error : std::runtime_error {
@@ -196,51 +199,56 @@ struct Level {
   uint32_t *v16p = nullptr;  // c16 levels: FP16 bits of slots 2w, 2w+1 in word w ([kPairWords][n])
   float *diag32 = nullptr;
   float *rc32 = nullptr, *xc32 = nullptr;
-  // Narrow column ids.  Tile t = device rows [kTile t, kTile t + kTile).  The
-  // slots of a tile are aligned: slot j holds the tile's j-th distinct
-  // natural column offset (col - row in natural numbering, ascending); a row
-  // without that offset holds a valid column and the value 0 there, so each
-  // row still meets its stored entries in ascending column order and the
-  // extra terms add exact zeros.  Column of slot j of row i in tile t:
-  //   tinfo[t] == kTile8:  cbase[j * ntiles + t] + byte (j % 4) of
-  //                        off8[(j / 4) * n + i]   (every slot spans <= 255)
-  //   tinfo[t] == kTile16: cbase[j * ntiles + t] + col16[j * n + i]
-  // tbase[t * kBaseStride + j] holds the same bases tile by tile.  The FP64
-  // kernels read cbase, whose lines serve 16 neighbouring tiles; the FP32
-  // kernels read tbase, where a tile's bases come in a few wide scalar loads
-  // (measured: each is the faster layout for its own kernels).
-  //   tinfo[t] == kTile32: col[j * n + i] (more than 27 distinct offsets, or
-  //                        a slot spanning more than 65535 columns)
+  // Narrow column ids.  A tile is 64 consecutive device rows of one colour,
+  // counted from the colour's first row (its last tile may hold fewer): tiles
+  // colour_tile[c] .. colour_tile[c + 1] - 1 are colour c's.  The slots of a
+  // tile are aligned: slot j holds the tile's j-th distinct natural column
+  // offset (col - row in natural numbering, ascending); a row without that
+  // offset holds a valid column and the value 0 there, so each row still
+  // meets its stored entries in ascending column order and the extra terms
+  // add exact zeros.  Column of slot j of row i in tile t, by the tile's class:
+  //   kTile8:  base[j] + byte (j % 4) of off8[(j / 4) * n + i] (every slot
+  //            spans <= 255), or base[j] + the row's place in the tile for
+  //            every slot of an offset word g whose affine bit is set
+  //   kTile16: base[j] + col16[j * n + i]
+  //   kTile32: col[j * n + i] (more than 27 distinct offsets, or a slot
+  //            spanning more than 65535 columns)
   // `col` holds the 32-bit ids of every tile, col16 those of every 8- and
-  // 16-bit tile.
+  // 16-bit tile.  Tile t's record, trec[t * kBaseStride ..], one 128-byte line
+  // that a wavefront reads with a few scalar loads: the 27 bases, then
+  // kRecFlags (class | affine bits << 8 | pairs << 16) and kRecLive.  One line
+  // for everything matters on small levels, whose steps are a chain of memory
+  // latencies: with bases, class and masks in arrays of their own (the bases
+  // strided by tile count) a step over 32768 rows took 13.0 us, 7.7 us from the
+  // record (k_gs_range16; 4.6 us with gs_row_deep's loads).  On 512^3 the
+  // record and the affine windows at the grid's edges (k_tile_layout) took the
+  // step from 994 to 889 us and the SpMV from 7.30 to 5.92 ms.
+  //   pairs: all offset words affine, base[3m + 2] == base[3m] + 1 for all m,
+  //   and every row's diagonal in slot kMidSlot
+  //   kRecLive: bit j set when some row of the tile stores a nonzero in slot j
+  //   whose column lies in a colour visited before the row's own (a device row
+  //   below its colour's first): the only slots the first forward sweep from
+  //   x = 0 reads (launch_symgs_rows_zero)
   bool c16 = false;
+  bool aligned = false;     // every colour starts at a multiple of kTile
   int64_t ntiles = 0;
   int64_t wide_tiles = 0;   // kTile32 tiles
   int64_t byte_tiles = 0;   // kTile8 tiles
   uint16_t *col16 = nullptr;
   uint32_t *off8 = nullptr;  // [kSlotWords * n]
-  // per kTile8 tile: bit g set when every row's offset word g is
-  // lane * 0x01010101 (each of its slots' columns is the slot base plus the
-  // row's position in the tile), so the kernels need not load it
-  uint8_t *amask = nullptr;
-  int32_t *cbase = nullptr;
-  int32_t *tbase = nullptr;
-  int32_t *tinfo = nullptr;
-  // Per tile, bit j set when some row of the tile stores a nonzero in slot j
-  // whose column lies in a colour visited before the row's own (a device
-  // row below the first row of the row's colour): the only slots the first
-  // forward sweep from x = 0 reads (launch_symgs_rows_zero).
-  uint32_t *zmask = nullptr;
+  int32_t *trec = nullptr;   // [kBaseStride * ntiles]
+  std::vector<int32_t> color_tile;  // [ncolors + 1]
+  int32_t *chunk_tile = nullptr;    // [nchunks] tile of a chunk's first row
   // transfer to the next level: f2c[coarse device row] = fine device row
   int64_t nc = 0;
   int32_t *f2c = nullptr;
   // When the fine rows f2c reaches, in ascending order, form runs of
-  // consecutive rows that each start at a multiple of kTile and (all but the
-  // last) hold a multiple of kTile rows (the injected points of the 27-point
-  // grid are one parity class, a colour block), the transfers run in fine
-  // order: thread t owns fine row fine_row(ftile, t) (ascending in t) and
-  // coarse row rperm[t], so a wavefront reads whole tiles of matrix rows.
-  int32_t *ftile = nullptr;  // per kTile transfer rows: fine row / kTile
+  // consecutive rows that each start a tile and (all but the last) hold a
+  // multiple of kTile rows (the injected points of the 27-point grid are one
+  // parity class, a colour block), the transfers run in fine order: thread t
+  // owns fine row ftile[2 (t / kTile)] + t % kTile (ascending in t) and coarse
+  // row rperm[t], so a wavefront reads whole tiles of matrix rows.
+  int32_t *ftile = nullptr;  // per kTile transfer rows: first fine row, its tile
   int32_t *rperm = nullptr;
   double *rc = nullptr, *xc = nullptr;  // next level's residual and correction
   LexPlan lex;
@@ -264,7 +272,7 @@ struct Problem {
   bool use_c16 = true;        // read narrow column ids where a level has them
   bool use_c8 = true;         // ... 8-bit ones where a tile has them
   bool use_pairs = true;      // FP32 colour steps of 8-bit tiles read FP16 value pairs
-  bool use_affine = true;     // skip the offset words Level::amask marks ("affine8")
+  bool use_affine = true;     // skip the affine offset words (Level::trec; "affine8")
   bool stream_p = false;      // p update with non-temporal accesses ("stream_p")
   bool zero_guess = true;     // V-cycle's first forward sweeps skip the zero x ("zero_guess")
   bool defer_x = true;        // CG takes x's step with the next p update ("defer_x")
@@ -394,42 +402,82 @@ struct Problem {
   } klog;
 };
 
-// Kernel view of a level's 16-bit column ids.  Kernels that use it start
-// every wavefront at a multiple of kTile rows, so a wavefront's rows share
-// one tile and its bases are wave-uniform (read through the scalar cache).
+// Kernel view of a level's narrow column ids.  Kernels that use it start every
+// wavefront at the first row of a tile, so a wavefront's rows share one tile
+// and its record is wave-uniform (read through the scalar cache).  The rows
+// of the launch (or, set by the kernel, of the row chunk or transfer group)
+// start at row0, tile tile0.
 struct Col16 {
   const uint16_t *off;
   const uint32_t *off8;
-  const int32_t *base;   // slot-major bases (Level::cbase)
-  const int32_t *tbase;  // tile-major bases (Level::tbase)
-  const int32_t *info;
-  int64_t ntiles;
-  int use8;  // read 8-bit offsets in kTile8 tiles (else their 16-bit ids)
-  const uint8_t *amask;  // Level::amask, or null: load every offset word
+  const int32_t *trec;   // Level::trec
+  const int32_t *ctile;  // Level::chunk_tile
+  int use8;    // read 8-bit offsets in kTile8 tiles (else their 16-bit ids)
+  int affine;  // skip the affine offset words (else load every one)
+  int tile0;
+  int64_t row0;
+  __device__ inline int tile(int64_t i) const {
+    return __builtin_amdgcn_readfirstlane(tile0 + (int)((i - row0) / kTile));
+  }
+  __device__ inline int place(int64_t i) const { return (int)((i - row0) % kTile); }
+  __device__ inline const int32_t *bases(int t) const {
+    return trec + (int64_t)t * kBaseStride;
+  }
+  __device__ inline uint32_t flags(int t) const {
+    return (uint32_t)trec[(int64_t)t * kBaseStride + kRecFlags];
+  }
+  __device__ inline uint32_t live(int t) const {
+    return (uint32_t)trec[(int64_t)t * kBaseStride + kRecLive];
+  }
+  // tile class, with use8 off 8-bit tiles read as 16-bit ones
+  __device__ inline int cls(uint32_t flags) const {
+    const int c = (int)(flags & 3u);
+    return c == kTile8 && !use8 ? (int)kTile16 : c;
+  }
+  // offset words that need no load (of a tile whose cls is kTile8)
+  __device__ inline unsigned words(uint32_t flags) const {
+    return affine ? (flags >> 8) & kAllAffine : 0u;
+  }
+  __device__ inline bool pairs(uint32_t flags) const {
+    return use8 && affine && (flags >> 16 & 1u);
+  }
+  __device__ inline void chunk(const int64_t *chunks, int64_t b) {
+    row0 = chunks[2 * b];
+    tile0 = ctile[b];
+  }
+  // transfer row t (a wavefront's share one group): the fine row
+  __device__ inline int64_t transfer(const int32_t *ftile, int64_t t) {
+    const int g = __builtin_amdgcn_readfirstlane((int)(t / kTile));
+    row0 = ftile[2 * g];
+    tile0 = ftile[2 * g + 1];
+    return row0 + t % kTile;
+  }
 };
-inline Col16 col16_of(const Problem &P, const Level &L) {
-  return Col16{L.col16, L.off8, L.cbase, L.tbase, L.tinfo, L.ntiles, P.use_c8 ? 1 : 0,
-               P.use_affine ? L.amask : nullptr};
+// The rows from `begin`, the first row of a colour.
+inline Col16 col16_of(const Problem &P, const Level &L, int64_t begin = 0) {
+  int t0 = 0;
+  for (int c = 0; c < L.ncolors && L.c16; ++c)
+    if (L.color_ptr[c] == begin) t0 = L.color_tile[c];
+  return Col16{L.col16, L.off8, L.trec, L.chunk_tile, P.use_c8 ? 1 : 0, P.use_affine ? 1 : 0, t0,
+               begin};
 }
-// Offset word g of row i on a kTile8 tile: loaded, or lane * 0x01010101
-// where the tile's Level::amask bit g says so (amask uniform per tile).
+// Offset word g of row i (the place-th of its tile) on a kTile8 tile: loaded,
+// or place * 0x01010101 where the tile's word is affine (uniform per tile).
 template <bool STREAM>
-__device__ inline uint32_t off8_word(const uint32_t *__restrict__ off8, unsigned amask, int g,
-                                     int64_t n, int64_t i) {
-  if ((amask >> g) & 1u) return (uint32_t)(i % kTile) * 0x01010101u;
+__device__ inline uint32_t off8_word(const uint32_t *__restrict__ off8, unsigned words, int g,
+                                     int64_t n, int64_t i, int place) {
+  if ((words >> g) & 1u) return (uint32_t)place * 0x01010101u;
   if (STREAM) return __builtin_nontemporal_load(off8 + (int64_t)g * n + i);
   return off8[(int64_t)g * n + i];
 }
 
 // Fine row of fine-order transfer row t (Level::ftile).
 __device__ inline int64_t fine_row(const int32_t *__restrict__ ftile, int64_t t) {
-  return (int64_t)ftile[t / kTile] * kTile + t % kTile;
+  return (int64_t)ftile[2 * (t / kTile)] + t % kTile;
 }
 
-// 16-bit kernels apply to rows [begin, ...) of L when this holds.
-inline bool use_col16(const Problem &P, const Level &L, int64_t begin) {
-  return P.use_c16 && L.c16 && begin % kTile == 0;
-}
+// The narrow column ids of L are built and switched on.
+inline bool use_col16(const Problem &P, const Level &L) { return P.use_c16 && L.c16; }
 
 // Slots of Problem::scalars used by CG.
 enum CgScalar { kRtz = 0, kOldRtz, kPAp, kAlpha, kBeta, kNormr2, kDot, kNumScalars };
@@ -457,7 +505,7 @@ void launch_symgs_list(const Level &L, const int32_t *rows, int64_t count,
 // (rows of colours already updated in this sweep) and takes 0 for every
 // other x, so x needs no zero fill; same bits as launch_symgs_rows on a
 // zero-filled x.  False (nothing launched) where it does not apply (no
-// narrow column ids at begin, no Level::zmask).
+// narrow column ids).
 bool launch_symgs_rows_zero(const Problem &P, const Level &L, int64_t begin, int64_t end,
                             const double *r, double *x, hipStream_t s);
 void launch_restriction(const Level &L, const double *rf, const double *Axf,

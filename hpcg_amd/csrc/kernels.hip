@@ -168,6 +168,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv(
     const int32_t *__restrict__ col, const double *__restrict__ val,
     const double *__restrict__ x, double *__restrict__ y, bool xcd) {
   const int64_t b = xcd_block(blockIdx.x, gridDim.x, xcd);
+  if (C16) C.chunk(chunks, b);
   const int64_t i = chunks[2 * b] + threadIdx.x;
   if (i < chunks[2 * b + 1])
     y[i] = C16 ? row_dot16<STREAM>(C, col, val, x, n, i) : row_dot<STREAM>(col, val, x, n, i);
@@ -200,26 +201,22 @@ __device__ inline double gs_row(int64_t i, int64_t n,
   return sum / d;
 }
 
-// Narrow column ids (Level::col16 / off8).  The caller's wavefront lies in
-// one tile, so the tile id, its class and its slot bases are uniform (read
-// through the scalar cache).  narrow_row() calls f(j, k, c) for every slot j
-// in order, with k = j*n + i and c the slot's column.
-__device__ inline int tile_of(int64_t i) {
-  return __builtin_amdgcn_readfirstlane((int)(i / kTile));
-}
-
+// Narrow column ids (Level::trec).  The caller's wavefront lies in one tile,
+// so the tile id and its record are uniform (read through the scalar cache).
+// narrow_row() calls f(j, k, c) for every slot j in order, with k = j*n + i
+// and c the slot's column.
 template <bool STREAM, class F>
-__device__ inline void narrow_row(const Col16 &C, int t, int info, int64_t n, int64_t i,
+__device__ inline void narrow_row(const Col16 &C, int t, uint32_t flags, int64_t n, int64_t i,
                                   F &&f) {
-  const int32_t *__restrict__ base = C.base + t;
-  if (info == kTile8 && C.use8 && C.amask && C.amask[t] == (1u << kSlotWords) - 1u) {
+  const int32_t *__restrict__ base = C.bases(t);
+  const int cls = C.cls(flags);
+  if (cls == kTile8 && C.words(flags) == kAllAffine) {
     // every offset word of the tile is affine: slot j's column is its base
-    // plus the row's position in the tile
-    const int32_t pos = (int32_t)(i % kTile);
+    // plus the row's place in the tile
+    const int32_t pos = C.place(i);
 #pragma unroll
-    for (int j = 0; j < kSlots; ++j)
-      f(j, (int64_t)j * n + i, base[(int64_t)j * C.ntiles] + pos);
-  } else if (info == kTile8 && C.use8) {
+    for (int j = 0; j < kSlots; ++j) f(j, (int64_t)j * n + i, base[j] + pos);
+  } else if (cls == kTile8) {
 #pragma unroll
     for (int g = 0; g < kSlotWords; ++g) {
       const uint32_t w = mload<STREAM>(C.off8 + (int64_t)g * n + i);
@@ -227,15 +224,14 @@ __device__ inline void narrow_row(const Col16 &C, int t, int info, int64_t n, in
       for (int b = 0; b < 4; ++b) {
         const int j = 4 * g + b;
         if (j < kSlots)
-          f(j, (int64_t)j * n + i,
-            base[(int64_t)j * C.ntiles] + (int32_t)((w >> (8 * b)) & 0xffu));
+          f(j, (int64_t)j * n + i, base[j] + (int32_t)((w >> (8 * b)) & 0xffu));
       }
     }
   } else {
 #pragma unroll
     for (int j = 0; j < kSlots; ++j) {
       const int64_t k = (int64_t)j * n + i;
-      f(j, k, base[(int64_t)j * C.ntiles] + (int32_t)mload<STREAM>(C.off + k));
+      f(j, k, base[j] + (int32_t)mload<STREAM>(C.off + k));
     }
   }
 }
@@ -252,12 +248,12 @@ __device__ inline void narrow_row(const Col16 &C, int t, int info, int64_t n, in
 template <class F>
 __device__ inline void affine_pairs_row(const Col16 &C, int t, int64_t n, int64_t i,
                                         const double *x, F &&f) {
-  const int32_t *__restrict__ base = C.base + t;
-  const int32_t pos = (int32_t)(i % kTile);
+  const int32_t *__restrict__ base = C.bases(t);
+  const int32_t pos = C.place(i);
 #pragma unroll
   for (int m = 0; m < kSlots / 3; ++m) {
-    const int32_t b0 = base[(int64_t)(3 * m) * C.ntiles];
-    const int32_t b1 = base[(int64_t)(3 * m + 1) * C.ntiles];
+    const int32_t b0 = base[3 * m];
+    const int32_t b1 = base[3 * m + 1];
     const double x0 = x[b0 + pos];
     const double x1 = x[b1 + pos];
     const double up = __shfl_down(x0, 1, 64);
@@ -269,19 +265,11 @@ __device__ inline void affine_pairs_row(const Col16 &C, int t, int64_t n, int64_
   }
 }
 
-// Whether the wavefront of row i can take affine_pairs_row: an affine
-// 8-bit tile all of whose 64 rows lie below `end`, with slot 3m + 2's base
-// one above slot 3m's for every m (uniform per wavefront).
-__device__ inline bool pairs_tile(const Col16 &C, int t, int info, int64_t end) {
-  if (!(info == kTile8 && C.use8 && C.amask && C.amask[t] == (1u << kSlotWords) - 1u &&
-        (int64_t)(t + 1) * kTile <= end))
-    return false;
-  const int32_t *__restrict__ base = C.base + t;
-  bool ok = true;
-#pragma unroll
-  for (int m = 0; m < kSlots / 3; ++m)
-    ok = ok && base[(int64_t)(3 * m + 2) * C.ntiles] == base[(int64_t)(3 * m) * C.ntiles] + 1;
-  return ok;
+// Whether the wavefront of row i can take affine_pairs_row: a tile whose
+// record says so, all of whose 64 rows lie below `end` (uniform).
+__device__ inline bool pairs_tile(const Col16 &C, uint32_t flags, int64_t i, int64_t end) {
+  const int first = __builtin_amdgcn_readfirstlane((int)(i - C.place(i)));
+  return C.pairs(flags) && (int64_t)first + kTile <= end;
 }
 
 template <bool STREAM, bool PAIRS>
@@ -289,17 +277,17 @@ __device__ inline double row_dot16(const Col16 &C, const int32_t *__restrict__ c
                                    const double *__restrict__ val,
                                    const double *__restrict__ x, int64_t n,
                                    int64_t i, int64_t end) {
-  const int t = tile_of(i);
-  const int info = C.info[t];
-  if (info == kTile32) return row_dot<STREAM>(col, val, x, n, i);
+  const int t = C.tile(i);
+  const uint32_t flags = C.flags(t);
+  if (C.cls(flags) == kTile32) return row_dot<STREAM>(col, val, x, n, i);
   double sum = 0.0;
-  if (PAIRS && pairs_tile(C, t, info, end)) {
+  if (PAIRS && pairs_tile(C, flags, i, end)) {
     affine_pairs_row(C, t, n, i, x, [&](int, int64_t k, int32_t, double xc) {
       sum += mload<STREAM>(val + k) * xc;
     });
     return sum;
   }
-  narrow_row<STREAM>(C, t, info, n, i, [&](int, int64_t k, int32_t c) {
+  narrow_row<STREAM>(C, t, flags, n, i, [&](int, int64_t k, int32_t c) {
     sum += mload<STREAM>(val + k) * x[c];
   });
   return sum;
@@ -310,19 +298,26 @@ __device__ inline double gs_row16(const Col16 &C, int64_t i, int64_t n,
                                   const int32_t *__restrict__ col,
                                   const double *__restrict__ val,
                                   const double *__restrict__ r, double *x, int64_t end = 0) {
-  const int t = tile_of(i);
-  const int info = C.info[t];
-  if (info == kTile32) return gs_row<STREAM>(i, n, col, val, r, x);
+  const int t = C.tile(i);
+  const uint32_t flags = C.flags(t);
+  if (C.cls(flags) == kTile32) return gs_row<STREAM>(i, n, col, val, r, x);
   double sum = r[i];
   double d = 0.0;
-  if (PAIRS && pairs_tile(C, t, info, end)) {
-    affine_pairs_row(C, t, n, i, x, [&](int, int64_t k, int32_t c, double xc) {
+  if (PAIRS && pairs_tile(C, flags, i, end)) {
+    double xi = 0.0;
+    affine_pairs_row(C, t, n, i, x, [&](int j, int64_t k, int32_t, double xc) {
       const double v = mload<STREAM>(val + k);
       sum -= v * xc;
-      if (c == i && v != 0.0) d = v;
+      if (j == kMidSlot) {  // the diagonal (Level::trec's pairs bit)
+        d = v;
+        xi = xc;
+      }
     });
+    sum += xi * d;
+    x[i] = sum / d;
+    return sum / d;
   } else {
-    narrow_row<STREAM>(C, t, info, n, i, [&](int, int64_t k, int32_t c) {
+    narrow_row<STREAM>(C, t, flags, n, i, [&](int, int64_t k, int32_t c) {
       const double v = mload<STREAM>(val + k);
       sum -= v * x[c];
       if (c == i && v != 0.0) d = v;
@@ -347,10 +342,9 @@ __global__ __launch_bounds__(kBlock) void k_gs_range(
   if (i < end) gs_row<STREAM>(i, n, col, val, r, x);
 }
 
-// k_gs_range with 16-bit column ids (begin is a multiple of kTile).  BS
+// k_gs_range with narrow column ids (begin is a colour's first row).  BS
 // threads per workgroup; W: the waves-per-EU floor given to the compiler
-// (7 caps it at 72 VGPRs, where its own choice, 77, allows 6 waves per
-// SIMD; 1 leaves it free).  The finest level's workgroup size and cap are
+// (7 caps it at 72 VGPRs; 1 leaves it free, 94 registers).  The finest level's workgroup size and cap are
 // tuning knobs ("gs_block", "gs_waves"); other levels use kBlock and 7.
 template <bool STREAM, bool FINEST, int BS, int W, bool PAIRS = false>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_gs_range16(
@@ -366,10 +360,9 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
 // V-cycle every row is updated once, so these partials hold r.z (CG.cpp:110)
 // without reading r and z again.  One partial per wavefront: a 64-lane
 // shuffle tree, with no LDS and no workgroup barrier (a per-workgroup sum
-// cost 40 us per launch at 512x512x640).  Under W = 6 the compiler fits 71
-// VGPRs, which still run 7 waves per SIMD as k_gs_range16 does, and keeps
-// k_gs_range16's memory waits; under W = 7 (70 VGPRs) it waited more often
-// and the step took 12% longer.  Uncapped it takes 120 (4 waves).
+// cost 40 us per launch at 512x512x640).  Under W = 6 it takes 78 VGPRs (6
+// waves per SIMD); under W = 7 it spills (15 registers) and a whole iteration
+// took 48.8 against 47.6 ms.
 template <bool STREAM, int BS, int W, bool PAIRS = false>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_gs_rz16(
     int64_t begin, int64_t end, int64_t n, Col16 C, const int32_t *__restrict__ col,
@@ -387,11 +380,89 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
   if ((threadIdx.x & 63) == 0 && begin + w * 64 < end) dpart[w] = s;
 }
 
+// The colour step with every load of a row in flight at once: the values, the
+// diagonal and the right-hand side go out before the tile's record is known,
+// then the offset words (if any), then all 27 x values, then the sum in slot
+// order.  k_gs_range16's 72 registers hold about a third of a row, so a row
+// there takes several memory round trips one after the other; on large steps
+// its 7 wavefronts per SIMD cover them, on smaller ones nothing does.  Here
+// 128 registers hold the row (4 wavefronts per SIMD).  The diagonal comes from
+// the diagonal array (as in the zero-x step): 8 bytes a row for 27 compares
+// and selects.
+//
+// kDeepRows, the largest step that runs so, is where the two cross (us a step,
+// k_gs_range16 / this, one job): 32768 rows 7.7 / 4.6, 137280 12.8 / 10.1,
+// 262144 20.5 / 16.2, 884736 50.0 / 45.4, 2.1M 107.3 / 106.7, 4.1M 237.4 /
+// 245.7, 16.8M 889 / 934.
+constexpr int64_t kDeepRows = (int64_t)3 << 20;
+template <bool STREAM>
+__device__ inline double gs_row_deep(const Col16 &C, int64_t i, int64_t n,
+                                     const int32_t *__restrict__ col,
+                                     const double *__restrict__ val,
+                                     const double *__restrict__ diag,
+                                     const double *__restrict__ r, double *x) {
+  double v[kSlots], xs[kSlots];
+#pragma unroll
+  for (int j = 0; j < kSlots; ++j) v[j] = mload<STREAM>(val + (int64_t)j * n + i);
+  const double d = mload<STREAM>(diag + i);
+  const double xi = x[i];
+  double sum = r[i];
+  const int t = C.tile(i);
+  const uint32_t flags = C.flags(t);
+  const int32_t *__restrict__ base = C.bases(t);
+  const int cls = C.cls(flags);
+  if (cls == kTile8 && C.words(flags) == kAllAffine) {
+    const uint32_t pos = (uint32_t)C.place(i);
+#pragma unroll
+    for (int j = 0; j < kSlots; ++j) xs[j] = (x + base[j])[pos];
+  } else if (cls == kTile8) {
+    uint32_t w[kSlotWords];
+#pragma unroll
+    for (int g = 0; g < kSlotWords; ++g) w[g] = mload<STREAM>(C.off8 + (int64_t)g * n + i);
+#pragma unroll
+    for (int j = 0; j < kSlots; ++j) xs[j] = (x + base[j])[(w[j / 4] >> (8 * (j % 4))) & 0xffu];
+  } else {
+    int32_t c[kSlots];
+#pragma unroll
+    for (int j = 0; j < kSlots; ++j) {
+      const int64_t k = (int64_t)j * n + i;
+      c[j] = cls == kTile32 ? mload<STREAM>(col + k)
+                            : base[j] + (int32_t)mload<STREAM>(C.off + k);
+    }
+#pragma unroll
+    for (int j = 0; j < kSlots; ++j) xs[j] = x[c[j]];
+  }
+#pragma unroll
+  for (int j = 0; j < kSlots; ++j) sum -= v[j] * xs[j];
+  sum += xi * d;
+  const double z = sum / d;
+  x[i] = z;
+  return z;
+}
+
+// RZ: also the r.z partials, as k_gs_rz16.
+template <bool STREAM, bool FINEST, bool RZ>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_gs_deep(
+    int64_t begin, int64_t end, int64_t n, Col16 C, const int32_t *__restrict__ col,
+    const double *__restrict__ val, const double *__restrict__ diag,
+    const double *__restrict__ r, double *x, double *__restrict__ dpart) {
+  const int64_t i = begin + gtid();
+  double s = 0.0;
+  if (i < end) {
+    const double z = gs_row_deep<STREAM>(C, i, n, col, val, diag, r, x);
+    if (RZ) s = r[i] * z;
+  }
+  if (!RZ) return;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+  if ((threadIdx.x & 63) == 0 && i < end) dpart[(i - begin) / 64] = s;
+}
+
 // The first forward sweep of a V-cycle level from x = 0 (ComputeMG_ref.cpp:
 // 42-47 zeroes x before the pre-smoother).  In the colour step over device
 // rows [begin, end), the only x values the reference's row update reads
 // that are not 0 are those of rows updated earlier in this sweep: device
-// rows below `begin`.  So a slot's values are read only when Level::zmask
+// rows below `begin`.  So a slot's values are read only when kRecLive
 // marks it for the tile (some row has a nonzero there with a column below
 // its colour's first row; uniform per tile), and x only below `begin`.
 // Skipped terms are v * 0 and the diagonal term is x_i * d = 0 * d:
@@ -426,7 +497,7 @@ __device__ inline uint32_t buf_u16(BufView v, uint32_t off) {
 }
 
 // Row i (lane `lane` of tile t, whose first row is tb) of a zero-x colour
-// step; zm is the tile's Level::zmask.  n * 8 < 2^32 (x offsets).  The
+// step; zm is the tile's kRecLive.  n * 8 < 2^32 (x offsets).  The
 // tile's class (32-bit ids, all-affine 8-bit offsets, 8-bit, 16-bit) is
 // decided once, outside the slot loops, so each class's loop is straight
 // code whose loads the compiler can issue together.
@@ -436,12 +507,13 @@ __device__ inline void gs_row_zero(const Col16 &C, uint32_t zm, int64_t begin, i
                                    const double *__restrict__ val,
                                    const double *__restrict__ diag,
                                    const double *__restrict__ r, double *x) {
-  const int t = tile_of(i);
-  const int info = C.info[t];
-  const int64_t tb = (int64_t)t * kTile;
-  const uint32_t lane = (uint32_t)(i - tb);
+  const int t = C.tile(i);
+  const uint32_t flags = C.flags(t);
+  const int cls = C.cls(flags);
+  const uint32_t lane = (uint32_t)C.place(i);
+  const int64_t tb = __builtin_amdgcn_readfirstlane((int)(i - lane));
   const uint32_t xlim = (uint32_t)begin * 8u;
-  const int32_t *__restrict__ base = C.base + t;
+  const int32_t *__restrict__ base = C.bases(t);
   double sum = r[i];
   // slot j's term, its value and x read through views that are empty for a
   // dead slot and end at `begin` for x
@@ -452,18 +524,17 @@ __device__ inline void gs_row_zero(const Col16 &C, uint32_t zm, int64_t begin, i
     const double xc = buf_f64<false>(buf_view(x, live ? xlim : 0u), (uint32_t)c * 8u);
     sum -= v * xc;
   };
-  if (info == kTile32) {
+  if (cls == kTile32) {
 #pragma unroll
     for (int j = 0; j < kSlots; ++j) {
       const bool live = (zm >> j) & 1u;
       term(j, (int32_t)buf_u32<STREAM>(buf_view(col + (int64_t)j * n + tb, live ? 256u : 0u),
                                        lane * 4u));
     }
-  } else if (info == kTile8 && C.use8 && C.amask &&
-             C.amask[t] == (1u << kSlotWords) - 1u) {
+  } else if (cls == kTile8 && C.words(flags) == kAllAffine) {
 #pragma unroll
-    for (int j = 0; j < kSlots; ++j) term(j, base[(int64_t)j * C.ntiles] + (int32_t)lane);
-  } else if (info == kTile8 && C.use8) {
+    for (int j = 0; j < kSlots; ++j) term(j, base[j] + (int32_t)lane);
+  } else if (cls == kTile8) {
 #pragma unroll
     for (int g = 0; g < kSlotWords; ++g) {
       const bool any = (zm >> (4 * g)) & 0xfu;
@@ -473,14 +544,14 @@ __device__ inline void gs_row_zero(const Col16 &C, uint32_t zm, int64_t begin, i
       for (int b = 0; b < 4; ++b) {
         const int j = 4 * g + b;
         if (j < kSlots)
-          term(j, base[(int64_t)j * C.ntiles] + (int32_t)((w >> (8 * b)) & 0xffu));
+          term(j, base[j] + (int32_t)((w >> (8 * b)) & 0xffu));
       }
     }
   } else {
 #pragma unroll
     for (int j = 0; j < kSlots; ++j) {
       const bool live = (zm >> j) & 1u;
-      term(j, base[(int64_t)j * C.ntiles] +
+      term(j, base[j] +
                   (int32_t)buf_u16<STREAM>(buf_view(C.off + (int64_t)j * n + tb,
                                                     live ? 128u : 0u),
                                            lane * 2u));
@@ -493,7 +564,7 @@ __device__ inline void gs_row_zero(const Col16 &C, uint32_t zm, int64_t begin, i
 
 constexpr int kLiveChunk = 8;  // live slots per chunk (8 measured faster than 16)
 
-// gs_row_zero over the live slots only ("zero_live"): Level::zmask's set
+// gs_row_zero over the live slots only ("zero_live"): kRecLive's set
 // bits in ascending slot order, CH per chunk, with the chunk's unused
 // entries read through empty views (a * 0).  The dead slots' loads are not
 // issued at all: gs_row_zero issues every slot's loads, and a step with few
@@ -506,7 +577,7 @@ __device__ inline double zero_live_sum(const Col16 &C, uint32_t zm, int t, int64
                                        const int32_t *__restrict__ col,
                                        const double *__restrict__ val, const double *x,
                                        double sum) {
-  const int32_t *__restrict__ base = C.base + t;
+  const int32_t *__restrict__ base = C.bases(t);
   uint32_t mm = zm;
   while (mm) {
     int js[CH];
@@ -540,11 +611,11 @@ __device__ inline double zero_live_sum(const Col16 &C, uint32_t zm, int t, int64
       if (CLS == 0)
         c = (int32_t)w[q];
       else if (CLS == 1)
-        c = base[(int64_t)j * C.ntiles] + (int32_t)lane;
+        c = base[j] + (int32_t)lane;
       else if (CLS == 2)
-        c = base[(int64_t)j * C.ntiles] + (int32_t)((w[q] >> (8 * (j & 3))) & 0xffu);
+        c = base[j] + (int32_t)((w[q] >> (8 * (j & 3))) & 0xffu);
       else
-        c = base[(int64_t)j * C.ntiles] + (int32_t)w[q];
+        c = base[j] + (int32_t)w[q];
       xc[q] = buf_f64<false>(buf_view(x, ok[q] ? xlim : 0u), (uint32_t)c * 8u);
     }
 #pragma unroll
@@ -554,26 +625,26 @@ __device__ inline double zero_live_sum(const Col16 &C, uint32_t zm, int t, int64
 }
 
 template <bool STREAM, int CH>
-__device__ inline void gs_row_zero_live(const Col16 &C, uint32_t zm, int64_t begin, int64_t i,
-                                        int64_t n, const int32_t *__restrict__ col,
+__device__ inline void gs_row_zero_live(const Col16 &C, int64_t begin, int64_t i, int64_t n,
+                                        const int32_t *__restrict__ col,
                                         const double *__restrict__ val,
                                         const double *__restrict__ diag,
                                         const double *__restrict__ r, double *x) {
-  // every wavefront's rows lie in one tile (colour blocks start on tiles in
-  // this layout, and workgroups are whole wavefronts), so the tile and its
+  // every wavefront's rows lie in one tile (a colour's tiles start at its
+  // first row, and workgroups are whole wavefronts), so the tile and its
   // mask are uniform: the slot loop runs on scalar registers
-  const int t = __builtin_amdgcn_readfirstlane(tile_of(i));
-  zm = __builtin_amdgcn_readfirstlane(zm);
-  const int info = C.info[t];
-  const int64_t tb = (int64_t)t * kTile;
-  const uint32_t lane = (uint32_t)(i - tb);
+  const int t = C.tile(i);
+  const uint32_t zm = C.live(t), flags = C.flags(t);
+  const int cls = C.cls(flags);
+  const uint32_t lane = (uint32_t)C.place(i);
+  const int64_t tb = __builtin_amdgcn_readfirstlane((int)(i - lane));
   const uint32_t xlim = (uint32_t)begin * 8u;
   double sum = r[i];
-  if (info == kTile32)
+  if (cls == kTile32)
     sum = zero_live_sum<STREAM, 0, CH>(C, zm, t, tb, lane, xlim, n, col, val, x, sum);
-  else if (info == kTile8 && C.use8 && C.amask && C.amask[t] == (1u << kSlotWords) - 1u)
+  else if (cls == kTile8 && C.words(flags) == kAllAffine)
     sum = zero_live_sum<STREAM, 1, CH>(C, zm, t, tb, lane, xlim, n, col, val, x, sum);
-  else if (info == kTile8 && C.use8)
+  else if (cls == kTile8)
     sum = zero_live_sum<STREAM, 2, CH>(C, zm, t, tb, lane, xlim, n, col, val, x, sum);
   else
     sum = zero_live_sum<STREAM, 3, CH>(C, zm, t, tb, lane, xlim, n, col, val, x, sum);
@@ -585,15 +656,14 @@ __device__ inline void gs_row_zero_live(const Col16 &C, uint32_t zm, int64_t beg
 // LIVE: the live slots only (gs_row_zero_live), else every slot (gs_row_zero)
 template <bool STREAM, bool FINEST, int BS, bool LIVE = false>
 __global__ __launch_bounds__(BS) void k_gs_zero16(
-    int64_t begin, int64_t end, int64_t n, Col16 C, const uint32_t *__restrict__ zmask,
-    const int32_t *__restrict__ col, const double *__restrict__ val,
-    const double *__restrict__ diag, const double *__restrict__ r, double *x, bool xcd) {
+    int64_t begin, int64_t end, int64_t n, Col16 C, const int32_t *__restrict__ col,
+    const double *__restrict__ val, const double *__restrict__ diag, const double *__restrict__ r, double *x, bool xcd) {
   const int64_t i = begin + xcd_block(blockIdx.x, gridDim.x, xcd) * BS + threadIdx.x;
   if (i >= end) return;
   if (LIVE)
-    gs_row_zero_live<STREAM, kLiveChunk>(C, zmask[tile_of(i)], begin, i, n, col, val, diag, r, x);
+    gs_row_zero_live<STREAM, kLiveChunk>(C, begin, i, n, col, val, diag, r, x);
   else
-    gs_row_zero<STREAM>(C, zmask[tile_of(i)], begin, i, n, col, val, diag, r, x);
+    gs_row_zero<STREAM>(C, C.live(C.tile(i)), begin, i, n, col, val, diag, r, x);
 }
 
 // Two adjacent rows per thread: the matrix is read with 16-byte (values) and
@@ -771,8 +841,8 @@ __global__ __launch_bounds__(kBlock) void k_resid_restrict(
   }
 }
 
-// The same in fine order (Level::ftile, rperm): thread t computes fine row
-// fine_row(ftile, t), so a wavefront reads whole tiles of the matrix (narrow
+// The same in fine order (Level::ftile, rperm): thread t computes the t-th fine
+// row, so a wavefront reads whole tiles of the matrix (narrow
 // column ids when C16), and stores the coarse row rperm[t].
 // PAIRS: row_dot16's x-pair path on wavefronts whose 64 transfer rows are
 // all present (each is then a whole fine tile).
@@ -783,7 +853,7 @@ __global__ __launch_bounds__(kBlock) void k_resid_restrict_f(
     const double *__restrict__ rf, const double *__restrict__ xf, double *__restrict__ rc) {
   const int64_t t = gtid();
   if (t >= nc) return;
-  const int64_t f = fine_row(ftile, t);
+  const int64_t f = C.transfer(ftile, t);
   const int64_t end = (t / kTile + 1) * kTile <= nc ? n : 0;
   const double ax = C16 ? row_dot16<STREAM, PAIRS>(C, col, val, xf, n, f, end)
                         : row_dot<STREAM>(col, val, xf, n, f);
@@ -963,6 +1033,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_dot(
   const int64_t lo = x * nchunks / 8, hi = (x + 1) * nchunks / 8;
   double s = 0.0;
   for (int64_t w = lo + slot; w < hi; w += per) {
+    if (C16) C.chunk(chunks, w);
     const int64_t i = chunks[2 * w] + threadIdx.x;
     if (i < chunks[2 * w + 1]) {
       const double y = C16 ? row_dot16<STREAM>(C, col, val, p, n, i)
@@ -990,6 +1061,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_dot_c(
     const double *__restrict__ val, const double *__restrict__ p, double *__restrict__ Ap,
     double *__restrict__ cpart, bool xcd) {
   const int64_t b = xcd_block(blockIdx.x, gridDim.x, xcd);
+  if (C16) C.chunk(chunks, b);
   const int64_t i = chunks[2 * b] + threadIdx.x;
   const int64_t end = chunks[2 * b + 1];
   double s = 0.0;
@@ -1012,16 +1084,16 @@ __device__ inline double row_dot_h(const Col16 &C, const uint32_t *__restrict__ 
                                    const int32_t *__restrict__ col,
                                    const double *__restrict__ val,
                                    const double *__restrict__ p, int64_t n, int64_t i) {
-  const int t = tile_of(i);
-  if (C.info[t] == kTile32) return row_dot<STREAM>(col, val, p, n, i);
-  const int32_t *__restrict__ base = C.base + t;
+  const int t = C.tile(i);
+  if ((C.flags(t) & 3u) == kTile32) return row_dot<STREAM>(col, val, p, n, i);
+  const int32_t *__restrict__ base = C.bases(t);
   const int ds = mload<STREAM>(dslot + i);
   const double di = mload<STREAM>(diag + i);
   double y = 0.0;
 #pragma unroll
   for (int j = 0; j < kSlots; ++j) {
     const uint32_t wd = mload<STREAM>(vc + (int64_t)j * n + i);
-    const int32_t c = base[(int64_t)j * C.ntiles] + (int32_t)(wd >> 16);
+    const int32_t c = base[j] + (int32_t)(wd >> 16);
     const double a = j == ds ? di : (double)__builtin_bit_cast(_Float16, (uint16_t)(wd & 0xffffu));
     y += a * p[c];
   }
@@ -1029,7 +1101,7 @@ __device__ inline double row_dot_h(const Col16 &C, const uint32_t *__restrict__ 
 }
 
 // row_dot_h on an 8-bit tile from the FP16 value pairs (vp, kPairWords words)
-// and the 8-bit offsets (none loaded where the tile's amask bits say affine):
+// and the 8-bit offsets (none loaded where the tile's words are affine):
 // the same FP16 values, columns and slot order, 2 to 3 bytes per slot in
 // place of 4.  Other tiles take row_dot_h.
 template <bool STREAM>
@@ -1040,14 +1112,15 @@ __device__ inline double row_dot_hp(const Col16 &C, const uint32_t *__restrict__
                                     const int32_t *__restrict__ col,
                                     const double *__restrict__ val,
                                     const double *__restrict__ p, int64_t n, int64_t i) {
-  const int t = tile_of(i);
-  if (C.info[t] != kTile8 || !C.use8)
-    return row_dot_h<STREAM>(C, vc, dslot, diag, col, val, p, n, i);
-  const int32_t *__restrict__ base = C.tbase + (int64_t)t * kBaseStride;
-  const unsigned am = C.amask ? C.amask[t] : 0u;
+  const int t = C.tile(i);
+  const uint32_t flags = C.flags(t);
+  if (C.cls(flags) != kTile8) return row_dot_h<STREAM>(C, vc, dslot, diag, col, val, p, n, i);
+  const int32_t *__restrict__ base = C.bases(t);
+  const unsigned words = C.words(flags);
+  const int place = C.place(i);
   uint32_t o8[kSlotWords], pv[kPairWords];
 #pragma unroll
-  for (int g = 0; g < kSlotWords; ++g) o8[g] = off8_word<STREAM>(C.off8, am, g, n, i);
+  for (int g = 0; g < kSlotWords; ++g) o8[g] = off8_word<STREAM>(C.off8, words, g, n, i, place);
 #pragma unroll
   for (int w = 0; w < kPairWords; ++w) pv[w] = mload<STREAM>(vp + (int64_t)w * n + i);
   const int ds = mload<STREAM>(dslot + i);
@@ -1073,6 +1146,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_dot_hc(
     const double *__restrict__ val, const double *__restrict__ p, double *__restrict__ Ap,
     double *__restrict__ cpart, bool xcd) {
   const int64_t b = xcd_block(blockIdx.x, gridDim.x, xcd);
+  C.chunk(chunks, b);
   const int64_t i = chunks[2 * b] + threadIdx.x;
   double s = 0.0;
   if (i < chunks[2 * b + 1]) {
@@ -1096,6 +1170,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_dot_h(
   const int64_t lo = xq * nchunks / 8, hi = (xq + 1) * nchunks / 8;
   double s = 0.0;
   for (int64_t w = lo + slot; w < hi; w += per) {
+    C.chunk(chunks, w);
     const int64_t i = chunks[2 * w] + threadIdx.x;
     if (i < chunks[2 * w + 1]) {
       const double y = row_dot_h<STREAM>(C, vc, dslot, diag, col, val, p, n, i);
@@ -1295,6 +1370,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_resid(
     const double *__restrict__ val, const double *__restrict__ x, const double *__restrict__ b,
     double *__restrict__ r, float *__restrict__ r32, double *__restrict__ cpart, bool xcd) {
   const int64_t blk = xcd_block(blockIdx.x, gridDim.x, xcd);
+  if (C16) C.chunk(chunks, blk);
   const int64_t i = chunks[2 * blk] + threadIdx.x;
   double s = 0.0;
   if (i < chunks[2 * blk + 1]) {
@@ -1320,6 +1396,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_resid_h(
     const double *__restrict__ val, const double *__restrict__ x, const double *__restrict__ b,
     double *__restrict__ r, float *__restrict__ r32, double *__restrict__ cpart, bool xcd) {
   const int64_t blk = xcd_block(blockIdx.x, gridDim.x, xcd);
+  C.chunk(chunks, blk);
   const int64_t i = chunks[2 * blk] + threadIdx.x;
   double s = 0.0;
   if (i < chunks[2 * blk + 1]) {
@@ -1371,7 +1448,7 @@ void launch_spmv(const Problem &P, const Level &L, const double *x, double *y,
                  hipStream_t s) {
   const unsigned g = (unsigned)L.nchunks;
   const Col16 C = col16_of(P, L);
-  const bool c16 = use_col16(P, L, 0);
+  const bool c16 = use_col16(P, L);
   if (L.stream && c16)
     k_spmv<true, true><<<g, kBlock, 0, s>>>(L.chunks, L.n, C, L.col, L.val, x, y, L.xcd);
   else if (L.stream)
@@ -1386,48 +1463,73 @@ void launch_spmv(const Problem &P, const Level &L, const double *x, double *y,
 void launch_symgs_rows(const Problem &P, const Level &L, int64_t begin, int64_t end,
                        const double *r, double *x, hipStream_t s, double *dpart) {
   if (end <= begin) return;
-  if (dpart && !use_col16(P, L, begin))
-    throw Error(HPCGX_EINVAL, "colour step with r.z partials needs 16-bit column ids");
-  if (use_col16(P, L, begin)) {
-    const Col16 C = col16_of(P, L);
+  if (dpart && !use_col16(P, L))
+    throw Error(HPCGX_EINVAL, "colour step with r.z partials needs narrow column ids");
+  if (use_col16(P, L)) {
+    const Col16 C = col16_of(P, L, begin);
     const int64_t rows = end - begin;
+    if (rows <= kDeepRows) {
+      const unsigned g = grid_for(rows);
+#define HPCGX_DEEP(ST, FI, RZ)                                                                 \
+  k_gs_deep<ST, FI, RZ><<<g, kBlock, 0, s>>>(begin, end, L.n, C, L.col, L.val, L.diag, r, x,   \
+                                             dpart)
+      if (L.finest && L.stream && dpart) HPCGX_DEEP(true, true, true);
+      else if (L.finest && L.stream) HPCGX_DEEP(true, true, false);
+      else if (L.finest && dpart) HPCGX_DEEP(false, true, true);
+      else if (L.finest) HPCGX_DEEP(false, true, false);
+      else if (L.stream) HPCGX_DEEP(true, false, false);
+      else HPCGX_DEEP(false, false, false);
+#undef HPCGX_DEEP
+      HPCGX_LAUNCHED();
+      return;
+    }
     // the x-pair colour steps (default shape only): bit 0 of x_pairs for the
     // steps without r.z, bit 1 for the r.z step
     if (L.finest && (P.x_pairs & (dpart ? 2 : 1)) && P.gs_block == kBlock && P.gs_waves) {
       const unsigned g = (unsigned)((rows + kBlock - 1) / kBlock);
-      if (dpart)
-        k_gs_rz16<true, kBlock, 6, true><<<g, kBlock, 0, s>>>(begin, end, L.n, C, L.col, L.val,
-                                                               r, x, L.xcd, dpart);
-      else
-        k_gs_range16<true, true, kBlock, 7, true><<<g, kBlock, 0, s>>>(begin, end, L.n, C, L.col,
-                                                                        L.val, r, x, L.xcd);
+#define HPCGX_GSP(ST)                                                                          \
+  do {                                                                                         \
+    if (dpart)                                                                                 \
+      k_gs_rz16<ST, kBlock, 6, true><<<g, kBlock, 0, s>>>(begin, end, L.n, C, L.col, L.val, r, \
+                                                          x, L.xcd, dpart);                    \
+    else                                                                                       \
+      k_gs_range16<ST, true, kBlock, 7, true><<<g, kBlock, 0, s>>>(begin, end, L.n, C, L.col,  \
+                                                                   L.val, r, x, L.xcd);        \
+  } while (0)
+      if (L.stream) HPCGX_GSP(true); else HPCGX_GSP(false);
+#undef HPCGX_GSP
       HPCGX_LAUNCHED();
       return;
     }
     if (L.finest) {  // tuned workgroup size and register cap
       const bool cap = P.gs_waves != 0;
-#define HPCGX_GS(BS)                                                                           \
+#define HPCGX_GS(ST, BS)                                                                       \
   do {                                                                                         \
     const unsigned g = (unsigned)((rows + BS - 1) / BS);                                       \
     if (dpart && cap)                                                                          \
-      k_gs_rz16<true, BS, 6><<<g, BS, 0, s>>>(begin, end, L.n, C, L.col, L.val, r, x, L.xcd, \
-                                              dpart);                                          \
+      k_gs_rz16<ST, BS, 6><<<g, BS, 0, s>>>(begin, end, L.n, C, L.col, L.val, r, x, L.xcd,     \
+                                            dpart);                                            \
     else if (dpart)                                                                            \
-      k_gs_rz16<true, BS, 1><<<g, BS, 0, s>>>(begin, end, L.n, C, L.col, L.val, r, x, L.xcd, \
-                                              dpart);                                          \
+      k_gs_rz16<ST, BS, 1><<<g, BS, 0, s>>>(begin, end, L.n, C, L.col, L.val, r, x, L.xcd,     \
+                                            dpart);                                            \
     else if (cap)                                                                              \
-      k_gs_range16<true, true, BS, 7><<<g, BS, 0, s>>>(begin, end, L.n, C, L.col, L.val, r,  \
-                                                       x, L.xcd);                              \
+      k_gs_range16<ST, true, BS, 7><<<g, BS, 0, s>>>(begin, end, L.n, C, L.col, L.val, r, x,   \
+                                                     L.xcd);                                   \
     else                                                                                       \
-      k_gs_range16<true, true, BS, 1><<<g, BS, 0, s>>>(begin, end, L.n, C, L.col, L.val, r,  \
-                                                       x, L.xcd);                              \
+      k_gs_range16<ST, true, BS, 1><<<g, BS, 0, s>>>(begin, end, L.n, C, L.col, L.val, r, x,   \
+                                                     L.xcd);                                   \
+  } while (0)
+#define HPCGX_GSB(BS)                                                                          \
+  do {                                                                                         \
+    if (L.stream) HPCGX_GS(true, BS); else HPCGX_GS(false, BS);                                \
   } while (0)
       switch (P.gs_block) {
-        case 64: HPCGX_GS(64); break;
-        case 128: HPCGX_GS(128); break;
-        case 512: HPCGX_GS(512); break;
-        default: HPCGX_GS(256); break;
+        case 64: HPCGX_GSB(64); break;
+        case 128: HPCGX_GSB(128); break;
+        case 512: HPCGX_GSB(512); break;
+        default: HPCGX_GSB(256); break;
       }
+#undef HPCGX_GSB
 #undef HPCGX_GS
       HPCGX_LAUNCHED();
       return;
@@ -1460,9 +1562,12 @@ void launch_symgs_rows(const Problem &P, const Level &L, int64_t begin, int64_t 
     return;
   }
   const unsigned g = grid_for(end - begin);
-  if (L.finest)
+  if (L.finest && L.stream)
     k_gs_range<true, true><<<g, kBlock, 0, s>>>(begin, end, L.n, L.col, L.val,
                                                 r, x, L.xcd);
+  else if (L.finest)
+    k_gs_range<false, true><<<g, kBlock, 0, s>>>(begin, end, L.n, L.col, L.val,
+                                                 r, x, L.xcd);
   else if (L.stream)
     k_gs_range<true, false><<<g, kBlock, 0, s>>>(begin, end, L.n, L.col, L.val,
                                                  r, x, L.xcd);
@@ -1475,15 +1580,16 @@ void launch_symgs_rows(const Problem &P, const Level &L, int64_t begin, int64_t 
 bool launch_symgs_rows_zero(const Problem &P, const Level &L, int64_t begin, int64_t end,
                             const double *r, double *x, hipStream_t s) {
   // x is read at byte offsets of 32 bits
-  if (!L.zmask || !use_col16(P, L, begin) || L.n >= ((int64_t)1 << 29)) return false;
+  if (!use_col16(P, L) || L.n >= ((int64_t)1 << 29)) return false;
   if (end <= begin) return true;
-  const Col16 C = col16_of(P, L);
+  const Col16 C = col16_of(P, L, begin);
   const int64_t rows = end - begin;
   const bool live = P.zero_live & (L.finest ? 1 : 2);
   if (L.finest) {  // the finest level: the colour steps' workgroup size (gs_block)
-#define HPCGX_GZ(BS, LI)                                                                      \
-  k_gs_zero16<true, true, BS, LI><<<(unsigned)((rows + BS - 1) / BS), BS, 0, s>>>(            \
-      begin, end, L.n, C, L.zmask, L.col, L.val, L.diag, r, x, L.xcd)
+#define HPCGX_GZS(ST, BS, LI)                                                                 \
+  k_gs_zero16<ST, true, BS, LI><<<(unsigned)((rows + BS - 1) / BS), BS, 0, s>>>(            \
+      begin, end, L.n, C, L.col, L.val, L.diag, r, x, L.xcd)
+#define HPCGX_GZ(BS, LI) (L.stream ? HPCGX_GZS(true, BS, LI) : HPCGX_GZS(false, BS, LI))
     switch (P.gs_block) {
       case 64: live ? HPCGX_GZ(64, true) : HPCGX_GZ(64, false); break;
       case 128: live ? HPCGX_GZ(128, true) : HPCGX_GZ(128, false); break;
@@ -1491,10 +1597,11 @@ bool launch_symgs_rows_zero(const Problem &P, const Level &L, int64_t begin, int
       default: live ? HPCGX_GZ(256, true) : HPCGX_GZ(256, false); break;
     }
 #undef HPCGX_GZ
+#undef HPCGX_GZS
   } else {
 #define HPCGX_GZC(ST, LI)                                                                     \
   k_gs_zero16<ST, false, kBlock, LI><<<grid_for(rows), kBlock, 0, s>>>(                       \
-      begin, end, L.n, C, L.zmask, L.col, L.val, L.diag, r, x, L.xcd)
+      begin, end, L.n, C, L.col, L.val, L.diag, r, x, L.xcd)
     if (L.stream && live) HPCGX_GZC(true, true);
     else if (L.stream) HPCGX_GZC(true, false);
     else if (live) HPCGX_GZC(false, true);
@@ -1523,7 +1630,7 @@ void launch_residual_restriction(const Problem &P, const Level &L, const double 
                                  const double *xf, double *rc, hipStream_t s) {
   if (L.rperm) {
     const Col16 C = col16_of(P, L);
-    const bool c16 = use_col16(P, L, 0);
+    const bool c16 = use_col16(P, L);
     const unsigned g = grid_for(L.nc);
     if (L.stream && c16 && L.finest && (P.x_pairs & 1))
       k_resid_restrict_f<true, true, true><<<g, kBlock, 0, s>>>(L.nc, L.ftile, L.rperm, L.n, C,
@@ -1643,10 +1750,10 @@ void launch_spmv_dot(Problem &P, const Level &L, const double *p, double *Ap,
 #define HPCGX_SDC(ST, C16)                                                                   \
   k_spmv_dot_c<ST, C16><<<G, kBlock, 0, s>>>(L.chunks, L.n, C, L.col, L.val, p, Ap,           \
                                              P.chunk_partials, L.xcd)
-    if (use_col16(P, L, 0) && L.finest && L.stream && (P.x_pairs & 1)) {
+    if (use_col16(P, L) && L.finest && L.stream && (P.x_pairs & 1)) {
       k_spmv_dot_c<true, true, true><<<G, kBlock, 0, s>>>(L.chunks, L.n, C, L.col, L.val, p, Ap,
                                                          P.chunk_partials, L.xcd);
-    } else if (use_col16(P, L, 0)) {
+    } else if (use_col16(P, L)) {
       if (L.stream) HPCGX_SDC(true, true); else HPCGX_SDC(false, true);
     } else {
       if (L.stream) HPCGX_SDC(true, false); else HPCGX_SDC(false, false);
@@ -1659,7 +1766,7 @@ void launch_spmv_dot(Problem &P, const Level &L, const double *p, double *Ap,
   int64_t g = std::min<int64_t>(L.nchunks, std::min(P.spmv_dot_blocks, kMaxPartials));
   g = std::max<int64_t>(8, (g + 7) / 8 * 8);
   const Col16 C = col16_of(P, L);
-  const bool c16 = use_col16(P, L, 0);
+  const bool c16 = use_col16(P, L);
   const unsigned G = (unsigned)g;
   if (L.stream && c16)
     k_spmv_dot<true, true><<<G, kBlock, 0, s>>>(L.nchunks, L.chunks, L.n, C, L.col, L.val, p,
@@ -1678,7 +1785,7 @@ void launch_spmv_dot(Problem &P, const Level &L, const double *p, double *Ap,
 
 void launch_spmv_dot_half(Problem &P, const Level &L, const double *p, double *Ap,
                           hipStream_t s) {
-  if (!L.vc || !P.half_exact || !use_col16(P, L, 0)) {
+  if (!L.vc || !P.half_exact || !use_col16(P, L)) {
     launch_spmv_dot(P, L, p, Ap, s);
     return;
   }
@@ -1816,7 +1923,7 @@ bool launch_residual_fused(Problem &P, const Level &L, const double *b, const do
   if (!P.resid_fused || !P.chunk_partials || L.nchunks != P.nchunk_partials) return false;
   const unsigned g = (unsigned)L.nchunks;
   const Col16 C = col16_of(P, L);
-  const bool c16 = use_col16(P, L, 0);
+  const bool c16 = use_col16(P, L);
   const bool h = P.hc_pairs && L.vc && P.half_exact && c16;
   const uint32_t *vp = h && L.v16p && P.use_c8 && L.byte_tiles > 0 ? L.v16p : nullptr;
 #define HPCGX_SR(ST, CC)                                                                       \

@@ -122,11 +122,8 @@ __device__ inline float row_dot32(int64_t i, int64_t n,
   return s;
 }
 
-// 16-bit column ids (Level::col16): the caller's wavefront lies in one tile.
-__device__ inline int tile_of(int64_t i) {
-  return __builtin_amdgcn_readfirstlane((int)(i / kTile));
-}
-
+// Narrow column ids (Level::trec): the caller's wavefront lies in one tile.
+//
 // Entry of a narrow tile packed in one 32-bit word (Level::vc):
 // high half = 16-bit column offset, low half = the FP16 value.  One load per
 // slot instead of two: the FP32 colour step is bound by the number of lane
@@ -141,10 +138,9 @@ __device__ inline float gs32_row16(const Col16 &C, const uint32_t *__restrict__ 
                                   const half_t *__restrict__ val16,
                                   const float *__restrict__ diag32,
                                   const float *__restrict__ r, float *x) {
-  const int t = tile_of(i);
-  const int info = C.info[t];
-  if (info == kTile32) return gs32_row<STREAM>(i, n, col, val16, diag32, r, x);
-  const int32_t *__restrict__ base = C.tbase + (int64_t)t * kBaseStride;
+  const int t = C.tile(i);
+  if ((C.flags(t) & 3u) == kTile32) return gs32_row<STREAM>(i, n, col, val16, diag32, r, x);
+  const int32_t *__restrict__ base = C.bases(t);
   float sum = r[i];
 #pragma unroll
   for (int j = 0; j < kSlots; ++j) {
@@ -163,10 +159,9 @@ __device__ inline float row_dot32_16(const Col16 &C, const uint32_t *__restrict_
                                      const half_t *__restrict__ val16,
                                      const float *__restrict__ diag32,
                                      const float *__restrict__ x) {
-  const int t = tile_of(i);
-  const int info = C.info[t];
-  if (info == kTile32) return row_dot32<STREAM>(i, n, col, val16, diag32, x);
-  const int32_t *__restrict__ base = C.tbase + (int64_t)t * kBaseStride;
+  const int t = C.tile(i);
+  if ((C.flags(t) & 3u) == kTile32) return row_dot32<STREAM>(i, n, col, val16, diag32, x);
+  const int32_t *__restrict__ base = C.bases(t);
   float s = 0.0f;
 #pragma unroll
   for (int j = 0; j < kSlots; ++j) {
@@ -178,17 +173,11 @@ __device__ inline float row_dot32_16(const Col16 &C, const uint32_t *__restrict_
   return s;
 }
 
-// Whether row i's wavefront can share x windows between slots 3m and 3m + 2
-// (kernels.hip's pairs_tile on the tile-major bases): all offset words of the
-// tile affine, slot 3m + 2's base one above slot 3m's for every m, and all
-// 64 rows below `end`.  Uniform per wavefront.
-__device__ inline bool pairs_tile32(const Col16 &C, int t, unsigned am, int64_t end) {
-  if (am != (1u << kSlotWords) - 1u || (int64_t)(t + 1) * kTile > end) return false;
-  const int32_t *__restrict__ base = C.tbase + (int64_t)t * kBaseStride;
-  bool ok = true;
-#pragma unroll
-  for (int m = 0; m < kSlots / 3; ++m) ok = ok && base[3 * m + 2] == base[3 * m] + 1;
-  return ok;
+// Whether row i's wavefront can share x windows between slots 3m and 3m + 2:
+// its tile's record says so, and all 64 rows lie below `end`.  Uniform.
+__device__ inline bool pairs_tile32(const Col16 &C, uint32_t flags, int64_t i, int64_t end) {
+  const int first = __builtin_amdgcn_readfirstlane((int)(i - C.place(i)));
+  return C.pairs(flags) && (int64_t)first + kTile <= end;
 }
 
 // FP32 colour step of an 8-bit tile (Level::off8, Level::v16p): per row
@@ -202,21 +191,21 @@ __device__ inline float gs32_row8(const Col16 &C, const uint32_t *__restrict__ v
                                  const half_t *__restrict__ val16,
                                  const float *__restrict__ diag32,
                                  const float *__restrict__ r, float *x, int64_t end = 0) {
-  const int t = tile_of(i);
-  const int info = C.info[t];
-  if (info != kTile8 || !C.use8) return gs32_row16<STREAM>(C, vc, i, n, col, val16, diag32, r, x);
-  const int32_t *__restrict__ base = C.tbase + (int64_t)t * kBaseStride;
-  const unsigned am = C.amask ? C.amask[t] : 0u;
+  const int t = C.tile(i);
+  const uint32_t flags = C.flags(t);
+  if (C.cls(flags) != kTile8) return gs32_row16<STREAM>(C, vc, i, n, col, val16, diag32, r, x);
+  const int32_t *__restrict__ base = C.bases(t);
+  const unsigned words = C.words(flags);
+  const int32_t pos = C.place(i);
   uint32_t o8[kSlotWords], pv[kPairWords];
 #pragma unroll
-  for (int g = 0; g < kSlotWords; ++g) o8[g] = off8_word<STREAM>(C.off8, am, g, n, i);
+  for (int g = 0; g < kSlotWords; ++g) o8[g] = off8_word<STREAM>(C.off8, words, g, n, i, pos);
 #pragma unroll
   for (int w = 0; w < kPairWords; ++w) pv[w] = mload<STREAM>(vp + (int64_t)w * n + i);
   float sum = r[i];
-  if (PAIRS && pairs_tile32(C, t, am, end)) {
+  if (PAIRS && pairs_tile32(C, flags, i, end)) {
     // kernels.hip's affine_pairs_row in FP32: slot 3m + 2's x from slot 3m's,
     // one lane down; lane 63's from one address for the wavefront
-    const int32_t pos = (int32_t)(i % kTile);
 #pragma unroll
     for (int m = 0; m < kSlots / 3; ++m) {
       const int32_t b0 = base[3 * m];
@@ -255,14 +244,15 @@ __device__ inline float row_dot32_8(const Col16 &C, const uint32_t *__restrict__
                                     const half_t *__restrict__ val16,
                                     const float *__restrict__ diag32,
                                     const float *__restrict__ x) {
-  const int t = tile_of(i);
-  const int info = C.info[t];
-  if (info != kTile8 || !C.use8) return row_dot32_16<STREAM>(C, vc, i, n, col, val16, diag32, x);
-  const int32_t *__restrict__ base = C.tbase + (int64_t)t * kBaseStride;
-  const unsigned am = C.amask ? C.amask[t] : 0u;
+  const int t = C.tile(i);
+  const uint32_t flags = C.flags(t);
+  if (C.cls(flags) != kTile8) return row_dot32_16<STREAM>(C, vc, i, n, col, val16, diag32, x);
+  const int32_t *__restrict__ base = C.bases(t);
+  const unsigned words = C.words(flags);
+  const int place = C.place(i);
   uint32_t o8[kSlotWords], pv[kPairWords];
 #pragma unroll
-  for (int g = 0; g < kSlotWords; ++g) o8[g] = off8_word<STREAM>(C.off8, am, g, n, i);
+  for (int g = 0; g < kSlotWords; ++g) o8[g] = off8_word<STREAM>(C.off8, words, g, n, i, place);
 #pragma unroll
   for (int w = 0; w < kPairWords; ++w) pv[w] = mload<STREAM>(vp + (int64_t)w * n + i);
   float s = 0.0f;
@@ -278,7 +268,7 @@ __device__ inline float row_dot32_8(const Col16 &C, const uint32_t *__restrict__
 
 // The first forward sweep of an FP32 V-cycle level from x = 0: the FP32
 // form of kernels.hip's zero-x colour step (see gs_row_zero there).  Slots
-// that Level::zmask leaves out of the tile, and x at or beyond `begin`,
+// that kRecLive leaves out of the tile, and x at or beyond `begin`,
 // are read through buffer views whose range check returns 0 without a
 // memory access, so the row's loads still go out together.  Each row keeps
 // gs32_row8's (8-bit tiles with FP16 value pairs), gs32_row16's (packed
@@ -309,15 +299,15 @@ __device__ inline void gs32_row_zero(const Col16 &C, uint32_t zm, int64_t begin,
                                      const half_t *__restrict__ val16,
                                      const float *__restrict__ diag32,
                                      const float *__restrict__ r, float *x) {
-  const int t = tile_of(i);
-  const int info = C.info[t];
-  const int64_t tb = (int64_t)t * kTile;
-  const uint32_t lane = (uint32_t)(i - tb);
+  const int t = C.tile(i);
+  const uint32_t flags = C.flags(t);
+  const int32_t *__restrict__ base = C.bases(t);
+  const uint32_t lane = (uint32_t)C.place(i);
+  const int64_t tb = __builtin_amdgcn_readfirstlane((int)(i - lane));
   const uint32_t xlim = (uint32_t)begin * 4u;
   float sum = r[i];
-  if (info == kTile8 && C.use8 && vp) {
-    const int32_t *__restrict__ base = C.tbase + (int64_t)t * kBaseStride;
-    const unsigned am = C.amask ? C.amask[t] : 0u;
+  if (C.cls(flags) == kTile8 && vp) {
+    const unsigned am = C.words(flags);
     uint32_t o8[kSlotWords], pv[kPairWords];
 #pragma unroll
     for (int g = 0; g < kSlotWords; ++g) {
@@ -339,8 +329,7 @@ __device__ inline void gs32_row_zero(const Col16 &C, uint32_t zm, int64_t begin,
       const half_t a = __builtin_bit_cast(half_t, (uint16_t)(pv[j / 2] >> (16 * (j % 2))));
       sum -= (float)a * buf_f32(buf_view(x, live ? xlim : 0u), (uint32_t)c * 4u);
     }
-  } else if (info != kTile32) {
-    const int32_t *__restrict__ base = C.tbase + (int64_t)t * kBaseStride;
+  } else if ((flags & 3u) != kTile32) {
 #pragma unroll
     for (int j = 0; j < kSlots; ++j) {
       const bool live = (zm >> j) & 1u;
@@ -365,8 +354,8 @@ __device__ inline void gs32_row_zero(const Col16 &C, uint32_t zm, int64_t begin,
   x[i] = sum / diag32[i];
 }
 
-// gs32_row_zero over the live slots only (tune key "zero_live"): Level::
-// zmask's set bits in ascending slot order, CH per chunk, with the
+// gs32_row_zero over the live slots only (tune key "zero_live"): kRecLive's
+// set bits in ascending slot order, CH per chunk, with the
 // chunk's unused entries read through empty views (0 * 0).  Each live slot
 // loads its own offset word and value word, so the loads of dead slots are
 // not issued.  CLS: 0 32-bit ids, 1 packed words, 2 8-bit offsets with FP16
@@ -382,8 +371,8 @@ __device__ inline float zero_live_sum32(const Col16 &C, uint32_t zm, int t, int6
                                         const int32_t *__restrict__ col,
                                         const half_t *__restrict__ val16, const float *x,
                                         float sum) {
-  const int32_t *__restrict__ base = C.tbase + (int64_t)t * kBaseStride;
-  const unsigned am = (CLS == 2 && C.amask) ? C.amask[t] : 0u;  // affine offset words
+  const int32_t *__restrict__ base = C.bases(t);
+  const unsigned am = CLS == 2 ? C.words(C.flags(t)) : 0u;  // affine offset words
   uint32_t mm = zm;
   while (mm) {
     int js[CH];
@@ -442,28 +431,28 @@ __device__ inline float zero_live_sum32(const Col16 &C, uint32_t zm, int t, int6
 }
 
 template <bool STREAM, int CH>
-__device__ inline void gs32_row_zero_live(const Col16 &C, uint32_t zm, int64_t begin,
+__device__ inline void gs32_row_zero_live(const Col16 &C, int64_t begin,
                                           const uint32_t *__restrict__ vp,
                                           const uint32_t *__restrict__ vc, int64_t i, int64_t n,
                                           const int32_t *__restrict__ col,
                                           const half_t *__restrict__ val16,
                                           const float *__restrict__ diag32,
                                           const float *__restrict__ r, float *x) {
-  // every wavefront's rows lie in one tile (colour blocks start on tiles in
-  // this layout, and workgroups are whole wavefronts), so the tile and its
+  // every wavefront's rows lie in one tile (a colour's tiles start at its
+  // first row, and workgroups are whole wavefronts), so the tile and its
   // mask are uniform: the slot loop runs on scalar registers
-  const int t = __builtin_amdgcn_readfirstlane(tile_of(i));
-  zm = __builtin_amdgcn_readfirstlane(zm);
-  const int info = C.info[t];
-  const int64_t tb = (int64_t)t * kTile;
-  const uint32_t lane = (uint32_t)(i - tb);
+  const int t = C.tile(i);
+  const uint32_t zm = C.live(t), flags = C.flags(t);
+  const bool narrow8 = C.cls(flags) == kTile8 && vp;
+  const uint32_t lane = (uint32_t)C.place(i);
+  const int64_t tb = __builtin_amdgcn_readfirstlane((int)(i - lane));
   const uint32_t xlim = (uint32_t)begin * 4u;
   float sum = r[i];
-  if (info == kTile8 && C.use8 && vp && C.amask && C.amask[t] == (1u << kSlotWords) - 1u)
+  if (narrow8 && C.words(flags) == kAllAffine)
     sum = zero_live_sum32<STREAM, 3, CH>(C, zm, t, tb, lane, xlim, n, vp, vc, col, val16, x, sum);
-  else if (info == kTile8 && C.use8 && vp)
+  else if (narrow8)
     sum = zero_live_sum32<STREAM, 2, CH>(C, zm, t, tb, lane, xlim, n, vp, vc, col, val16, x, sum);
-  else if (info != kTile32)
+  else if ((flags & 3u) != kTile32)
     sum = zero_live_sum32<STREAM, 1, CH>(C, zm, t, tb, lane, xlim, n, vp, vc, col, val16, x, sum);
   else
     sum = zero_live_sum32<STREAM, 0, CH>(C, zm, t, tb, lane, xlim, n, vp, vc, col, val16, x, sum);
@@ -507,17 +496,16 @@ __global__ __launch_bounds__(kBlock) void k_gs32_range8(
 // LIVE: the live slots only (gs32_row_zero_live), else every slot (gs32_row_zero)
 template <bool STREAM, bool FINEST, bool LIVE = false>
 __global__ __launch_bounds__(kBlock) void k_gs32_zero(
-    int64_t begin, int64_t end, int64_t n, Col16 C, const uint32_t *__restrict__ zmask,
-    const uint32_t *__restrict__ vp, const uint32_t *__restrict__ vc,
-    const int32_t *__restrict__ col, const half_t *__restrict__ val16,
-    const float *__restrict__ diag32, const float *__restrict__ r, float *x, bool xcd) {
+    int64_t begin, int64_t end, int64_t n, Col16 C, const uint32_t *__restrict__ vp,
+    const uint32_t *__restrict__ vc, const int32_t *__restrict__ col,
+    const half_t *__restrict__ val16, const float *__restrict__ diag32,
+    const float *__restrict__ r, float *x, bool xcd) {
   const int64_t i = begin + xcd_block(blockIdx.x, gridDim.x, xcd) * kBlock + threadIdx.x;
   if (i >= end) return;
   if (LIVE)
-    gs32_row_zero_live<STREAM, 8>(C, zmask[tile_of(i)], begin, vp, vc, i, n, col, val16, diag32,
-                                  r, x);
+    gs32_row_zero_live<STREAM, 8>(C, begin, vp, vc, i, n, col, val16, diag32, r, x);
   else
-    gs32_row_zero<STREAM>(C, zmask[tile_of(i)], begin, vp, vc, i, n, col, val16, diag32, r, x);
+    gs32_row_zero<STREAM>(C, C.live(C.tile(i)), begin, vp, vc, i, n, col, val16, diag32, r, x);
 }
 
 // k_gs32_range8 for the V-cycle's last sweep (the finest level's backward
@@ -574,6 +562,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv32_16(
     const float *__restrict__ diag32, const float *__restrict__ x,
     float *__restrict__ y) {
   const int64_t b = blockIdx.x;
+  C.chunk(chunks, b);
   const int64_t i = chunks[2 * b] + threadIdx.x;
   if (i < chunks[2 * b + 1])
     y[i] = row_dot32_16<STREAM>(C, vc, i, n, col, val16, diag32, x);
@@ -627,8 +616,8 @@ __global__ __launch_bounds__(kBlock) void k_prolong32(
   if (c < nc) xf[f2c[c]] += xc[c];
 }
 
-// The transfers in fine order (Level::ftile, rperm): thread t owns fine row
-// fine_row(ftile, t) (whole tiles per wavefront, packed words when C16) and
+// The transfers in fine order (Level::ftile, rperm): thread t owns the t-th
+// fine row (whole tiles per wavefront, packed words when C16) and
 // coarse row rperm[t].
 // C16 = 2: FP16 value pairs on 8-bit tiles (row_dot32_8).
 template <bool STREAM, int C16>
@@ -640,7 +629,7 @@ __global__ __launch_bounds__(kBlock) void k_resid_restrict32_f(
     const float *__restrict__ xf, float *__restrict__ rc) {
   const int64_t t = gtid();
   if (t >= nc) return;
-  const int64_t f = fine_row(ftile, t);
+  const int64_t f = C.transfer(ftile, t);
   const float ax = C16 == 2   ? row_dot32_8<STREAM>(C, vp, vc, f, n, col, val16, diag32, xf)
                    : C16 == 1 ? row_dot32_16<STREAM>(C, vc, f, n, col, val16, diag32, xf)
                               : row_dot32<STREAM>(f, n, col, val16, diag32, xf);
@@ -657,8 +646,8 @@ __global__ __launch_bounds__(kBlock) void k_prolong32_f(int64_t nc,
 }
 
 // The FP16-pair colour step applies (8-bit offsets and FP16 value pairs).
-bool pairs_step(const Problem &P, const Level &L, int64_t begin) {
-  return use_col16(P, L, begin) && L.v16p && P.use_pairs && P.use_c8 && L.byte_tiles > 0;
+bool pairs_step(const Problem &P, const Level &L) {
+  return use_col16(P, L) && L.v16p && P.use_pairs && P.use_c8 && L.byte_tiles > 0;
 }
 
 // With dpart (only where pairs_step holds), also the r.z partials of
@@ -668,10 +657,10 @@ void gs32_step(const Problem &P, const Level &L, int64_t begin, int64_t end,
                const double *r64 = nullptr) {
   if (end <= begin) return;
   const unsigned g = grid_for(end - begin);
-  if (dpart && !pairs_step(P, L, begin))
+  if (dpart && !pairs_step(P, L))
     throw Error(HPCGX_EINVAL, "FP32 colour step with r.z partials needs the FP16-pair layout");
-  if (pairs_step(P, L, begin)) {
-    const Col16 C = col16_of(P, L);
+  if (pairs_step(P, L)) {
+    const Col16 C = col16_of(P, L, begin);
     const bool xp = L.finest && (P.x_pairs & 4);  // the x-pair steps (finest level)
     if (dpart && xp) {
       k_gs32_rz8<true, true><<<g, kBlock, 0, s>>>(begin, end, L.n, C, L.v16p, L.vc, L.col,
@@ -680,15 +669,18 @@ void gs32_step(const Problem &P, const Level &L, int64_t begin, int64_t end,
       k_gs32_range8<true, true, true><<<g, kBlock, 0, s>>>(begin, end, L.n, C, L.v16p, L.vc,
                                                            L.col, L.val16, L.diag32, r, x, L.xcd);
     } else if (dpart) {
-      if (L.finest || L.stream)
+      if (L.stream)
         k_gs32_rz8<true><<<g, kBlock, 0, s>>>(begin, end, L.n, C, L.v16p, L.vc, L.col, L.val16,
                                               L.diag32, r, x, L.xcd, r64, dpart);
       else
         k_gs32_rz8<false><<<g, kBlock, 0, s>>>(begin, end, L.n, C, L.v16p, L.vc, L.col,
                                                L.val16, L.diag32, r, x, L.xcd, r64, dpart);
-    } else if (L.finest)
+    } else if (L.finest && L.stream)
       k_gs32_range8<true, true><<<g, kBlock, 0, s>>>(begin, end, L.n, C, L.v16p, L.vc, L.col,
                                                      L.val16, L.diag32, r, x, L.xcd);
+    else if (L.finest)
+      k_gs32_range8<false, true><<<g, kBlock, 0, s>>>(begin, end, L.n, C, L.v16p, L.vc, L.col,
+                                                      L.val16, L.diag32, r, x, L.xcd);
     else if (L.stream)
       k_gs32_range8<true, false><<<g, kBlock, 0, s>>>(begin, end, L.n, C, L.v16p, L.vc, L.col,
                                                       L.val16, L.diag32, r, x, L.xcd);
@@ -698,8 +690,8 @@ void gs32_step(const Problem &P, const Level &L, int64_t begin, int64_t end,
     HPCGX_LAUNCHED();
     return;
   }
-  if (use_col16(P, L, begin)) {
-    const Col16 C = col16_of(P, L);
+  if (use_col16(P, L)) {
+    const Col16 C = col16_of(P, L, begin);
     if (L.finest)
       k_gs32_range16<true, true><<<g, kBlock, 0, s>>>(begin, end, L.n, C, L.vc, L.col, L.val16,
                                                       L.diag32, r, x);
@@ -728,17 +720,19 @@ void gs32_step(const Problem &P, const Level &L, int64_t begin, int64_t end,
 // (nothing launched) where it does not apply.
 bool gs32_step_zero(const Problem &P, const Level &L, int64_t begin, int64_t end,
                     const float *r, float *x, hipStream_t s) {
-  if (!L.zmask || !L.vc || !use_col16(P, L, begin) || L.n >= ((int64_t)1 << 29)) return false;
+  if (!L.vc || !use_col16(P, L) || L.n >= ((int64_t)1 << 29)) return false;
   if (end <= begin) return true;
   const unsigned g = grid_for(end - begin);
-  const Col16 C = col16_of(P, L);
+  const Col16 C = col16_of(P, L, begin);
   const uint32_t *vp = (L.v16p && P.use_pairs && P.use_c8) ? L.v16p : nullptr;
 #define HPCGX_GZ32(ST, FI, LI)                                                                \
-  k_gs32_zero<ST, FI, LI><<<g, kBlock, 0, s>>>(begin, end, L.n, C, L.zmask, vp, L.vc, L.col,    \
+  k_gs32_zero<ST, FI, LI><<<g, kBlock, 0, s>>>(begin, end, L.n, C, vp, L.vc, L.col,    \
                                                L.val16, L.diag32, r, x, L.xcd)
   const bool live = P.zero_live & 4;
-  if (L.finest && live) HPCGX_GZ32(true, true, true);
-  else if (L.finest) HPCGX_GZ32(true, true, false);
+  if (L.finest && L.stream && live) HPCGX_GZ32(true, true, true);
+  else if (L.finest && L.stream) HPCGX_GZ32(true, true, false);
+  else if (L.finest && live) HPCGX_GZ32(false, true, true);
+  else if (L.finest) HPCGX_GZ32(false, true, false);
   else if (L.stream && live) HPCGX_GZ32(true, false, true);
   else if (L.stream) HPCGX_GZ32(true, false, false);
   else if (live) HPCGX_GZ32(false, false, true);
@@ -752,12 +746,8 @@ bool gs32_step_zero(const Problem &P, const Level &L, int64_t begin, int64_t end
 // unfilled x (every colour step through gs32_step_zero).
 bool zero_guess_sweep32(const Problem &P, int l, int ordering) {
   const Level &L = P.L[l];
-  if (!P.zero_guess || ordering != HPCGX_ORDER_MULTICOLOR || !L.zmask || !L.vc ||
-      !use_col16(P, L, 0) || L.n >= ((int64_t)1 << 29))
-    return false;
-  for (int c = 0; c < L.ncolors; ++c)
-    if (L.color_ptr[c] % kTile) return false;
-  return true;
+  return P.zero_guess && ordering == HPCGX_ORDER_MULTICOLOR && L.vc && use_col16(P, L) &&
+         L.n < ((int64_t)1 << 29);
 }
 }  // namespace
 
@@ -835,7 +825,7 @@ void symgs32(Problem &P, int l, int ordering, const float *r, float *x,
 }
 
 void spmv32(const Problem &P, const Level &L, const float *x, float *y, hipStream_t s) {
-  if (use_col16(P, L, 0)) {
+  if (use_col16(P, L)) {
     const Col16 C = col16_of(P, L);
     if (L.stream)
       k_spmv32_16<true><<<(unsigned)L.nchunks, kBlock, 0, s>>>(L.chunks, L.n, C, L.vc,
@@ -872,7 +862,7 @@ void mg32(Problem &P, int l, int ordering, const float *r, float *x,
     const unsigned g = grid_for(L.nc);
     if (L.rperm) {
       const Col16 C = col16_of(P, L);
-      const bool c16 = L.vc && use_col16(P, L, 0);
+      const bool c16 = L.vc && use_col16(P, L);
       const bool pairs = c16 && L.v16p && P.use_pairs && P.use_c8;
 #define HPCGX_RR32(ST, K)                                                                  \
   k_resid_restrict32_f<ST, K><<<g, kBlock, 0, s>>>(L.nc, L.ftile, L.rperm, L.n, C, L.vc, L.v16p, \
@@ -937,7 +927,7 @@ int64_t rz_partials32(const Problem &P, int ordering) {
   for (int c = 0; c < L.ncolors; ++c) {
     const int64_t b = L.color_ptr[c], e = L.color_ptr[c + 1];
     if (e <= b) continue;
-    if (!pairs_step(P, L, b)) return 0;
+    if (!pairs_step(P, L)) return 0;
     count += rz_slots(e - b);
   }
   return count <= P.nrz_partials ? count : 0;

@@ -15,8 +15,8 @@
 // Rows are then renumbered colour by colour, in the colours' sweep order
 // (kSweepOrders; natural order inside a colour), and the 27-slot ELL is
 // rebuilt in that order, with the slots of every tile of 64 rows aligned by
-// natural column offset so that the column ids of a slot fit 16 bits above a
-// per-tile base (k_tile_layout).
+// natural column offset so that the column ids of a slot fit 8 or 16 bits above
+// a per-tile base, most often the row's place in the tile (k_tile_layout).
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
@@ -47,6 +47,7 @@ constexpr int kNumSweepOrders = (int)(sizeof(kSweepOrders) / sizeof(kSweepOrders
 
 constexpr int kStepBlocks = 2048;      // fixed grid of the Kahn steps
 constexpr int kSyncEvery = 128;        // Kahn steps between host checks
+constexpr int64_t kNarrowRows = 4096;  // levels with unaligned colours: narrow ids from here
 constexpr int64_t kMaxSched = 1 << 22; // bound on schedule levels
 
 inline unsigned grid_for(int64_t n) {
@@ -330,30 +331,49 @@ __device__ inline int wave_max_i32(int v) {
   return v;
 }
 
-// Tile-aligned slots and 16-bit column ids (Level::col16), one wavefront per
-// tile of kTile device rows, in place on the device-order ELL.
+// First row and rows of each tile (Level::color_tile): tile t of colour c is
+// its (t - ctile[c])-th 64 rows.
+__global__ __launch_bounds__(kBlock) void k_tile_rows(int64_t T, int ncolors,
+                                                      const int64_t *__restrict__ cptr,
+                                                      const int32_t *__restrict__ ctile,
+                                                      int32_t *__restrict__ rows) {
+  const int64_t t = gtid();
+  if (t >= T) return;
+  int c = 0;
+  while (c + 1 < ncolors && ctile[c + 1] <= t) ++c;
+  const int64_t b = cptr[c] + (t - ctile[c]) * kTile;
+  rows[2 * t] = (int32_t)b;
+  rows[2 * t + 1] = (int32_t)min((int64_t)kTile, cptr[c + 1] - b);
+}
+
+// Tile-aligned slots and narrow column ids (Level::trec), one wavefront per
+// tile, in place on the device-order ELL.
 //  1. The tile's distinct natural column offsets (column - row, natural
 //     numbering), ascending: repeated wavefront minimum of each row's next
 //     offset.  A row's offsets ascend with its columns, so entry e of a row
 //     lands in a slot >= e and the row's entries keep their order.
 //  2. Entries move to their slots (highest slot first, so nothing is
 //     overwritten before it is read); a row without an entry in a slot gets
-//     a column already in that slot's range and the value 0.  The slot's base
-//     is its smallest column.  The tile's class: 8-bit offsets if every slot
-//     spans at most 255 columns, 16-bit if at most 65535, else (or with more
-//     than 27 distinct offsets) 32-bit ids only.
+//     the value 0 and a valid column: where the slot's entries all lie at one
+//     base plus their row's place in the tile, the column at that place too
+//     (the slot is then affine), else one already in the slot's range.  The
+//     slot's base is its smallest column.  The tile's class: 8-bit offsets if
+//     every slot spans at most 255 columns, 16-bit if at most 65535, else (or
+//     with more than 27 distinct offsets) 32-bit ids only.
 __global__ __launch_bounds__(kBlock) void k_tile_layout(
-    int64_t n, int64_t ntiles, const int32_t *__restrict__ iperm, int32_t *col,
-    double *val, const uint8_t *__restrict__ nnz_row, uint8_t *dslot,
-    uint16_t *col16, uint32_t *off8, int32_t *cbase, int32_t *tbase, int32_t *tinfo,
-    uint8_t *amask) {
+    int64_t n, int64_t ntiles, const int32_t *__restrict__ rows,
+    const int32_t *__restrict__ iperm, int32_t *col, double *val,
+    const uint8_t *__restrict__ nnz_row, uint8_t *dslot, uint16_t *col16, uint32_t *off8,
+    int32_t *trec) {
   const int64_t t = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
   if (t >= ntiles) return;  // whole wavefronts
   const int lane = threadIdx.x & 63;
-  const int64_t i = t * kTile + lane;
-  const bool row = i < n;
+  const int32_t first = rows[2 * t];
+  const int64_t i = first + lane;
+  const bool row = lane < rows[2 * t + 1];
   const int m = row ? nnz_row[i] : 0;
   const int64_t inat = row ? iperm[i] : 0;
+  int32_t *rec = trec + t * kBaseStride;
 
   unsigned mask = 0;  // slots holding one of this row's entries
   int ptr = 0, nu = 0;
@@ -374,16 +394,15 @@ __global__ __launch_bounds__(kBlock) void k_tile_layout(
     ++nu;
   }
   if (!fits) {
-    if (lane == 0) {
-      tinfo[t] = kTile32;
-      amask[t] = 0;
-    }
+    if (lane < kBaseStride) rec[lane] = lane == kRecFlags ? (int32_t)kTile32 : 0;
     return;
   }
 
-  bool narrow = true, narrow8 = true;
-  unsigned affine = 0;  // slots whose column is base + lane in every row
+  bool narrow = true, narrow8 = true, step2 = true;
+  unsigned affine = 0;  // slots whose column is base + place in every row
   int ds = 0;
+  int32_t above = 0;  // base of slot u + 2
+  int32_t above1 = 0;
   uint32_t o8[kSlotWords] = {};
 #pragma unroll
   for (int u = kSlots - 1; u >= 0; --u) {
@@ -395,26 +414,35 @@ __global__ __launch_bounds__(kBlock) void k_tile_layout(
       c = col[(int64_t)e * n + i];
       v = val[(int64_t)e * n + i];
     }
-    const int lo = wave_min_i32(has ? c : INT_MAX);
-    const int hi = wave_max_i32(has ? c : INT_MIN);
+    int lo = wave_min_i32(has ? c : INT_MAX);
+    int hi = wave_max_i32(has ? c : INT_MIN);
     const bool used = lo != INT_MAX;
+    // one base for all entries, with every row's place in range: the slot's
+    // window.  An unused slot's window is the tile itself.
+    const int w0 = used ? wave_min_i32(has ? c - lane : INT_MAX) : first;
+    const int w1 = used ? wave_max_i32(has ? c - lane : INT_MIN) : first;
+    const bool window = w0 == w1 && w0 >= 0 && (int64_t)w0 + kTile <= n;
+    const int32_t cc = has ? c : window ? w0 + lane : used ? lo : (int32_t)i;
+    if (window) {
+      lo = w0;
+      hi = w0 + kTile - 1;
+    }
     if (used && hi - lo > 65535) narrow = false;
     if (used && hi - lo > 255) narrow8 = false;
-    const int32_t base = used ? lo : (int32_t)(t * kTile);
+    const int32_t base = used || window ? lo : first;
     if (row) {
-      const int32_t cc = has ? c : (used ? lo : (int32_t)i);
       col[(int64_t)u * n + i] = cc;
       val[(int64_t)u * n + i] = has ? v : 0.0;
       col16[(int64_t)u * n + i] = (uint16_t)(cc - base);
       o8[u / 4] |= ((uint32_t)(cc - base) & 0xffu) << (8 * (u % 4));
       if (has && c == i) ds = u;
     }
-    const int32_t cl = row ? (has ? c : (used ? lo : (int32_t)i)) : base + lane;
-    if (wave_min_i32(cl - base == lane ? 1 : 0) == 1) affine |= 1u << u;
-    if (lane == 0) {
-      cbase[(int64_t)u * ntiles + t] = base;
-      tbase[t * kBaseStride + u] = base;
-    }
+    if (wave_min_i32(!row || cc - base == lane ? 1 : 0) == 1) affine |= 1u << u;
+    if (u % 3 == 0) step2 = step2 && above == base + 1;
+    if (u == kMidSlot) step2 = step2 && wave_min_i32(!row || (has && c == i) ? 1 : 0) == 1;
+    above = above1;
+    above1 = base;
+    if (lane == 0) rec[u] = base;
   }
   if (row) {
     dslot[i] = (uint8_t)ds;
@@ -422,13 +450,28 @@ __global__ __launch_bounds__(kBlock) void k_tile_layout(
     for (int g = 0; g < kSlotWords; ++g) off8[(int64_t)g * n + i] = o8[g];
   }
   if (lane == 0) {
-    tinfo[t] = !narrow ? kTile32 : narrow8 ? kTile8 : kTile16;
-    uint8_t m = 0;  // offset word g: slots 4g .. 4g+3 (below kSlots) all affine
+    uint32_t words = 0;  // offset word g: slots 4g .. 4g+3 (below kSlots) all affine
     for (int g = 0; g < kSlotWords; ++g) {
       const unsigned want = ((1u << 4) - 1u) << (4 * g) & ((1u << kSlots) - 1u);
-      if ((affine & want) == want) m |= (uint8_t)(1u << g);
+      if ((affine & want) == want) words |= 1u << g;
     }
-    amask[t] = narrow8 ? m : 0;
+    const int cls = !narrow ? kTile32 : narrow8 ? kTile8 : kTile16;
+    if (cls != kTile8) words = 0;
+    rec[kRecFlags] =
+        (int32_t)(cls | words << 8 | (words == kAllAffine && step2 ? 1u << 16 : 0u));
+    for (int u = kRecLive; u < kBaseStride; ++u) rec[u] = 0;
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void k_count_classes(int64_t T,
+                                                          const int32_t *__restrict__ trec,
+                                                          unsigned *count) {
+  const int64_t t = gtid();
+  const int cls = t < T ? trec[t * kBaseStride + kRecFlags] & 3 : 3;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const unsigned m = (unsigned)__popcll(__ballot(cls == c));
+    if ((threadIdx.x & 63) == 0 && m) atomicAdd(&count[c], m);
   }
 }
 
@@ -576,20 +619,22 @@ __global__ __launch_bounds__(kBlock) void k_tiles(int C, int S, int64_t W,
   tile_ptr[k] = lo;
 }
 
-// Level::zmask: one wavefront per tile.  Row i's colour begins at the last
-// colour pointer <= i; slot j is live for the tile when some row holds a
-// nonzero there whose column lies below its colour's first row.
+// kRecLive of the tile records: one wavefront per tile.  Slot j is live for
+// the tile when some row holds a nonzero there whose column lies below the
+// first row of the tile's colour.
 __global__ __launch_bounds__(kBlock) void k_zero_mask(int64_t n, int64_t T, int ncolors,
                                                        const int64_t *__restrict__ cptr,
+                                                       const int32_t *__restrict__ rows,
                                                        const int32_t *__restrict__ col,
                                                        const double *__restrict__ val,
-                                                       uint32_t *__restrict__ zmask) {
+                                                       int32_t *__restrict__ trec) {
   const int64_t t = gtid() / 64;
   const int lane = threadIdx.x & 63;
   if (t >= T) return;  // uniform over the wavefront
-  const int64_t i = t * kTile + lane;
+  const int64_t i = rows[2 * t] + lane;
+  const bool row = lane < rows[2 * t + 1];
   int64_t cb = 0;
-  if (i < n) {
+  if (row) {
     int c = 0;
     while (c + 1 < ncolors && cptr[c + 1] <= i) ++c;
     cb = cptr[c];
@@ -597,13 +642,13 @@ __global__ __launch_bounds__(kBlock) void k_zero_mask(int64_t n, int64_t T, int 
   uint32_t m = 0;
   for (int j = 0; j < kSlots; ++j) {
     bool live = false;
-    if (i < n) {
+    if (row) {
       const int64_t k = (int64_t)j * n + i;
       live = val[k] != 0.0 && col[k] < cb;
     }
     if (__ballot(live)) m |= 1u << j;
   }
-  if (lane == 0) zmask[t] = m;
+  if (lane == 0) trec[t * kBaseStride + kRecLive] = (int32_t)m;
 }
 
 }  // namespace
@@ -616,8 +661,14 @@ __global__ __launch_bounds__(kBlock) void k_zero_mask(int64_t n, int64_t T, int 
 // eighth of the list) then streams about one colour block's matrix rows in
 // order, as a colour step does.
 void build_chunks(Problem &P, Level &L, bool interleave) {
-  if (L.chunks) P.arena.release(L.chunks, sizeof(int64_t) * 2 * L.nchunks);
+  auto words = [](int64_t m) { return (size_t)(2 * m + (m + 1) / 2); };
+  if (L.chunks) P.arena.release(L.chunks, sizeof(int64_t) * words(L.nchunks));
   L.chunks = nullptr;
+  // tiles of the colours (Level::color_tile)
+  L.color_tile.assign(1, 0);
+  for (int c = 0; c < L.ncolors; ++c)
+    L.color_tile.push_back(L.color_tile[c] +
+                           (int32_t)((L.color_ptr[c + 1] - L.color_ptr[c] + kTile - 1) / kTile));
   struct Chunk {
     double key;
     int colour;
@@ -636,15 +687,19 @@ void build_chunks(Problem &P, Level &L, bool interleave) {
       return a.key < b.key || (a.key == b.key && a.colour < b.colour);
     });
   L.chunks_interleaved = interleave;
-  std::vector<int64_t> h(2 * v.size());
+  std::vector<int64_t> h(words((int64_t)v.size()));  // [begin, end) pairs, then the tiles
+  int32_t *ht = reinterpret_cast<int32_t *>(h.data() + 2 * v.size());
   for (size_t k = 0; k < v.size(); ++k) {
     h[2 * k] = v[k].begin;
     h[2 * k + 1] = v[k].end;
+    ht[k] = L.color_tile[v[k].colour] +
+            (int32_t)((v[k].begin - L.color_ptr[v[k].colour]) / kTile);
   }
   L.nchunks = (int64_t)v.size();
   L.chunks = P.arena.alloc<int64_t>(h.size());
   HPCGX_HIP(hipMemcpy(L.chunks, h.data(), sizeof(int64_t) * h.size(),
                       hipMemcpyHostToDevice));
+  L.chunk_tile = reinterpret_cast<int32_t *>(L.chunks + 2 * L.nchunks);
 }
 
 void generate_natural(NaturalLevel &N, hipStream_t s) {
@@ -845,39 +900,47 @@ void finalize_level(Problem &P, int l, NaturalLevel &N, int flags,
                                                N.nnz_row, L.col, L.val, L.diag,
                                                L.dslot, L.nnz_row);
   HPCGX_LAUNCHED();
-  // 16-bit column ids where every colour block starts on a tile boundary
-  // (the colour-step and SpMV launches then keep each wavefront in a tile)
-  bool aligned = n >= kTile;
-  for (int c = 0; c <= L.ncolors; ++c) aligned = aligned && L.color_ptr[c] % kTile == 0;
-  if (aligned) {
-    const int64_t T = (n + kTile - 1) / kTile;
+  // Narrow column ids, tile by tile of each colour: the colour-step, SpMV and
+  // transfer launches keep each wavefront in a tile whatever row the colour
+  // starts at.  Not on levels of few rows whose colours fill no tiles: a step
+  // there is a handful of partly filled wavefronts either way.
+  L.aligned = n >= kTile;
+  for (int c = 0; c <= L.ncolors; ++c) L.aligned = L.aligned && L.color_ptr[c] % kTile == 0;
+  if (L.aligned || n >= kNarrowRows) {
+    const int64_t T = L.color_tile[L.ncolors];
     L.ntiles = T;
     L.col16 = P.arena.alloc<uint16_t>((size_t)kSlots * n);
-    L.cbase = P.arena.alloc<int32_t>((size_t)kSlots * T);
-    L.tbase = P.arena.alloc<int32_t>((size_t)kBaseStride * T);
-    L.tinfo = P.arena.alloc<int32_t>(T);
-    L.amask = P.arena.alloc<uint8_t>(T);
+    L.trec = P.arena.alloc<int32_t>((size_t)kBaseStride * T);
     L.off8 = P.arena.alloc<uint32_t>((size_t)kSlotWords * n);
+    // one temporary: colour pointers and tiles, tiles of each class (0), tile rows
+    std::vector<int64_t> head(L.color_ptr);
+    const size_t nc = head.size();
+    head.resize(nc + (nc + 1) / 2 + 2, 0);
+    std::copy(L.color_tile.begin(), L.color_tile.end(), reinterpret_cast<int32_t *>(&head[nc]));
+    const size_t hb = sizeof(int64_t) * head.size();
+    TempBuf temp(hb + sizeof(int32_t) * 2 * T);
+    HPCGX_HIP(hipMemcpyAsync(temp.p, head.data(), hb, hipMemcpyHostToDevice, s));
+    const int64_t *cp = temp.as<int64_t>();
+    const int32_t *ct = reinterpret_cast<const int32_t *>(cp + nc);
+    unsigned *nof = reinterpret_cast<unsigned *>(temp.as<int64_t>() + head.size() - 2);
+    int32_t *rows = reinterpret_cast<int32_t *>(temp.as<int64_t>() + head.size());
+    k_tile_rows<<<grid_for(T), kBlock, 0, s>>>(T, L.ncolors, cp, ct, rows);
+    HPCGX_LAUNCHED();
     const int64_t wpb = kBlock / 64;
     k_tile_layout<<<(unsigned)((T + wpb - 1) / wpb), kBlock, 0, s>>>(
-        n, T, L.iperm, L.col, L.val, L.nnz_row, L.dslot, L.col16, L.off8, L.cbase, L.tbase, L.tinfo,
-        L.amask);
+        n, T, rows, L.iperm, L.col, L.val, L.nnz_row, L.dslot, L.col16, L.off8, L.trec);
     HPCGX_LAUNCHED();
-    std::vector<int32_t> info(T);
-    HPCGX_HIP(hipMemcpyAsync(info.data(), L.tinfo, sizeof(int32_t) * T,
-                             hipMemcpyDeviceToHost, s));
+    k_count_classes<<<grid_for(T), kBlock, 0, s>>>(T, L.trec, nof);
+    HPCGX_LAUNCHED();
+    k_zero_mask<<<(unsigned)((T + wpb - 1) / wpb), kBlock, 0, s>>>(n, T, L.ncolors, cp, rows,
+                                                                   L.col, L.val, L.trec);
+    HPCGX_LAUNCHED();
+    unsigned counts[4] = {};
+    HPCGX_HIP(hipMemcpyAsync(counts, nof, sizeof counts, hipMemcpyDeviceToHost, s));
     HPCGX_HIP(hipStreamSynchronize(s));
-    L.wide_tiles = std::count(info.begin(), info.end(), (int32_t)kTile32);
-    L.byte_tiles = std::count(info.begin(), info.end(), (int32_t)kTile8);
+    L.wide_tiles = counts[kTile32];
+    L.byte_tiles = counts[kTile8];
     L.c16 = true;
-    L.zmask = P.arena.alloc<uint32_t>(T);
-    TempBuf cp(sizeof(int64_t) * (L.ncolors + 1));
-    HPCGX_HIP(hipMemcpyAsync(cp.p, L.color_ptr.data(), sizeof(int64_t) * (L.ncolors + 1),
-                             hipMemcpyHostToDevice, s));
-    k_zero_mask<<<(unsigned)((T + wpb - 1) / wpb), kBlock, 0, s>>>(
-        n, T, L.ncolors, cp.as<int64_t>(), L.col, L.val, L.zmask);
-    HPCGX_LAUNCHED();
-    HPCGX_HIP(hipStreamSynchronize(s));
   }
   HPCGX_HIP(hipStreamSynchronize(s));
   if (P.use_wave && n >= kWaveMinRows)
@@ -967,7 +1030,7 @@ void link_levels(Problem &P, int l, const NaturalLevel &Nf, hipStream_t s) {
   HPCGX_LAUNCHED();
   // Fine-order transfers (Level::ftile, rperm): the fine rows f2c reaches,
   // sorted, with their coarse rows; kept when every kTile of them (the last
-  // group possibly fewer) are consecutive rows from a multiple of kTile.
+  // group possibly fewer) are consecutive rows of one tile, from its first.
   const int64_t nc = C.n;
   std::vector<int32_t> fr(nc), cr(nc);
   {
@@ -988,19 +1051,22 @@ void link_levels(Problem &P, int l, const NaturalLevel &Nf, hipStream_t s) {
     HPCGX_HIP(hipStreamSynchronize(s));
   }
   const int64_t ng = (nc + kTile - 1) / kTile;
-  std::vector<int32_t> ft(ng);
+  std::vector<int32_t> ft(2 * ng);
   bool tiled = true;
+  int c = 0;  // the group's colour
   for (int64_t g = 0; g < ng && tiled; ++g) {
-    const int64_t f0 = fr[g * kTile];
-    tiled = f0 % kTile == 0 && (g == 0 || f0 > fr[g * kTile - 1]);
-    for (int64_t t = g * kTile + 1; t < std::min(nc, (g + 1) * kTile) && tiled; ++t)
-      tiled = fr[t] == f0 + (t - g * kTile);
-    ft[g] = (int32_t)(f0 / kTile);
+    const int64_t f0 = fr[g * kTile], te = std::min(nc, (g + 1) * kTile);
+    while (c + 1 < F.ncolors && F.color_ptr[c + 1] <= f0) ++c;
+    tiled = (f0 - F.color_ptr[c]) % kTile == 0 && (g == 0 || f0 > fr[g * kTile - 1]) &&
+            f0 + (te - g * kTile) <= F.color_ptr[c + 1];
+    for (int64_t t = g * kTile + 1; t < te && tiled; ++t) tiled = fr[t] == f0 + (t - g * kTile);
+    ft[2 * g] = (int32_t)f0;
+    ft[2 * g + 1] = F.color_tile[c] + (int32_t)((f0 - F.color_ptr[c]) / kTile);
   }
   if (tiled) {
-    F.ftile = P.arena.alloc<int32_t>(ng);
+    F.ftile = P.arena.alloc<int32_t>(2 * ng);
     F.rperm = P.arena.alloc<int32_t>(nc);
-    HPCGX_HIP(hipMemcpy(F.ftile, ft.data(), sizeof(int32_t) * ng, hipMemcpyHostToDevice));
+    HPCGX_HIP(hipMemcpy(F.ftile, ft.data(), sizeof(int32_t) * 2 * ng, hipMemcpyHostToDevice));
     HPCGX_HIP(hipMemcpy(F.rperm, cr.data(), sizeof(int32_t) * nc, hipMemcpyHostToDevice));
   }
 }

@@ -63,12 +63,9 @@ void wave_sweep(Problem &P, const Level &L, int dir, const double *r, double *x,
 // unfilled x (launch_symgs_rows_zero for every colour step).
 bool zero_guess_sweep(const Problem &P, int l, int ordering) {
   const Level &L = P.L[l];
-  if (!P.zero_guess || ordering != HPCGX_ORDER_MULTICOLOR || !L.zmask ||
-      (L.wave && P.use_wave) || !use_col16(P, L, 0))
-    return false;
-  for (int c = 0; c < L.ncolors; ++c)
-    if (L.color_ptr[c] % kTile) return false;
-  return true;
+  // launch_symgs_rows_zero reads x at byte offsets of 32 bits
+  return P.zero_guess && ordering == HPCGX_ORDER_MULTICOLOR && !(L.wave && P.use_wave) &&
+         use_col16(P, L) && L.n < ((int64_t)1 << 29);
 }
 
 // The backward sweep visits every row once and leaves its final x, so with
@@ -138,7 +135,7 @@ int64_t rz_partials(const Problem &P, int ordering) {
   for (int c = 0; c < L.ncolors; ++c) {
     const int64_t b = L.color_ptr[c], e = L.color_ptr[c + 1];
     if (e <= b) continue;
-    if (!use_col16(P, L, b)) return 0;
+    if (!use_col16(P, L)) return 0;
     count += rz_slots(e - b);
   }
   return count <= P.nrz_partials ? count : 0;

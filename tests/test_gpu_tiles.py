@@ -1,0 +1,55 @@
+"""Narrow column ids on levels whose colours start anywhere (tiles counted from
+each colour's first row) and the colour steps with all of a row's loads in
+flight: the bits of the 32-bit column ids, which other tests compare with the
+oracle.  Sizes: fewer rows than a tile; colours shorter than a tile and of no
+multiple of it; tiles over several grid lines and planes; one tile per line;
+steps on both sides of the largest all-in-flight step (3 * 2^20 rows)."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [((3, 5, 4), 1), ((9, 7, 5), 1), ((17, 13, 11), 1), ((26, 22, 30), 2), ((40, 24, 56), 4),
+         ((128, 6, 10), 1), ((151, 33, 20), 1), ((258, 30, 14), 2), ((300, 296, 286), 1)]
+
+
+@pytest.mark.parametrize("dims,levels", SIZES)
+def test_tiles_same_bits(dims, levels):
+    import hpcg_amd
+    import torch
+    print("[case]", dims, levels, flush=True)
+    P = hpcg_amd.Problem.generate(*dims, nlevels=levels)
+    big = P.nrow(0) > 1 << 24
+    g = torch.Generator(device="cuda")
+    g.manual_seed(5)
+    outs = []
+    for c16 in (1, 0):
+        P.tune("col16", c16)
+        g.manual_seed(5)
+        got = []
+        for l in range(levels):
+            n = P.nrow(l)
+            r, x = (torch.rand(n, generator=g, dtype=torch.float64, device="cuda") - 0.5
+                    for _ in range(2))
+            y = torch.empty_like(x)
+            P.spmv(x, y, level=l)
+            P.symgs(r, x, level=l, ordering="multicolor")
+            got += [y, x]
+            x4 = x.float()
+            P.symgs32(r.float(), x4, level=l, ordering="multicolor")
+            got.append(x4)
+        z = torch.empty_like(got[1])
+        b = torch.rand(P.nrow(0), generator=g, dtype=torch.float64, device="cuda") - 0.5
+        P.mg(b, z, ordering="multicolor")
+        z4 = torch.empty_like(z.float())
+        P.mg32(b.float(), z4, ordering="multicolor")
+        got += [z, z4]
+        if not big:
+            B = torch.rand((P.nrow(0), 8), generator=g, dtype=torch.float64, device="cuda")
+            Y, Z = torch.empty_like(B), torch.empty_like(B.float())
+            P.spmv_block(B, Y)
+            P.mg32_block(B.float(), Z, ordering="multicolor")
+            got += [Y, Z]
+        outs.append(got)
+    for k, (a, b) in enumerate(zip(*outs)):
+        assert torch.equal(a, b), k
+    P.close()
