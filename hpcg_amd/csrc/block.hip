@@ -157,26 +157,42 @@ __device__ inline void stv(double *p, const double (&v)[S]) {
     *reinterpret_cast<double2 *>(p + 2 * q) = make_double2(v[2 * q], v[2 * q + 1]);
 }
 
-// f(a, c) for every slot of row i in slot order: a the FP16 value (FP32),
-// c the column.  C16: packed words of a narrow tile (the caller's wavefront
-// lies in one tile), else the FP16 array and 32-bit ids.
-template <bool STREAM, bool C16, class F>
-__device__ inline void slots32(const Col16 &C, const uint32_t *__restrict__ vc,
-                               const int32_t *__restrict__ col,
-                               const half_t *__restrict__ val16, int64_t n, int64_t i, F &&f) {
+// f(j, a, xr) for every slot j of row i in order: a the FP16 value (FP32), xr
+// the lane's right-hand sides (column o on) of the slot's row of X.  C16: the
+// caller's wavefront lies in one tile.  On a tile whose offset words are all
+// affine the rows of X follow from the tile's record alone, as a uniform
+// pointer per slot and one lane offset, so their loads do not wait for the
+// matrix words, and the values come two to a word (Level::v16p): half the
+// matrix bytes of the packed words that other narrow tiles read.  256^3, one
+// A X: 2.59 -> 2.36 ms (s = 8), 5.41 -> 4.88 (s = 16); a colour step's
+// average 144.8 -> 135.8 us (s = 8), 265 -> 254 (s = 16).
+template <bool STREAM, bool C16, int S, class T, class F>
+__device__ __attribute__((always_inline)) inline void row_terms(
+    const Col16 &C, const uint32_t *__restrict__ vc, const int32_t *__restrict__ col,
+    const half_t *__restrict__ val16, int64_t n, int64_t i, int o, const T *X, F &&f) {
   const int t = C16 ? C.tile(i) : 0;
-  if (C16 && (C.flags(t) & 3u) != kTile32) {
+  const uint32_t flags = C16 ? C.flags(t) : 0u;
+  if (C16 && C.vp && C.cls(flags) == kTile8 && C.words(flags) == kAllAffine) {
+    const int32_t *__restrict__ base = C.bases(t);
+    const uint32_t off = (uint32_t)(C.place(i) * S + o);
+    uint32_t pv[kPairWords];
+#pragma unroll
+    for (int w = 0; w < kPairWords; ++w) pv[w] = mload<STREAM>(C.vp + (int64_t)w * n + i);
+#pragma unroll
+    for (int j = 0; j < kSlots; ++j)
+      f(j, (float)vc_val(pv[j / 2] >> (16 * (j % 2))), X + (int64_t)base[j] * S + off);
+  } else if (C16 && (flags & 3u) != kTile32) {
     const int32_t *__restrict__ base = C.bases(t);
 #pragma unroll
     for (int j = 0; j < kSlots; ++j) {
       const uint32_t w = mload<STREAM>(vc + (int64_t)j * n + i);
-      f((float)vc_val(w), base[j] + (int32_t)(w >> 16));
+      f(j, (float)vc_val(w), X + (int64_t)(base[j] + (int32_t)(w >> 16)) * S + o);
     }
   } else {
 #pragma unroll
     for (int j = 0; j < kSlots; ++j) {
       const int64_t e = (int64_t)j * n + i;
-      f((float)mload<STREAM>(val16 + e), mload<STREAM>(col + e));
+      f(j, (float)mload<STREAM>(val16 + e), X + (int64_t)mload<STREAM>(col + e) * S + o);
     }
   }
 }
@@ -195,8 +211,8 @@ __device__ __attribute__((always_inline)) inline void bgs32_row(int64_t i, int o
   constexpr int V = 4;
   float sum[V], xv[V];
   ldv<V>(R + i * S + o, sum);
-  slots32<STREAM, C16>(C, vc, col, val16, n, i, [&](float a, int32_t c) {
-    ldv<V>(X + (int64_t)c * S + o, xv);
+  row_terms<STREAM, C16, S>(C, vc, col, val16, n, i, o, X, [&](int, float a, const float *xr) {
+    ldv<V>(xr, xv);
 #pragma unroll
     for (int k = 0; k < V; ++k) sum[k] -= a * xv[k];
   });
@@ -363,6 +379,20 @@ __device__ __attribute__((always_inline)) inline void bgs32_row_zero_live(
   stv<V>(X + i * S + o, sum);
 }
 
+// The launch's workgroups in windows: the hardware hands workgroup b to die
+// b % 8, so with kWin = 8 each die takes eight neighbouring workgroups of
+// every 64 and finds the X rows that they share in its own L2 (the last,
+// partial window keeps its order).  A colour step's average of eight zero and
+// eight full steps, with and without: 136x120x104, s = 16 23.1 us against
+// 28.7; 256^3 128.8 against 134.3 (s = 8), 246 against 248 (s = 16).  Windows
+// of 4 measure the same; each die's own eighth of the rows is slower at 256^3
+// (139.6, s = 8).
+constexpr unsigned kWin = 8;
+__device__ inline unsigned window_block() {
+  const unsigned b = blockIdx.x, q = b % (8 * kWin), w = b - q;
+  return w + 8 * kWin <= gridDim.x ? w + (q % 8) * kWin + q / 8 : b;
+}
+
 // A colour step of the first forward sweep from X = 0, rows [begin, end)
 // (begin a colour's first row).
 // LIVE: the live slots only (bgs32_row_zero_live), else every slot (bgs32_row_zero)
@@ -372,7 +402,7 @@ __global__ __launch_bounds__(kBlock) void k_bgs32_rows_zero(
     const half_t *__restrict__ val16, const float *__restrict__ diag32,
     const float *__restrict__ R, float *X) {
   constexpr int W = S / 4;
-  const int64_t g = gtid();
+  const int64_t g = (int64_t)window_block() * kBlock + threadIdx.x;
   const int64_t i = begin + g / W;
   if (i >= end) return;
   if (LIVE)
@@ -439,20 +469,21 @@ __device__ __attribute__((always_inline)) inline void bgs32_row_pairs(int64_t i,
 }
 
 // One colour step, rows [begin, end) (begin a colour's first row when C16).
-// PAIRS: bgs32_row_pairs on the wavefronts where it applies.
+// PAIRS: bgs32_row_pairs on the wavefronts where it applies.  Bound by the
+// loads in flight: 128 registers (four wavefronts a SIMD) hold about twice
+// the X rows that the compiler keeps by itself (256^3, average of zero and
+// full steps, s = 16: 248 us against 254; two wavefronts: 274).
 template <bool STREAM, int S, bool C16, bool PAIRS = false>
-__global__ __launch_bounds__(kBlock) void k_bgs32_rows(int64_t begin, int64_t end, int64_t n,
-                                                       Col16 C, const uint32_t *__restrict__ vc,
-                                                       const int32_t *__restrict__ col,
-                                                       const half_t *__restrict__ val16,
-                                                       const float *__restrict__ diag32,
-                                                       const float *__restrict__ R, float *X) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void k_bgs32_rows(int64_t begin, int64_t end, int64_t n, Col16 C, const uint32_t *__restrict__ vc,
+                  const int32_t *__restrict__ col, const half_t *__restrict__ val16,
+                  const float *__restrict__ diag32, const float *__restrict__ R, float *X) {
   constexpr int W = S / 4;
-  const int64_t g = gtid();
+  const int64_t g = (int64_t)window_block() * kBlock + threadIdx.x;
   const int64_t i = begin + g / W;
   if (PAIRS) {
     // the wavefront's first row; all its 64 / W rows present (uniform)
-    const int64_t i0 = begin + ((int64_t)blockIdx.x * kBlock + (threadIdx.x & ~63u)) / W;
+    const int64_t i0 = begin + (g & ~(int64_t)63) / W;
     if (i0 + 64 / W <= end && bpairs_tile(C, C.tile(i0))) {
       bgs32_row_pairs<STREAM, S>(i, (int)(g % W) * 4, n, C, vc, diag32, R, X);
       return;
@@ -479,8 +510,8 @@ __global__ __launch_bounds__(kBlock) void k_bresid_restrict32_rows(
   float a[V], xv[V];
 #pragma unroll
   for (int k = 0; k < V; ++k) a[k] = 0.0f;
-  slots32<STREAM, C16>(C, vc, col, val16, n, f, [&](float v, int32_t c) {
-    ldv<V>(XF + (int64_t)c * S + o, xv);
+  row_terms<STREAM, C16, S>(C, vc, col, val16, n, f, o, XF, [&](int, float v, const float *xr) {
+    ldv<V>(xr, xv);
 #pragma unroll
     for (int k = 0; k < V; ++k) a[k] += v * xv[k];
   });
@@ -533,20 +564,16 @@ __device__ inline void bspmv_row(int64_t i, int o, int64_t n, const Col16 &C,
   double xv[V];
 #pragma unroll
   for (int k = 0; k < V; ++k) y[k] = 0.0;
-  const int t = H ? C.tile(i) : 0;
-  if (H && (C.flags(t) & 3u) != kTile32) {
-    const int32_t *__restrict__ base = C.bases(t);
+  if (H && (C.flags(C.tile(i)) & 3u) != kTile32) {
     const int ds = dslot[i];
     const double di = diag[i];
+    row_terms<STREAM, true, S>(C, vc, col, (const half_t *)nullptr, n, i, o, X,
+                               [&](int j, float h, const double *xr) {
+                                 const double a = j == ds ? di : (double)h;
+                                 ldv<V>(xr, xv);
 #pragma unroll
-    for (int j = 0; j < kSlots; ++j) {
-      const uint32_t w = mload<STREAM>(vc + (int64_t)j * n + i);
-      const int32_t c = base[j] + (int32_t)(w >> 16);
-      const double a = j == ds ? di : (double)vc_val(w);
-      ldv<V>(X + (int64_t)c * S + o, xv);
-#pragma unroll
-      for (int k = 0; k < V; ++k) y[k] += a * xv[k];
-    }
+                                 for (int k = 0; k < V; ++k) y[k] += a * xv[k];
+                               });
   } else {
 #pragma unroll
     for (int j = 0; j < kSlots; ++j) {

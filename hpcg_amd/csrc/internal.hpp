@@ -412,6 +412,7 @@ struct Col16 {
   const uint32_t *off8;
   const int32_t *trec;   // Level::trec
   const int32_t *ctile;  // Level::chunk_tile
+  const uint32_t *vp;    // Level::v16p where FP16 value pairs are to be read, else null
   int use8;    // read 8-bit offsets in kTile8 tiles (else their 16-bit ids)
   int affine;  // skip the affine offset words (else load every one)
   int tile0;
@@ -458,8 +459,9 @@ inline Col16 col16_of(const Problem &P, const Level &L, int64_t begin = 0) {
   int t0 = 0;
   for (int c = 0; c < L.ncolors && L.c16; ++c)
     if (L.color_ptr[c] == begin) t0 = L.color_tile[c];
-  return Col16{L.col16, L.off8, L.trec, L.chunk_tile, P.use_c8 ? 1 : 0, P.use_affine ? 1 : 0, t0,
-               begin};
+  return Col16{L.col16, L.off8, L.trec, L.chunk_tile,
+               P.use_pairs && P.use_c8 ? L.v16p : nullptr, P.use_c8 ? 1 : 0, P.use_affine ? 1 : 0,
+               t0, begin};
 }
 // Offset word g of row i (the place-th of its tile) on a kTile8 tile: loaded,
 // or place * 0x01010101 where the tile's word is affine (uniform per tile).

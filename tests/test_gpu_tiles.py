@@ -53,3 +53,29 @@ def test_tiles_same_bits(dims, levels):
     for k, (a, b) in enumerate(zip(*outs)):
         assert torch.equal(a, b), k
     P.close()
+
+
+@pytest.mark.parametrize("s", [4, 8, 16])
+@pytest.mark.parametrize("dims,levels", [((3, 5, 4), 1), ((17, 13, 11), 1), ((40, 24, 56), 4),
+                                         ((130, 66, 62), 2)])
+def test_block_tiles_same_bits(dims, levels, s):
+    """Row pointers from the tile's record and values two to a word, workgroups
+    in windows of 64 (whole windows and a partial last one): the bits of the
+    packed words and of the 32-bit ids."""
+    import hpcg_amd
+    import torch
+    P = hpcg_amd.Problem.generate(*dims, nlevels=levels)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(7)
+    B = torch.rand((P.nrow(0), s), generator=g, dtype=torch.float64, device="cuda") - 0.5
+    outs = []
+    for knobs in ({"x_pairs": 1, "col16": 1}, {"x_pairs": 0, "col16": 1}, {"col16": 0}):
+        for k, v in knobs.items():
+            P.tune(k, v)
+        Y, Z = torch.empty_like(B), torch.empty_like(B.float())
+        P.spmv_block(B, Y)
+        P.mg32_block(B.float(), Z, ordering="multicolor")
+        outs.append((Y, Z))
+    for got in outs[1:]:
+        assert torch.equal(got[0], outs[0][0]) and torch.equal(got[1], outs[0][1])
+    P.close()
