@@ -1202,6 +1202,9 @@ void bsymgs32(Problem &P, int l, int ordering, int s, const float *R, float *X,
         const int c = pass == 0 ? q : L.ncolors - 1 - q;
         const int64_t b = L.color_ptr[c], e = L.color_ptr[c + 1];
         if (e <= b) continue;
+        // the backward sweep's first step repeats the forward sweep's last
+        // (mixed.hip's symgs32)
+        if (pass == 1 && q == 0 && P.use_turn) continue;
         if (pass == 0 && zero_x)
           gs_rows_zero(P, L, s, b, e, R, X, st);
         else
@@ -1212,7 +1215,7 @@ void bsymgs32(Problem &P, int l, int ordering, int s, const float *R, float *X,
       for (int q = 0; q < L.ncolors; ++q) {
         const int c = pass == 0 ? q : L.ncolors - 1 - q;
         const int64_t b = L.color_ptr[c], e = L.color_ptr[c + 1];
-        if (e <= b) continue;
+        if (e <= b || (pass == 1 && q == 0 && P.use_turn)) continue;
         const unsigned g = grid_for((e - b) * s);
         if (L.stream)
           k_bgs32<true><<<g, kBlock, 0, st>>>(b, e, L.n, s, L.col, L.val16, L.diag32, R, X);

@@ -302,6 +302,9 @@ struct Problem {
   // block PCG finest colour steps: slot 3m + 2's x rows from slot 3m's by
   // W-lane moves on affine tiles ("block_pairs")
   bool block_pairs = false;
+  // one launch for the two colour steps at the turn of a symmetric multicolour
+  // sweep ("turn")
+  bool use_turn = true;
   int spmv_dot_blocks = 4096; // persistent grid of the fused SpMV + dot
   // The fused SpMV + dot with one workgroup per row chunk of the fine level
   // ("spmv_dot_chunks"): the p.Ap partial of each chunk, summed in fixed
@@ -498,6 +501,11 @@ void launch_symgs_rows(const Problem &P, const Level &L, int64_t begin, int64_t 
                        const double *r, double *x, hipStream_t s, double *dpart = nullptr);
 // Reference-order symmetric sweep by panels (lex.hip); false (nothing
 // launched) where it does not apply.
+// The last colour's forward and backward step in one launch, device rows
+// [begin, end); zero_x as launch_symgs_rows_zero.  False (nothing launched)
+// where the level has no narrow ids.
+bool launch_symgs_turn(const Problem &P, const Level &L, int64_t begin, int64_t end,
+                       const double *r, double *x, hipStream_t s, double *dpart, bool zero_x);
 bool launch_symgs_lex(Problem &P, int l, const double *r, double *x, hipStream_t s);
 void lex_replace_diag(Level &L, const double *d, hipStream_t s);
 void launch_symgs_list(const Level &L, const int32_t *rows, int64_t count,

@@ -562,6 +562,97 @@ __device__ inline void gs_row_zero(const Col16 &C, uint32_t zm, int64_t begin, i
   x[i] = sum / d;
 }
 
+// The turn of a symmetric sweep: the last colour's forward step and the first
+// backward step, the same colour's, in one launch.  Rows of one colour share
+// no matrix entry, so between the two updates of a row nothing that it reads
+// changes but its own x: the row is read once (as gs_row_deep, every load in
+// flight) and its products summed twice, the second time with the first
+// update's result in the diagonal's.
+// ZERO: the forward sweep began from x = 0, so x is read below `begin` only
+// (gs_row_zero: the last colour's other columns all lie there, and a slot at
+// or beyond `begin` is the row itself or holds no value).
+// It costs what one step costs (both are bound by the matrix bytes), also
+// above kDeepRows, where the register-capped step is the faster single one:
+// a sweep from x = 0 at 256^3 1356 -> 1238 us, any other 1722 -> 1599; one at
+// 96x104x112 139 -> 129; from x = 0 at 384x448x416 5967 -> 5469.
+template <bool STREAM, bool ZERO>
+__device__ inline double gs_row_turn(const Col16 &C, int64_t begin, int64_t i, int64_t n,
+                                     const int32_t *__restrict__ col,
+                                     const double *__restrict__ val,
+                                     const double *__restrict__ diag,
+                                     const uint8_t *__restrict__ dslot,
+                                     const double *__restrict__ r, double *x) {
+  double v[kSlots], xs[kSlots];
+#pragma unroll
+  for (int j = 0; j < kSlots; ++j) v[j] = mload<STREAM>(val + (int64_t)j * n + i);
+  const double d = mload<STREAM>(diag + i);
+  const double xi = ZERO ? 0.0 : x[i];
+  const double ri = r[i];
+  const int t = C.tile(i);
+  const uint32_t flags = C.flags(t);
+  const int32_t *__restrict__ base = C.bases(t);
+  const int cls = C.cls(flags);
+  const BufView xv = buf_view(x, (uint32_t)begin * 8u);
+  auto get = [&](int32_t b, uint32_t o) {  // x[b + o], b uniform
+    return ZERO ? buf_f64<false>(xv, (uint32_t)b * 8u + o * 8u) : (x + b)[o];
+  };
+  if (cls == kTile8 && C.words(flags) == kAllAffine) {
+    const uint32_t pos = (uint32_t)C.place(i);
+#pragma unroll
+    for (int j = 0; j < kSlots; ++j) xs[j] = get(base[j], pos);
+  } else if (cls == kTile8) {
+    uint32_t w[kSlotWords];
+#pragma unroll
+    for (int g = 0; g < kSlotWords; ++g) w[g] = mload<STREAM>(C.off8 + (int64_t)g * n + i);
+#pragma unroll
+    for (int j = 0; j < kSlots; ++j)
+      xs[j] = get(base[j], (w[j / 4] >> (8 * (j % 4))) & 0xffu);
+  } else {
+    int32_t c[kSlots];
+#pragma unroll
+    for (int j = 0; j < kSlots; ++j) {
+      const int64_t k = (int64_t)j * n + i;
+      c[j] = cls == kTile32 ? mload<STREAM>(col + k)
+                            : base[j] + (int32_t)mload<STREAM>(C.off + k);
+    }
+#pragma unroll
+    for (int j = 0; j < kSlots; ++j) xs[j] = get(0, (uint32_t)c[j]);
+  }
+  double sum = ri;
+#pragma unroll
+  for (int j = 0; j < kSlots; ++j) {
+    xs[j] = v[j] * xs[j];
+    sum -= xs[j];
+  }
+  sum += xi * d;
+  const int ds = dslot[i];
+  const double z = sum / d, zd = z * d;
+  sum = ri;
+#pragma unroll
+  for (int j = 0; j < kSlots; ++j) sum -= j == ds ? zd : xs[j];
+  sum += zd;
+  x[i] = sum / d;
+  return sum / d;
+}
+
+// RZ: also the r.z partials of the backward step, as k_gs_rz16.
+template <bool STREAM, bool ZERO, bool RZ>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_gs_turn(
+    int64_t begin, int64_t end, int64_t n, Col16 C, const int32_t *__restrict__ col,
+    const double *__restrict__ val, const double *__restrict__ diag,
+    const uint8_t *__restrict__ dslot, const double *__restrict__ r, double *x, double *__restrict__ dpart) {
+  const int64_t i = begin + gtid();
+  double s = 0.0;
+  if (i < end) {
+    const double z = gs_row_turn<STREAM, ZERO>(C, begin, i, n, col, val, diag, dslot, r, x);
+    if (RZ) s = r[i] * z;
+  }
+  if (!RZ) return;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+  if ((threadIdx.x & 63) == 0 && i < end) dpart[(i - begin) / 64] = s;
+}
+
 constexpr int kLiveChunk = 8;  // live slots per chunk (8 measured faster than 16)
 
 // gs_row_zero over the live slots only ("zero_live"): kRecLive's set
@@ -1575,6 +1666,29 @@ void launch_symgs_rows(const Problem &P, const Level &L, int64_t begin, int64_t 
     k_gs_range<false, false><<<g, kBlock, 0, s>>>(begin, end, L.n, L.col,
                                                   L.val, r, x, L.xcd);
   HPCGX_LAUNCHED();
+}
+
+bool launch_symgs_turn(const Problem &P, const Level &L, int64_t begin, int64_t end,
+                       const double *r, double *x, hipStream_t s, double *dpart, bool zero_x) {
+  if (!use_col16(P, L)) return false;
+  if (end <= begin) return true;
+  const Col16 C = col16_of(P, L, begin);
+  const unsigned g = grid_for(end - begin);
+#define HPCGX_TURN(ST, ZE, RZ)                                                                 \
+  k_gs_turn<ST, ZE, RZ><<<g, kBlock, 0, s>>>(begin, end, L.n, C, L.col, L.val, L.diag,         \
+                                             L.dslot, r, x, dpart)
+#define HPCGX_TURNS(ST)                                                                        \
+  do {                                                                                         \
+    if (zero_x && dpart) HPCGX_TURN(ST, true, true);                                           \
+    else if (zero_x) HPCGX_TURN(ST, true, false);                                              \
+    else if (dpart) HPCGX_TURN(ST, false, true);                                               \
+    else HPCGX_TURN(ST, false, false);                                                         \
+  } while (0)
+  if (L.stream) HPCGX_TURNS(true); else HPCGX_TURNS(false);
+#undef HPCGX_TURNS
+#undef HPCGX_TURN
+  HPCGX_LAUNCHED();
+  return true;
 }
 
 bool launch_symgs_rows_zero(const Problem &P, const Level &L, int64_t begin, int64_t end,

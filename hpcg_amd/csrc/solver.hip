@@ -85,15 +85,23 @@ void symgs(Problem &P, int l, int ordering, const double *r, double *x,
     wave_sweep(P, L, 0, r, x, s);
     wave_sweep(P, L, 1, r, x, s);
   } else if (ordering == HPCGX_ORDER_MULTICOLOR) {
-    for (int c = 0; c < L.ncolors; ++c) {
+    // the turn: the last colour's two steps in one launch (not where each
+    // colour step is timed by itself)
+    const int last = L.ncolors - 1;
+    const bool turn = P.use_turn && last > 0 && !(L.finest && P.klog.on);
+    bool turned = false;
+    for (int c = 0; c <= last; ++c) {
+      if (c == last && turn)
+        turned = launch_symgs_turn(P, L, L.color_ptr[c], L.color_ptr[c + 1], r, x, s, rz, zero_x);
+      if (turned) break;
       if (zero_x)
         (void)launch_symgs_rows_zero(P, L, L.color_ptr[c], L.color_ptr[c + 1], r, x, s);
       else
         colour_step(P, L, c, r, x, s);
     }
     int64_t off = 0;
-    for (int c = L.ncolors - 1; c >= 0; --c) {
-      colour_step(P, L, c, r, x, s, rz ? rz + off : nullptr);
+    for (int c = last; c >= 0; --c) {
+      if (c < last || !turned) colour_step(P, L, c, r, x, s, rz ? rz + off : nullptr);
       off += rz_slots(L.color_ptr[c + 1] - L.color_ptr[c]);
     }
   } else if (!launch_symgs_lex(P, l, r, x, s)) {

@@ -454,6 +454,14 @@ int hpcgx_cg_fleet(hpcgx_problem *p, int ordering, const double *b, double *x, i
  *                      leaves r.z partials; bit 2: the FP32 V-cycle's colour
  *                      steps on FP16 value pairs; bit 3: the FP64 colour
  *                      steps of the coarser levels (default 3; the same bits)
+ *   "turn"             1/0: the turn of a symmetric multicolour sweep, where
+ *                      the backward sweep begins with the colour that the
+ *                      forward sweep ended with, runs both updates of that
+ *                      colour in one launch (FP64), or one of them where the
+ *                      second repeats the first (FP32, whose update does not
+ *                      read the row's own x); not where the finest level's
+ *                      FP64 colour steps are being timed (default 1; the
+ *                      same bits)
  *   "block_pairs"      1/0: the block PCG's finest colour steps at s = 8,
  *                      on tiles where "x_pairs" applies, take slot 3m + 2's
  *                      neighbour rows from slot 3m's moved one row (2

@@ -79,3 +79,45 @@ def test_block_tiles_same_bits(dims, levels, s):
     for got in outs[1:]:
         assert torch.equal(got[0], outs[0][0]) and torch.equal(got[1], outs[0][1])
     P.close()
+
+
+@pytest.mark.parametrize("dims,levels", SIZES)
+def test_turn_same_bits(dims, levels):
+    """The turn of a symmetric sweep in one launch: the bits of the two colour
+    steps, from any x and from x = 0, with narrow and 32-bit ids (where the
+    FP64 steps stay apart), and r.z as a sum over the same partials."""
+    import hpcg_amd
+    import torch
+    print("[case]", dims, levels, flush=True)
+    P = hpcg_amd.Problem.generate(*dims, nlevels=levels)
+    n = P.nrow(0)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(9)
+    b, x0 = (torch.rand(n, generator=g, dtype=torch.float64, device="cuda") - 0.5
+             for _ in range(2))
+    s = 8 if n < 1 << 20 else 0
+    B = torch.rand((n, 10), generator=g, dtype=torch.float32, device="cuda") - 0.5
+    for c16 in (1, 0):
+        P.tune("col16", c16)
+        outs = []
+        for turn in (1, 0):
+            P.tune("turn", turn)
+            x, z, z4, x4 = x0.clone(), torch.empty_like(b), torch.empty_like(B[:, 0]), x0.float()
+            P.symgs(b, x, ordering="multicolor")
+            P.mg(b, z, ordering="multicolor")
+            P.symgs32(b.float(), x4, ordering="multicolor")
+            P.mg32(b.float(), z4, ordering="multicolor")
+            got = [x, z, x4, z4]
+            for lo, hi in ((0, 8), (8, 10)) if s else ():
+                R = B[:, lo:hi].contiguous()
+                Z = torch.empty_like(R)
+                P.mg32_block(R, Z, ordering="multicolor")
+                got.append(Z)
+            for solve in (P.cg, P.cg_mixed):
+                y = torch.zeros_like(b)
+                got.append(torch.tensor(float(solve(b, y, max_iter=4, tolerance=0.0)["normr"])))
+                got.append(y)
+            outs.append(got)
+        for k, (p, q) in enumerate(zip(*outs)):
+            assert torch.equal(p, q), (c16, k)
+    P.close()
