@@ -446,6 +446,10 @@ int hpcgx_tune(hpcgx_problem *p, const char *key, double value) {
       P.zero_live = (int)value;
       return;
     }
+    if (k == "tail") {
+      P.use_tail = value != 0.0;
+      return;
+    }
     if (k == "turn") {
       P.use_turn = value != 0.0;
       return;

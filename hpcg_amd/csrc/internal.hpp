@@ -305,6 +305,8 @@ struct Problem {
   // one launch for the two colour steps at the turn of a symmetric multicolour
   // sweep ("turn")
   bool use_turn = true;
+  // the V-cycle's smallest levels in one launch (tail.hip; "tail")
+  bool use_tail = true;
   int spmv_dot_blocks = 4096; // persistent grid of the fused SpMV + dot
   // The fused SpMV + dot with one workgroup per row chunk of the fine level
   // ("spmv_dot_chunks"): the p.Ap partial of each chunk, summed in fixed
@@ -501,6 +503,11 @@ void launch_symgs_rows(const Problem &P, const Level &L, int64_t begin, int64_t 
                        const double *r, double *x, hipStream_t s, double *dpart = nullptr);
 // Reference-order symmetric sweep by panels (lex.hip); false (nothing
 // launched) where it does not apply.
+// The multicolour V-cycle from level l down in one launch (tail.hip), rz as
+// symgs; false (nothing launched) where the levels are too large for it.
+bool launch_tail(const Problem &P, int l, const double *r, double *x, hipStream_t s, double *rz);
+bool launch_tail32(const Problem &P, int l, const float *r, float *x, hipStream_t s, double *rz,
+                   const double *r64);
 // The last colour's forward and backward step in one launch, device rows
 // [begin, end); zero_x as launch_symgs_rows_zero.  False (nothing launched)
 // where the level has no narrow ids.

@@ -879,13 +879,14 @@ void spmv32(const Problem &P, const Level &L, const float *x, float *y, hipStrea
 void mg32(Problem &P, int l, int ordering, const float *r, float *x,
           hipStream_t s, double *rz, const double *r64) {
   Level &L = P.L[l];
+  if (rz && l + 1 >= P.nlevels)
+    throw Error(HPCGX_EINVAL, "r.z partials come from a post-smoother sweep");
+  if (ordering == HPCGX_ORDER_MULTICOLOR && launch_tail32(P, l, r, x, s, rz, r64)) return;
   const bool zg = zero_guess_sweep32(P, l, ordering);
   if (!zg) {
     k_fill32<<<grid_for(L.n), kBlock, 0, s>>>(x, L.n);
     HPCGX_LAUNCHED();
   }
-  if (rz && l + 1 >= P.nlevels)
-    throw Error(HPCGX_EINVAL, "r.z partials come from a post-smoother sweep");
   symgs32(P, l, ordering, r, x, s, zg);
   if (l + 1 < P.nlevels) {
     const unsigned g = grid_for(L.nc);

@@ -121,6 +121,7 @@ void symgs(Problem &P, int l, int ordering, const double *r, double *x,
 void mg(Problem &P, int l, int ordering, const double *r, double *x,
         hipStream_t s, double *rz) {
   Level &L = P.L[l];
+  if (ordering == HPCGX_ORDER_MULTICOLOR && launch_tail(P, l, r, x, s, rz)) return;
   const bool zg = zero_guess_sweep(P, l, ordering);
   if (!zg) launch_fill(x, L.n, 0.0, s);                 // :42
   if (l + 1 < P.nlevels) {
