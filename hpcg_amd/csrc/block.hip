@@ -379,20 +379,6 @@ __device__ __attribute__((always_inline)) inline void bgs32_row_zero_live(
   stv<V>(X + i * S + o, sum);
 }
 
-// The launch's workgroups in windows: the hardware hands workgroup b to die
-// b % 8, so with kWin = 8 each die takes eight neighbouring workgroups of
-// every 64 and finds the X rows that they share in its own L2 (the last,
-// partial window keeps its order).  A colour step's average of eight zero and
-// eight full steps, with and without: 136x120x104, s = 16 23.1 us against
-// 28.7; 256^3 128.8 against 134.3 (s = 8), 246 against 248 (s = 16).  Windows
-// of 4 measure the same; each die's own eighth of the rows is slower at 256^3
-// (139.6, s = 8).
-constexpr unsigned kWin = 8;
-__device__ inline unsigned window_block() {
-  const unsigned b = blockIdx.x, q = b % (8 * kWin), w = b - q;
-  return w + 8 * kWin <= gridDim.x ? w + (q % 8) * kWin + q / 8 : b;
-}
-
 // A colour step of the first forward sweep from X = 0, rows [begin, end)
 // (begin a colour's first row).
 // LIVE: the live slots only (bgs32_row_zero_live), else every slot (bgs32_row_zero)
@@ -402,7 +388,7 @@ __global__ __launch_bounds__(kBlock) void k_bgs32_rows_zero(
     const half_t *__restrict__ val16, const float *__restrict__ diag32,
     const float *__restrict__ R, float *X) {
   constexpr int W = S / 4;
-  const int64_t g = (int64_t)window_block() * kBlock + threadIdx.x;
+  const int64_t g = window_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   const int64_t i = begin + g / W;
   if (i >= end) return;
   if (LIVE)
@@ -479,7 +465,7 @@ void k_bgs32_rows(int64_t begin, int64_t end, int64_t n, Col16 C, const uint32_t
                   const int32_t *__restrict__ col, const half_t *__restrict__ val16,
                   const float *__restrict__ diag32, const float *__restrict__ R, float *X) {
   constexpr int W = S / 4;
-  const int64_t g = (int64_t)window_block() * kBlock + threadIdx.x;
+  const int64_t g = window_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   const int64_t i = begin + g / W;
   if (PAIRS) {
     // the wavefront's first row; all its 64 / W rows present (uniform)

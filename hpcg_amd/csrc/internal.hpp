@@ -468,6 +468,23 @@ inline Col16 col16_of(const Problem &P, const Level &L, int64_t begin = 0) {
                P.use_pairs && P.use_c8 ? L.v16p : nullptr, P.use_c8 ? 1 : 0, P.use_affine ? 1 : 0,
                t0, begin};
 }
+// Workgroup b of G in windows: the hardware hands workgroup b to die b % 8, so
+// with kWin = 8 each die takes eight neighbouring workgroups of every 64 and
+// finds the x that they share in its own L2 (the last, partial window keeps
+// its order).  Plain order / windows, us: a one-level FP32 V-cycle at 256^3
+// 470 / 434, at 192x160x176 196 / 187; an FP64 one 1240 / 1192 and 433 / 419;
+// SpMV of 1.1M rows 47 / 42; a block colour step (average of zero and full
+// ones) at 136x120x104, s = 16 28.7 / 23.1, at 256^3 134.3 / 128.8 (s = 8).
+// The SpMV of a matrix beyond the last-level cache gains nothing (838 / 840 at
+// 256^3), nor do colour steps above kDeepRows, and both keep the plain order.
+// Windows of 4 and 16 measure the same in FP64, 446 and 468 in FP32 at 256^3;
+// each die's own eighth of the rows (xcd_block) is slower than windows.
+constexpr int64_t kWin = 8;
+__device__ inline int64_t window_block(int64_t b, int64_t G) {
+  const int64_t q = b % (8 * kWin), w = b - q;
+  return w + 8 * kWin <= G ? w + (q % 8) * kWin + q / 8 : b;
+}
+
 // Offset word g of row i (the place-th of its tile) on a kTile8 tile: loaded,
 // or place * 0x01010101 where the tile's word is affine (uniform per tile).
 template <bool STREAM>

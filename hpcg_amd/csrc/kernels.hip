@@ -119,6 +119,12 @@ __device__ inline int64_t xcd_block(int64_t b, int64_t G, bool on) {
   return (b % 8) * (G8 / 8) + b / 8;
 }
 
+// xcd_block, with windows in place of the plain order where `win`
+__device__ inline int64_t xcd_window(bool on, bool win) {
+  return win && !on ? window_block(blockIdx.x, gridDim.x)
+                    : xcd_block(blockIdx.x, gridDim.x, on);
+}
+
 // Sum over the workgroup in a fixed tree: 64-lane shuffles, then the four
 // wavefront sums in order.  Result valid in thread 0.
 __device__ inline double block_sum(double v) {
@@ -167,7 +173,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv(
     const int64_t *__restrict__ chunks, int64_t n, Col16 C,
     const int32_t *__restrict__ col, const double *__restrict__ val,
     const double *__restrict__ x, double *__restrict__ y, bool xcd) {
-  const int64_t b = xcd_block(blockIdx.x, gridDim.x, xcd);
+  const int64_t b = xcd_window(xcd, !STREAM);
   if (C16) C.chunk(chunks, b);
   const int64_t i = chunks[2 * b] + threadIdx.x;
   if (i < chunks[2 * b + 1])
@@ -391,10 +397,11 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
 // and selects.
 //
 // kDeepRows, the largest step that runs so, is where the two cross (us a step,
-// k_gs_range16 / this, one job): 32768 rows 7.7 / 4.6, 137280 12.8 / 10.1,
-// 262144 20.5 / 16.2, 884736 50.0 / 45.4, 2.1M 107.3 / 106.7, 4.1M 237.4 /
-// 245.7, 16.8M 889 / 934.
-constexpr int64_t kDeepRows = (int64_t)3 << 20;
+// k_gs_range16 / this, the medians of several allocations from 3.5M rows on):
+// 32768 rows 7.7 / 4.6, 137280 12.8 / 10.1, 262144 20.5 / 16.2, 884736 50.0 /
+// 45.4, 2.1M 107.3 / 101, 3.55M 189 / 170, 4.7M 266 / 258, 8.9M 474 / 487,
+// 16.8M 921 / 923.
+constexpr int64_t kDeepRows = (int64_t)6 << 20;
 template <bool STREAM>
 __device__ inline double gs_row_deep(const Col16 &C, int64_t i, int64_t n,
                                      const int32_t *__restrict__ col,
@@ -446,7 +453,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 4))) 
     int64_t begin, int64_t end, int64_t n, Col16 C, const int32_t *__restrict__ col,
     const double *__restrict__ val, const double *__restrict__ diag,
     const double *__restrict__ r, double *x, double *__restrict__ dpart) {
-  const int64_t i = begin + gtid();
+  const int64_t i = begin + window_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   double s = 0.0;
   if (i < end) {
     const double z = gs_row_deep<STREAM>(C, i, n, col, val, diag, r, x);
@@ -641,7 +648,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 4))) 
     int64_t begin, int64_t end, int64_t n, Col16 C, const int32_t *__restrict__ col,
     const double *__restrict__ val, const double *__restrict__ diag,
     const uint8_t *__restrict__ dslot, const double *__restrict__ r, double *x, double *__restrict__ dpart) {
-  const int64_t i = begin + gtid();
+  const int64_t i = begin + window_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   double s = 0.0;
   if (i < end) {
     const double z = gs_row_turn<STREAM, ZERO>(C, begin, i, n, col, val, diag, dslot, r, x);
@@ -749,7 +756,7 @@ template <bool STREAM, bool FINEST, int BS, bool LIVE = false>
 __global__ __launch_bounds__(BS) void k_gs_zero16(
     int64_t begin, int64_t end, int64_t n, Col16 C, const int32_t *__restrict__ col,
     const double *__restrict__ val, const double *__restrict__ diag, const double *__restrict__ r, double *x, bool xcd) {
-  const int64_t i = begin + xcd_block(blockIdx.x, gridDim.x, xcd) * BS + threadIdx.x;
+  const int64_t i = begin + xcd_window(xcd, true) * BS + threadIdx.x;
   if (i >= end) return;
   if (LIVE)
     gs_row_zero_live<STREAM, kLiveChunk>(C, begin, i, n, col, val, diag, r, x);
@@ -1151,7 +1158,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_dot_c(
     const int64_t *__restrict__ chunks, int64_t n, Col16 C, const int32_t *__restrict__ col,
     const double *__restrict__ val, const double *__restrict__ p, double *__restrict__ Ap,
     double *__restrict__ cpart, bool xcd) {
-  const int64_t b = xcd_block(blockIdx.x, gridDim.x, xcd);
+  const int64_t b = xcd_window(xcd, !STREAM);
   if (C16) C.chunk(chunks, b);
   const int64_t i = chunks[2 * b] + threadIdx.x;
   const int64_t end = chunks[2 * b + 1];
@@ -1236,7 +1243,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_dot_hc(
     const double *__restrict__ diag, const int32_t *__restrict__ col,
     const double *__restrict__ val, const double *__restrict__ p, double *__restrict__ Ap,
     double *__restrict__ cpart, bool xcd) {
-  const int64_t b = xcd_block(blockIdx.x, gridDim.x, xcd);
+  const int64_t b = xcd_window(xcd, !STREAM);
   C.chunk(chunks, b);
   const int64_t i = chunks[2 * b] + threadIdx.x;
   double s = 0.0;
@@ -1460,7 +1467,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_resid(
     const int64_t *__restrict__ chunks, int64_t n, Col16 C, const int32_t *__restrict__ col,
     const double *__restrict__ val, const double *__restrict__ x, const double *__restrict__ b,
     double *__restrict__ r, float *__restrict__ r32, double *__restrict__ cpart, bool xcd) {
-  const int64_t blk = xcd_block(blockIdx.x, gridDim.x, xcd);
+  const int64_t blk = xcd_window(xcd, !STREAM);
   if (C16) C.chunk(chunks, blk);
   const int64_t i = chunks[2 * blk] + threadIdx.x;
   double s = 0.0;
@@ -1486,7 +1493,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_resid_h(
     const double *__restrict__ diag, const int32_t *__restrict__ col,
     const double *__restrict__ val, const double *__restrict__ x, const double *__restrict__ b,
     double *__restrict__ r, float *__restrict__ r32, double *__restrict__ cpart, bool xcd) {
-  const int64_t blk = xcd_block(blockIdx.x, gridDim.x, xcd);
+  const int64_t blk = xcd_window(xcd, !STREAM);
   C.chunk(chunks, blk);
   const int64_t i = chunks[2 * blk] + threadIdx.x;
   double s = 0.0;

@@ -494,9 +494,10 @@ __global__ __launch_bounds__(kBlock) void k_pack_v16p(int64_t n, const half_t *_
 }
 
 // The hardware hands workgroup b to XCD b % 8; with `xcd` XCD k takes the
-// k-th eighth of the rows in order (its L2 then holds its own x window).
+// k-th eighth of the rows in order (its L2 then holds its own x window), else
+// windows of them.
 __device__ inline int64_t xcd_block(int64_t b, int64_t G, bool on) {
-  if (!on) return b;
+  if (!on) return window_block(b, G);
   const int64_t G8 = G - G % 8;
   if (b >= G8) return b;
   return (b % 8) * (G8 / 8) + b / 8;

@@ -3,13 +3,13 @@ each colour's first row) and the colour steps with all of a row's loads in
 flight: the bits of the 32-bit column ids, which other tests compare with the
 oracle.  Sizes: fewer rows than a tile; colours shorter than a tile and of no
 multiple of it; tiles over several grid lines and planes; one tile per line;
-steps on both sides of the largest all-in-flight step (3 * 2^20 rows)."""
+steps on both sides of the largest all-in-flight step (6 * 2^20 rows)."""
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 SIZES = [((3, 5, 4), 1), ((9, 7, 5), 1), ((17, 13, 11), 1), ((26, 22, 30), 2), ((40, 24, 56), 4),
-         ((128, 6, 10), 1), ((151, 33, 20), 1), ((258, 30, 14), 2), ((300, 296, 286), 1)]
+         ((128, 6, 10), 1), ((151, 33, 20), 1), ((258, 30, 14), 2), ((400, 368, 344), 1)]
 
 
 @pytest.mark.parametrize("dims,levels", SIZES)
