@@ -289,7 +289,7 @@ struct Problem {
   // bit 0 the FP64 finest level, bit 1 the FP64 coarser levels, bit 2 the
   // FP32 V-cycle, bit 3 the block V-cycle
   int zero_live = 11;
-  // the mixed CG's FP64 residual recompute in one pass ("resid_fused")
+  // CG's FP64 residuals in one pass ("resid_fused")
   bool resid_fused = true;
   // the mixed CG's FP64 A p reads 8-bit tiles as FP16 value pairs and 8-bit
   // offsets, not 4-byte offset/value words ("hc_pairs")
@@ -596,8 +596,8 @@ void launch_update_p32(int64_t n, const float *z, double *p, const double *scala
                        hipStream_t s, bool stream);
 void launch_update_p(int64_t n, const double *z, double *p,
                      const double *scalars, hipStream_t s, bool stream);
-// r = b - A x on the finest level L with r32 = (float)r and r.r (into the
-// scalars) in one pass over the row chunks; false (nothing launched) where
+// r = b - A x on the finest level L with r32 = (float)r (unless null; with it,
+// from FP16 values where they are exact) and r.r (into the scalars) in one pass over the row chunks; false (nothing launched) where
 // the chunk partials do not cover L
 bool launch_residual_fused(Problem &P, const Level &L, const double *b, const double *x,
                            double *r, float *r32, hipStream_t s);

@@ -167,8 +167,9 @@ __device__ inline double row_dot16(const Col16 &C, const int32_t *__restrict__ c
                                    const double *__restrict__ x, int64_t n,
                                    int64_t i, int64_t end = 0);
 
-// C16: 16-bit column ids (chunks start at multiples of kTile).
-template <bool STREAM, bool C16>
+// C16: narrow column ids (a chunk starts at a tile).  PAIRS: shared x windows on
+// the tiles that have them (affine_pairs_row; 13.4M rows 675 -> 644 us).
+template <bool STREAM, bool C16, bool PAIRS = false>
 __global__ __launch_bounds__(kBlock) void k_spmv(
     const int64_t *__restrict__ chunks, int64_t n, Col16 C,
     const int32_t *__restrict__ col, const double *__restrict__ val,
@@ -176,8 +177,10 @@ __global__ __launch_bounds__(kBlock) void k_spmv(
   const int64_t b = xcd_window(xcd, !STREAM);
   if (C16) C.chunk(chunks, b);
   const int64_t i = chunks[2 * b] + threadIdx.x;
-  if (i < chunks[2 * b + 1])
-    y[i] = C16 ? row_dot16<STREAM>(C, col, val, x, n, i) : row_dot<STREAM>(col, val, x, n, i);
+  const int64_t end = chunks[2 * b + 1];
+  if (i < end)
+    y[i] = C16 ? row_dot16<STREAM, PAIRS>(C, col, val, x, n, i, end)
+               : row_dot<STREAM>(col, val, x, n, i);
 }
 
 // One Gauss-Seidel row update in the reference's form
@@ -1458,11 +1461,13 @@ __global__ __launch_bounds__(kBlock) void k_residual0(
   grid_finish(s, partials, ticket, scalars, &scalars[kNormr2], kFinishStore);
 }
 
-// r = b - A x, r32 = (float)r and one r.r partial per row chunk in one pass
-// (CG.cpp:86-89's residual, as the mixed CG recomputes it in FP64): k_spmv's
-// row sums, k_residual0's r and the FP32 rounding, without writing and
-// reading A x and r again; k_chunk_dot sums the partials.
-template <bool STREAM, bool C16>
+// r = b - A x, r32 = (float)r (unless null) and one r.r partial per row chunk
+// in one pass (CG.cpp:86-89's residual, and as the mixed CG recomputes it in
+// FP64): k_spmv's row sums, k_residual0's r and the FP32 rounding, without
+// copying x, writing and reading A x and reading r again; k_chunk_dot sums the
+// partials.  A CG call's start at 256^3 1182 -> 824 us
+// (FP64), 1225 -> 418 us (mixed).
+template <bool STREAM, bool C16, bool PAIRS = false>
 __global__ __launch_bounds__(kBlock) void k_spmv_resid(
     const int64_t *__restrict__ chunks, int64_t n, Col16 C, const int32_t *__restrict__ col,
     const double *__restrict__ val, const double *__restrict__ x, const double *__restrict__ b,
@@ -1472,10 +1477,11 @@ __global__ __launch_bounds__(kBlock) void k_spmv_resid(
   const int64_t i = chunks[2 * blk] + threadIdx.x;
   double s = 0.0;
   if (i < chunks[2 * blk + 1]) {
-    const double y = C16 ? row_dot16<STREAM>(C, col, val, x, n, i) : row_dot<STREAM>(col, val, x, n, i);
+    const double y = C16 ? row_dot16<STREAM, PAIRS>(C, col, val, x, n, i, chunks[2 * blk + 1])
+                         : row_dot<STREAM>(col, val, x, n, i);
     const double ri = mload<STREAM>(b + i) + -1.0 * y;
     mstore<STREAM>(r + i, ri);
-    mstore<STREAM>(r32 + i, (float)ri);
+    if (r32) mstore<STREAM>(r32 + i, (float)ri);
     s = ri * ri;
   }
   s = block_sum(s);
@@ -1547,7 +1553,9 @@ void launch_spmv(const Problem &P, const Level &L, const double *x, double *y,
   const unsigned g = (unsigned)L.nchunks;
   const Col16 C = col16_of(P, L);
   const bool c16 = use_col16(P, L);
-  if (L.stream && c16)
+  if (L.stream && c16 && L.finest && (P.x_pairs & 1))
+    k_spmv<true, true, true><<<g, kBlock, 0, s>>>(L.chunks, L.n, C, L.col, L.val, x, y, L.xcd);
+  else if (L.stream && c16)
     k_spmv<true, true><<<g, kBlock, 0, s>>>(L.chunks, L.n, C, L.col, L.val, x, y, L.xcd);
   else if (L.stream)
     k_spmv<true, false><<<g, kBlock, 0, s>>>(L.chunks, L.n, C, L.col, L.val, x, y, L.xcd);
@@ -2045,7 +2053,7 @@ bool launch_residual_fused(Problem &P, const Level &L, const double *b, const do
   const unsigned g = (unsigned)L.nchunks;
   const Col16 C = col16_of(P, L);
   const bool c16 = use_col16(P, L);
-  const bool h = P.hc_pairs && L.vc && P.half_exact && c16;
+  const bool h = r32 && P.hc_pairs && L.vc && P.half_exact && c16;
   const uint32_t *vp = h && L.v16p && P.use_c8 && L.byte_tiles > 0 ? L.v16p : nullptr;
 #define HPCGX_SR(ST, CC)                                                                       \
   k_spmv_resid<ST, CC><<<g, kBlock, 0, s>>>(L.chunks, L.n, C, L.col, L.val, x, b, r, r32,      \
@@ -2055,6 +2063,9 @@ bool launch_residual_fused(Problem &P, const Level &L, const double *b, const do
                                           L.val, x, b, r, r32, P.chunk_partials, L.xcd)
   if (h && L.stream) HPCGX_SRH(true);
   else if (h) HPCGX_SRH(false);
+  else if (L.stream && c16 && L.finest && (P.x_pairs & 1))
+    k_spmv_resid<true, true, true><<<g, kBlock, 0, s>>>(L.chunks, L.n, C, L.col, L.val, x, b, r,
+                                                        r32, P.chunk_partials, L.xcd);
   else if (L.stream && c16) HPCGX_SR(true, true);
   else if (L.stream) HPCGX_SR(true, false);
   else if (c16) HPCGX_SR(false, true);

@@ -1017,16 +1017,17 @@ void cg_mixed(Problem &P, int ordering, const double *b, double *x,
   const Level &A = P.L[0];
   const int64_t n = A.n;
   *niters = 0;
-  launch_copy(x, P.p, n, s);
-  launch_spmv(P, A, P.p, P.Ap, s);
-  launch_residual0(P, n, b, P.Ap, P.r, s);
-  double nr = std::sqrt(read_scalar(P, kNormr2, s));
-  *normr0 = nr;
-  const bool check_each = tol > 0.0;
   // r32 = r rounded to FP32 is kept up to date by the r update itself; z
   // stays FP32 (z32) and is widened inside the dot and the p update, which
   // gives the bits of widening it first.
-  to_f32(n, P.r, P.r32, s);
+  if (!launch_residual_fused(P, A, b, x, P.r, P.r32, s)) {
+    launch_spmv(P, A, x, P.Ap, s);
+    launch_residual0(P, n, b, P.Ap, P.r, s);
+    to_f32(n, P.r, P.r32, s);
+  }
+  double nr = std::sqrt(read_scalar(P, kNormr2, s));
+  *normr0 = nr;
+  const bool check_each = tol > 0.0;
   for (int k = 1; k <= max_iter && nr / *normr0 > tol; ++k) {
     if (k >= 2 && P.use_mixed_graph && !P.klog.on)
       HPCGX_HIP(hipGraphLaunch(mixed_graph(P, ordering, x), s));

@@ -280,12 +280,15 @@ void cg(Problem &P, int ordering, const double *b, double *x, int max_iter,
   PhaseTimer T(P, (flags & HPCGX_CG_TIMERS) != 0, s);
 
   *niters = 0;
-  launch_copy(x, P.p, n, s);                             // :86
   T.tick();
-  launch_spmv(P, A, P.p, P.Ap, s);                          // :87
+  const bool fused = launch_residual_fused(P, A, b, x, P.r, nullptr, s);  // :86-89
+  if (!fused) {
+    launch_copy(x, P.p, n, s);                           // :86
+    launch_spmv(P, A, P.p, P.Ap, s);                        // :87
+  }
   T.tock(3);
   T.tick();
-  launch_residual0(P, n, b, P.Ap, P.r, s);               // :88-89
+  if (!fused) launch_residual0(P, n, b, P.Ap, P.r, s);   // :88-89
   T.tock(2);
   double nr = std::sqrt(read_scalar(P, kNormr2, s));
   *normr0 = nr;

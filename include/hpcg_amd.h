@@ -405,10 +405,11 @@ int hpcgx_cg_fleet(hpcgx_problem *p, int ordering, const double *b, double *x, i
  *                      r updates) use non-temporal loads and stores on
  *                      multivectors of 2^24 or more values (default 1; the
  *                      same bits)
- *   "resid_fused"      1/0: hpcgx_cg_mixed's (and, for s = 4, 8, 16,
- *                      hpcgx_cg_block_mixed's) FP64 residual recompute
- *                      (r = b - A x, its FP32 copy and r.r) in one pass over
- *                      the row chunks, or as SpMV, residual and rounding
+ *   "resid_fused"      1/0: the FP64 residual r = b - A x with r.r, at the
+ *                      start of hpcgx_cg and (with r's FP32 copy) of
+ *                      hpcgx_cg_mixed and in its recompute (and, for s = 4,
+ *                      8, 16, hpcgx_cg_block_mixed's), in one pass over the
+ *                      row chunks, or as copy, SpMV, residual and rounding
  *                      passes (default 1; the same r, r.r summed in another
  *                      order)
  *   "hc_pairs"         1/0: hpcgx_cg_mixed's FP64 A p reads the 8-bit
@@ -449,7 +450,7 @@ int hpcgx_cg_fleet(hpcgx_problem *p, int ordering, const double *b, double *x, i
  *                      (cross-lane permute) instead of a second gather.
  *                      Bit 0: the FP64 colour steps without r.z partials
  *                      (at 256 threads per workgroup with the register
- *                      caps), the chunked SpMV + dot and the fused residual
+ *                      caps), the SpMV and SpMV + dot and the fused residual
  *                      and restriction; bit 1: the FP64 colour step that
  *                      leaves r.z partials; bit 2: the FP32 V-cycle's colour
  *                      steps on FP16 value pairs; bit 3: the FP64 colour
