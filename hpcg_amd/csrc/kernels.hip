@@ -1212,7 +1212,8 @@ __device__ inline double row_dot_hp(const Col16 &C, const uint32_t *__restrict__
                                     const double *__restrict__ diag,
                                     const int32_t *__restrict__ col,
                                     const double *__restrict__ val,
-                                    const double *__restrict__ p, int64_t n, int64_t i) {
+                                    const double *__restrict__ p, int64_t n, int64_t i,
+                                    int64_t end) {
   const int t = C.tile(i);
   const uint32_t flags = C.flags(t);
   if (C.cls(flags) != kTile8) return row_dot_h<STREAM>(C, vc, dslot, diag, col, val, p, n, i);
@@ -1220,6 +1221,45 @@ __device__ inline double row_dot_hp(const Col16 &C, const uint32_t *__restrict__
   const unsigned words = C.words(flags);
   const int place = C.place(i);
   uint32_t o8[kSlotWords], pv[kPairWords];
+  if (words == kAllAffine) {
+    // every load in flight (96 registers, five wavefronts a SIMD), and on a
+    // full tile with shared x windows 18 gathers for 27 (affine_pairs_row).
+    // 256^3: 393 -> 375 us, with the windows 348.  A wavefront's 8-byte gather
+    // costs the L1 16 accesses, and those bound it: other orders of the chunks
+    // that halve the bytes from beyond the L2 leave the time as it is.
+    double xs[kSlots], y = 0.0;
+#pragma unroll
+    for (int w = 0; w < kPairWords; ++w) pv[w] = mload<STREAM>(vp + (int64_t)w * n + i);
+    const int ds = mload<STREAM>(dslot + i);
+    const double di = mload<STREAM>(diag + i);
+    if (pairs_tile(C, flags, i, end)) {
+#pragma unroll
+      for (int m = 0; m < kSlots / 3; ++m) {
+        xs[3 * m] = (p + base[3 * m])[(uint32_t)place];
+        xs[3 * m + 1] = (p + base[3 * m + 1])[(uint32_t)place];
+        xs[3 * m + 2] = p[base[3 * m] + kTile];
+      }
+#pragma unroll
+      for (int m = 0; m < kSlots / 3; ++m) {
+        const double up = __shfl_down(xs[3 * m], 1, 64);
+        xs[3 * m + 2] = place == kTile - 1 ? xs[3 * m + 2] : up;
+      }
+#pragma unroll
+      for (int j = 0; j < kSlots; ++j) {
+        const uint16_t h = (uint16_t)(pv[j / 2] >> (16 * (j % 2)));
+        y += (j == kMidSlot ? di : (double)__builtin_bit_cast(_Float16, h)) * xs[j];
+      }
+      return y;
+    }
+#pragma unroll
+    for (int j = 0; j < kSlots; ++j) xs[j] = (p + base[j])[(uint32_t)place];
+#pragma unroll
+    for (int j = 0; j < kSlots; ++j) {
+      const uint16_t h = (uint16_t)(pv[j / 2] >> (16 * (j % 2)));
+      y += (j == ds ? di : (double)__builtin_bit_cast(_Float16, h)) * xs[j];
+    }
+    return y;
+  }
 #pragma unroll
   for (int g = 0; g < kSlotWords; ++g) o8[g] = off8_word<STREAM>(C.off8, words, g, n, i, place);
 #pragma unroll
@@ -1240,18 +1280,19 @@ __device__ inline double row_dot_hp(const Col16 &C, const uint32_t *__restrict__
 // k_spmv_dot_h with one workgroup per row chunk; partials as k_spmv_dot_c.
 // vp non-null: 8-bit tiles take row_dot_hp.
 template <bool STREAM>
-__global__ __launch_bounds__(kBlock) void k_spmv_dot_hc(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 5)))
+void k_spmv_dot_hc(
     const int64_t *__restrict__ chunks, int64_t n, Col16 C, const uint32_t *__restrict__ vc,
     const uint32_t *__restrict__ vp, const uint8_t *__restrict__ dslot,
     const double *__restrict__ diag, const int32_t *__restrict__ col,
     const double *__restrict__ val, const double *__restrict__ p, double *__restrict__ Ap,
     double *__restrict__ cpart, bool xcd) {
-  const int64_t b = xcd_window(xcd, !STREAM);
+  const int64_t b = xcd_window(xcd, true);
   C.chunk(chunks, b);
-  const int64_t i = chunks[2 * b] + threadIdx.x;
+  const int64_t i = chunks[2 * b] + threadIdx.x, end = chunks[2 * b + 1];
   double s = 0.0;
-  if (i < chunks[2 * b + 1]) {
-    const double y = vp ? row_dot_hp<STREAM>(C, vp, vc, dslot, diag, col, val, p, n, i)
+  if (i < end) {
+    const double y = vp ? row_dot_hp<STREAM>(C, vp, vc, dslot, diag, col, val, p, n, i, end)
                         : row_dot_h<STREAM>(C, vc, dslot, diag, col, val, p, n, i);
     mstore<STREAM>(Ap + i, y);
     s = p[i] * y;
@@ -1493,18 +1534,19 @@ __global__ __launch_bounds__(kBlock) void k_spmv_resid(
 // tiles where vp is non-null): the same products in the same order, so the
 // same r.
 template <bool STREAM>
-__global__ __launch_bounds__(kBlock) void k_spmv_resid_h(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 5)))
+void k_spmv_resid_h(
     const int64_t *__restrict__ chunks, int64_t n, Col16 C, const uint32_t *__restrict__ vc,
     const uint32_t *__restrict__ vp, const uint8_t *__restrict__ dslot,
     const double *__restrict__ diag, const int32_t *__restrict__ col,
     const double *__restrict__ val, const double *__restrict__ x, const double *__restrict__ b,
     double *__restrict__ r, float *__restrict__ r32, double *__restrict__ cpart, bool xcd) {
-  const int64_t blk = xcd_window(xcd, !STREAM);
+  const int64_t blk = xcd_window(xcd, true);
   C.chunk(chunks, blk);
-  const int64_t i = chunks[2 * blk] + threadIdx.x;
+  const int64_t i = chunks[2 * blk] + threadIdx.x, end = chunks[2 * blk + 1];
   double s = 0.0;
-  if (i < chunks[2 * blk + 1]) {
-    const double y = vp ? row_dot_hp<STREAM>(C, vp, vc, dslot, diag, col, val, x, n, i)
+  if (i < end) {
+    const double y = vp ? row_dot_hp<STREAM>(C, vp, vc, dslot, diag, col, val, x, n, i, end)
                         : row_dot_h<STREAM>(C, vc, dslot, diag, col, val, x, n, i);
     const double ri = mload<STREAM>(b + i) + -1.0 * y;
     mstore<STREAM>(r + i, ri);

@@ -121,3 +121,26 @@ def test_turn_same_bits(dims, levels):
         for k, (p, q) in enumerate(zip(*outs)):
             assert torch.equal(p, q), (c16, k)
     P.close()
+
+
+@pytest.mark.parametrize("dims,levels", [((17, 13, 11), 1), ((130, 66, 62), 2), ((258, 30, 14), 2),
+                                         ((128, 64, 64), 3)])
+def test_half_spmv_same_bits(dims, levels):
+    """The mixed solve's A p and residual from FP16 value pairs, on affine tiles
+    with every load in flight (with and without shared x windows) and on others:
+    the bits of the packed words."""
+    import hpcg_amd
+    import torch
+    P = hpcg_amd.Problem.generate(*dims, nlevels=levels)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(13)
+    b, x0 = (torch.rand(P.nrow(0), generator=g, dtype=torch.float64, device="cuda") - 0.5
+             for _ in range(2))
+    outs = []
+    for hp in (1, 0):
+        P.tune("hc_pairs", hp)
+        x = x0.clone()
+        r = P.cg_mixed(b, x, max_iter=5, tolerance=0.0, recompute=2)
+        outs.append((x, r["normr"]))
+    assert torch.equal(outs[0][0], outs[1][0]) and outs[0][1] == outs[1][1]
+    P.close()
