@@ -414,19 +414,22 @@ __global__ __launch_bounds__(kBlock) void k_tile_layout(
       c = col[(int64_t)e * n + i];
       v = val[(int64_t)e * n + i];
     }
-    int lo = wave_min_i32(has ? c : INT_MAX);
-    int hi = wave_max_i32(has ? c : INT_MIN);
-    const bool used = lo != INT_MAX;
+    const uint64_t holders = __ballot(has);
+    const bool used = holders != 0;
     // one base for all entries, with every row's place in range: the slot's
-    // window.  An unused slot's window is the tile itself.
-    const int w0 = used ? wave_min_i32(has ? c - lane : INT_MAX) : first;
-    const int w1 = used ? wave_max_i32(has ? c - lane : INT_MIN) : first;
-    const bool window = w0 == w1 && w0 >= 0 && (int64_t)w0 + kTile <= n;
-    const int32_t cc = has ? c : window ? w0 + lane : used ? lo : (int32_t)i;
-    if (window) {
-      lo = w0;
-      hi = w0 + kTile - 1;
+    // window.  An unused slot's window is the tile itself.  (Ballots: the
+    // wavefront minima and maxima that this needs no longer take a third of
+    // the layout's time.)
+    const int32_t w0 =
+        used ? __shfl(c - lane, used ? __builtin_ctzll(holders) : 0, 64) : first;
+    const bool one = __ballot(has && c - lane != w0) == 0;
+    const bool window = one && w0 >= 0 && (int64_t)w0 + kTile <= n;
+    int lo = w0, hi = w0 + kTile - 1;
+    if (!window && used) {
+      lo = wave_min_i32(has ? c : INT_MAX);
+      hi = wave_max_i32(has ? c : INT_MIN);
     }
+    const int32_t cc = has ? c : window ? w0 + lane : used ? lo : (int32_t)i;
     if (used && hi - lo > 65535) narrow = false;
     if (used && hi - lo > 255) narrow8 = false;
     const int32_t base = used || window ? lo : first;
@@ -437,9 +440,9 @@ __global__ __launch_bounds__(kBlock) void k_tile_layout(
       o8[u / 4] |= ((uint32_t)(cc - base) & 0xffu) << (8 * (u % 4));
       if (has && c == i) ds = u;
     }
-    if (wave_min_i32(!row || cc - base == lane ? 1 : 0) == 1) affine |= 1u << u;
+    if (__ballot(row && cc - base != lane) == 0) affine |= 1u << u;
     if (u % 3 == 0) step2 = step2 && above == base + 1;
-    if (u == kMidSlot) step2 = step2 && wave_min_i32(!row || (has && c == i) ? 1 : 0) == 1;
+    if (u == kMidSlot) step2 = step2 && __ballot(row && !(has && c == i)) == 0;
     above = above1;
     above1 = base;
     if (lane == 0) rec[u] = base;
