@@ -85,10 +85,10 @@ void symgs(Problem &P, int l, int ordering, const double *r, double *x,
     wave_sweep(P, L, 0, r, x, s);
     wave_sweep(P, L, 1, r, x, s);
   } else if (ordering == HPCGX_ORDER_MULTICOLOR) {
-    // the turn: the last colour's two steps in one launch (not where each
-    // colour step is timed by itself)
+    // the turn: the last colour's two steps in one launch (which the launch
+    // log leaves out, as it does the zero-x steps: it times full colour steps)
     const int last = L.ncolors - 1;
-    const bool turn = P.use_turn && last > 0 && !(L.finest && P.klog.on);
+    const bool turn = P.use_turn && last > 0;
     bool turned = false;
     for (int c = 0; c <= last; ++c) {
       if (c == last && turn)

@@ -466,9 +466,8 @@ int hpcgx_cg_fleet(hpcgx_problem *p, int ordering, const double *b, double *x, i
  *                      forward sweep ended with, runs both updates of that
  *                      colour in one launch (FP64), or one of them where the
  *                      second repeats the first (FP32, whose update does not
- *                      read the row's own x); not where the finest level's
- *                      FP64 colour steps are being timed (default 1; the
- *                      same bits)
+ *                      read the row's own x).  hpcgx_kernel_timing does not
+ *                      log that launch (default 1; the same bits)
  *   "block_pairs"      1/0: the block PCG's finest colour steps at s = 8,
  *                      on tiles where "x_pairs" applies, take slot 3m + 2's
  *                      neighbour rows from slot 3m's moved one row (2
@@ -524,9 +523,10 @@ int hpcgx_check_status(hpcgx_problem *p, void *stream);
 
 /* No counterpart in the reference (its timers are host clocks around whole
  * kernels, CG.cpp:36-37): records a HIP event pair on the launch stream
- * around every launch of the finest level's multicolour Gauss-Seidel step,
- * the kernel that dominates the V-cycle.  enable = 1 clears the log and
- * starts recording, 0 stops. */
+ * around every launch of one full colour step of the finest level's
+ * multicolour Gauss-Seidel sweeps, the kernel that dominates the V-cycle (not
+ * the steps from x = 0, nor the launch that holds the two steps of a sweep's
+ * turn).  enable = 1 clears the log and starts recording, 0 stops. */
 int hpcgx_kernel_timing(hpcgx_problem *p, int enable);
 /* Synchronous: summed event time (ms) and number of recorded launches. */
 int hpcgx_kernel_timing_read(hpcgx_problem *p, double *total_ms,
