@@ -1291,6 +1291,8 @@ void mg32_block(Problem &P, int l, int ordering, int s, const float *R, float *X
   Level &L = P.L[l];
   // X = 0 (ComputeMG_ref.cpp:42): a fill, or implied by a first forward
   // sweep that reads only the X it has written
+  if (ordering == HPCGX_ORDER_MULTICOLOR && launch_tail32(P, l, R, X, st, nullptr, nullptr, s))
+    return;
   const bool zg = zero_guess_block(P, l, ordering, s);
   if (!zg) {
     k_bfill32<<<grid_for(L.n * s), kBlock, 0, st>>>(X, L.n * s);

@@ -523,8 +523,9 @@ void launch_symgs_rows(const Problem &P, const Level &L, int64_t begin, int64_t 
 // The multicolour V-cycle from level l down in one launch (tail.hip), rz as
 // symgs; false (nothing launched) where the levels are too large for it.
 bool launch_tail(const Problem &P, int l, const double *r, double *x, hipStream_t s, double *rz);
+// (FP32: of `columns` right-hand sides, [n][columns])
 bool launch_tail32(const Problem &P, int l, const float *r, float *x, hipStream_t s, double *rz,
-                   const double *r64);
+                   const double *r64, int columns = 1);
 // The last colour's forward and backward step in one launch, device rows
 // [begin, end); zero_x as launch_symgs_rows_zero.  False (nothing launched)
 // where the level has no narrow ids.

@@ -456,7 +456,8 @@ int hpcgx_cg_fleet(hpcgx_problem *p, int ordering, const double *b, double *x, i
  *                      steps on FP16 value pairs; bit 3: the FP64 colour
  *                      steps of the coarser levels (default 3; the same bits)
  *   "tail"             1/0: the multicolour V-cycle's levels of at most 6000
- *                      rows run in one launch of one workgroup, with x in
+ *                      rows run in one launch of one workgroup (the block
+ *                      V-cycle: one for each right-hand side), with x in
  *                      LDS (FP64 and FP32; levels of more than 16 colours or
  *                      1024 rows a colour, and the finest level while its
  *                      steps are timed, as launches; default 1; the same

@@ -64,3 +64,24 @@ def test_tail_streams():
     for w, v in zip(want, got):
         assert torch.equal(w, v)
     P.close()
+
+
+@pytest.mark.parametrize("s", [1, 2, 8, 64])
+@pytest.mark.parametrize("dims,levels", [((3, 3, 3), 1), ((16, 16, 16), 4), ((24, 20, 28), 3)])
+def test_tail_block_same_bits(dims, levels, s):
+    """A workgroup per right-hand side: the bits of the block launches."""
+    import hpcg_amd
+    import torch
+    P = hpcg_amd.Problem.generate(*dims, nlevels=levels)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(17)
+    B = torch.rand((P.nrow(0), s), generator=g, dtype=torch.float64, device="cuda") - 0.5
+    outs = []
+    for tail in (1, 0):
+        P.tune("tail", tail)
+        Z, X = torch.full_like(B.float(), float("nan")), torch.zeros_like(B)
+        P.mg32_block(B.float(), Z, ordering="multicolor")
+        P.cg_block_mixed(B, X, max_iter=3, recompute=2)
+        outs.append((Z, X))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    P.close()
