@@ -821,7 +821,8 @@ void symgs32(Problem &P, int l, int ordering, const float *r, float *x,
   if (ordering == HPCGX_ORDER_MULTICOLOR) {
     // The turn: a row's update reads no entry of its own colour (the FP16
     // diagonal slots hold 0), so the backward sweep's first colour step would
-    // write the values that the forward sweep's last one has just written.
+    // write the values that the forward sweep's last one has just written (an
+    // overflowed x, infinite, would become NaN one step earlier).
     // It is left out, and the forward step leaves its r.z partials.  One of
     // 16 full steps: an FP32 V-cycle of one level
     // at 256^3 528 -> 490 us.
