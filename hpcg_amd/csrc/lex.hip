@@ -55,6 +55,12 @@ constexpr int kLexStore = kSlots + 1;      // values stored per row
 constexpr int kLexEdge = 64;               // rows of 0 before and after the copy of x
 constexpr int kLexRing = 2048;             // fresh x values held in LDS
 constexpr int kLexReach = kLexRing - 64 * kLexWaves - 64;  // furthest fresh row
+// The wait that a sweep's progress rests on (k_lex_sweep): vector memory
+// operations that may still be outstanding when a step ends.
+constexpr int kLexLoads = kLexStore / 2 + 2 + (kSlots - kLexIn - 1) + 1;  // of one step
+constexpr int kLexPinned = (kSlots - kLexIn - 1) + 2;  // those of x and of the neighbour's progress
+constexpr int kLexWait = kLexLoads + 3;  // and a step's store, the progress, the last store
+static_assert(kLexWait <= 2 * kLexPinned && kLexWait < 63, "covers the stores of two steps before");
 
 inline unsigned grid_for(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 __device__ inline int64_t gtid() { return (int64_t)blockIdx.x * blockDim.x + threadIdx.x; }
@@ -301,11 +307,16 @@ __global__ __launch_bounds__(kBlock) void k_lex_out(int64_t n, const int32_t *__
 // for the neighbour panel; x of the own panel's fresh rows from a ring in LDS.
 //
 // Progress: counter p holds the steps of panel p whose x stores have
-// completed.  Vector memory operations of a wavefront complete in order.  Its
-// stores of step k are followed by the gathers for step k + 2, so once step
-// k + 2 has used those, the stores have been acknowledged; after the barrier
-// that ends step k + 2 this holds for every wavefront and step k is
-// published: no wait for a store stands in the chain of steps.
+// completed.  Vector memory operations of a wavefront complete in order, and
+// every wavefront ends every step, with rows in it or without, with a wait that
+// leaves the last kLexWait of them outstanding.  Between a store of step k and
+// the end of step k + 2 lie the loads that steps k + 1 and k + 2 issue
+// unconditionally; the compiler moves none of those of x or of the neighbour's
+// progress (kLexPinned a step) over the waits, which clobber memory.  They are
+// more than kLexWait, so after the barrier that ends step k + 2 the stores of
+// step k have been acknowledged for every wavefront, and step k is published.
+// The wait costs the chain of steps nothing: what it waits for besides, the
+// loads that step k + 1 issued, step k + 2 has used.
 template <bool STREAM, int DIR>
 __global__ __launch_bounds__(64 * kLexWaves) void k_lex_sweep(
     int npanels, int waves, const LexRec *__restrict__ recs, const int32_t *__restrict__ sptr,
@@ -461,6 +472,7 @@ __global__ __launch_bounds__(64 * kLexWaves) void k_lex_sweep(
       gather(G[(a + 1) & 1], S[1], k + a + 1);
       const Span next = span(k + a + kLexAhead + 2);
       step(M[a % (kLexAhead + 1)], G[a & 1], S[0]);
+      asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kLexWait) : "memory");
       __syncthreads();
       if (threadIdx.x == 0 && k + a >= 2)
         __hip_atomic_store(mine, (unsigned)(k + a - 1), __ATOMIC_RELAXED,
@@ -470,7 +482,7 @@ __global__ __launch_bounds__(64 * kLexWaves) void k_lex_sweep(
       S[kLexAhead + 1] = next;
     }
   }
-  __builtin_amdgcn_s_waitcnt(0);  // this wavefront's x stores are complete
+  asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // this wavefront's x stores are complete
   __syncthreads();
   if (threadIdx.x == 0)
     __hip_atomic_store(mine, (unsigned)nsteps, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
