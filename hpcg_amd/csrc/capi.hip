@@ -436,6 +436,12 @@ int hpcgx_tune(hpcgx_problem *p, const char *key, double value) {
       P.use_lex = value != 0.0;
       return;
     }
+    if (k == "lex_polls") {
+      if (value < 0 || value > (1 << 22) || value != (int)value)
+        throw Error(HPCGX_EINVAL, "lex_polls must be an integer in [0, 2^22]");
+      P.lex_polls = (unsigned)value;
+      return;
+    }
     if (k == "hc_pairs") {
       P.hc_pairs = value != 0.0;
       return;

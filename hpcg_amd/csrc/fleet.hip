@@ -501,6 +501,7 @@ void cg_fleet(Problem &P, int ordering, const double *b, double *x, int max_iter
   if (times)
     times[0] += std::chrono::duration<double>(std::chrono::steady_clock::now() - t_begin)
                     .count();
+  check_status(P);
   if (!finite) throw Error(HPCGX_EINVAL, "CG residual is not finite");
 }
 

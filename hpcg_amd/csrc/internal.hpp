@@ -266,7 +266,7 @@ struct Problem {
   double *partials = nullptr;
   unsigned *ticket = nullptr;
   double *scalars = nullptr;  // see CgScalar
-  int *wave_err = nullptr;    // set when a wavefront wait gives up
+  int *wave_err = nullptr;    // set when a wait of a wavefront or panel sweep gives up
   int wave_grid = 0;          // co-resident workgroups of the wavefront kernel
   bool use_wave = false;      // multicolour sweeps as wavefronts (measured slower)
   bool use_c16 = true;        // read narrow column ids where a level has them
@@ -299,6 +299,7 @@ struct Problem {
   bool block_nt = true;
   // reference-order FP64 sweeps by panels of rows (lex.hip; "lex_panels")
   bool use_lex = true;
+  unsigned lex_polls = 1u << 22;  // polls before a wait gives up (seconds; "lex_polls")
   // block PCG finest colour steps: slot 3m + 2's x rows from slot 3m's by
   // W-lane moves on affine tiles ("block_pairs")
   bool block_pairs = false;

@@ -46,7 +46,6 @@ namespace {
 
 constexpr int kLexWaves = 4;               // wavefronts per workgroup, at most
 constexpr int kLexPad = 32;                // progress counters 128 bytes apart
-constexpr unsigned kLexSpins = 1u << 22;   // polls before a wait gives up (seconds)
 constexpr int64_t kLexRows = 256;          // see build_lex
 constexpr int kLexAhead = 1;               // steps the matrix loads run ahead
 constexpr int kLexIn = 4, kLexOut = 9;     // slots of the own and of a neighbour panel
@@ -297,8 +296,8 @@ __global__ __launch_bounds__(kBlock) void k_lex_out(int64_t n, const int32_t *__
 
 // One sweep direction.  Workgroup order comes from a ticket, so a workgroup
 // only ever waits for panels whose workgroups have already started; a wait
-// that exceeds kLexSpins polls sets *err and gives up, as all later ones do,
-// and the sweep ends with wrong values instead of hanging.
+// that exceeds `polls` polls sets *err and gives up, as all later ones do,
+// and the sweep ends with wrong values instead of hanging (check_status).
 //
 // A step's loads run ahead of it, so that between two barriers only the chain
 // through the rows just finished remains: values, right-hand side, diagonal
@@ -322,7 +321,7 @@ __global__ __launch_bounds__(64 * kLexWaves) void k_lex_sweep(
     int npanels, int waves, const LexRec *__restrict__ recs, const int32_t *__restrict__ sptr,
     const int64_t *__restrict__ pstart, const double *__restrict__ lval,
     const int32_t *__restrict__ lcol, const double *__restrict__ r, double *x, unsigned *prog,
-    int *err) {
+    unsigned polls, int *err) {
   __shared__ double ring[kLexRing];
   __shared__ int s_ticket;
   // rows without an entry in a fresh slot read the ring too (times 0)
@@ -388,7 +387,7 @@ __global__ __launch_bounds__(64 * kLexWaves) void k_lex_sweep(
       unsigned spins = 0;
       while (seen < need) {
         seen = __builtin_amdgcn_readfirstlane(pload(nbr));
-        if (++spins > kLexSpins ||
+        if (++spins > polls ||
             ((spins & 1023u) == 0u &&
              __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
           if (lane == 0) atomicOr(err, 1);
@@ -683,7 +682,7 @@ bool launch_symgs_lex(Problem &P, int l, const double *r, double *x, hipStream_t
   const dim3 g(X.npanels), b(64 * X.waves);
 #define HPCGX_LEX(ST, DIR)                                                                       \
   k_lex_sweep<ST, DIR><<<g, b, 0, s>>>(X.npanels, X.waves, X.recs, X.sptr, X.pstart, X.val,      \
-                                       X.col, X.r, X.x, X.prog + DIR * X.nprog, P.wave_err)
+                                       X.col, X.r, X.x, X.prog + DIR * X.nprog, P.lex_polls, P.wave_err)
   if (L.stream) {
     HPCGX_LEX(true, 0);
     HPCGX_LEX(true, 1);

@@ -206,7 +206,7 @@ void check_status(Problem &P) {
   HPCGX_HIP(hipMemcpy(&e, P.wave_err, sizeof e, hipMemcpyDeviceToHost));
   if (e) {
     HPCGX_HIP(hipMemset(P.wave_err, 0, sizeof(int)));
-    throw Error(HPCGX_EHIP, "wavefront sweep: a dependency wait timed out");
+    throw Error(HPCGX_EHIP, "Gauss-Seidel sweep: a dependency wait timed out");
   }
 }
 

@@ -15,6 +15,9 @@ int DeviceMG(const SparseMatrix &A, const Vector &r, Vector &x, int ordering) {
   int rc = Upload(*L, r, dr);
   if (rc) return rc;
   rc = hpcgx_mg(L->ctx->problem, L->level, ordering, dr, dx, nullptr);
+  // a reference-order sweep may have given up a wait (hpcgx_check_status)
+  if (!rc && ordering == HPCGX_ORDER_LEXICOGRAPHIC)
+    rc = hpcgx_check_status(L->ctx->problem, nullptr);
   if (rc) return Report("ComputeMG", rc);
   return Download(*L, dx, x);
 }

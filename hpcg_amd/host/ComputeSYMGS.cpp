@@ -16,6 +16,9 @@ int DeviceSYMGS(const SparseMatrix &A, const Vector &r, Vector &x, int ordering)
   if (!rc) rc = Upload(*L, x, dx);
   if (rc) return rc;
   rc = hpcgx_symgs(L->ctx->problem, L->level, ordering, dr, dx, nullptr);
+  // a reference-order sweep may have given up a wait (hpcgx_check_status)
+  if (!rc && ordering == HPCGX_ORDER_LEXICOGRAPHIC)
+    rc = hpcgx_check_status(L->ctx->problem, nullptr);
   if (rc) return Report("ComputeSYMGS", rc);
   return Download(*L, dx, x);
 }

@@ -256,13 +256,14 @@ class Problem:
         return call("hpcgx_spmv", self._h, level, _ptr(x, n, "x"), _ptr(y, n, "y"), _stream())
 
     def symgs(self, r, x, level=0, ordering="lexicographic"):
-        """ComputeSYMGS (ComputeSYMGS.cpp:50): one symmetric sweep on x."""
+        """ComputeSYMGS (ComputeSYMGS.cpp:50): one symmetric sweep on x.
+        check() tells whether a lexicographic sweep completed."""
         n = self.nrow(level)
         return call("hpcgx_symgs", self._h, level, _order(ordering), _ptr(r, n, "r"),
                     _ptr(x, n, "x"), _stream())
 
     def mg(self, r, x, level=0, ordering="lexicographic"):
-        """ComputeMG (ComputeMG.cpp:33): x = V-cycle(r)."""
+        """ComputeMG (ComputeMG.cpp:33): x = V-cycle(r); check() as for symgs."""
         n = self.nrow(level)
         return call("hpcgx_mg", self._h, level, _order(ordering), _ptr(r, n, "r"),
                     _ptr(x, n, "x"), _stream())
@@ -399,7 +400,8 @@ class Problem:
         return buf.value.decode().splitlines()
 
     def check(self):
-        """Wait for the stream; raise if a wavefront sweep gave up waiting."""
+        """Wait for the stream; raise if a lexicographic or wavefront sweep gave
+        up waiting (its x is then wrong)."""
         return call("hpcgx_check_status", self._h, _stream())
 
     def kernel_timing(self, enable=True):

@@ -186,13 +186,16 @@ int hpcgx_spmv(const hpcgx_problem *p, int level, const double *x, double *y,
 
 /* replaces ComputeSYMGS (ComputeSYMGS.cpp:50-55 -> ComputeSYMGS_ref.cpp:
  * 54-103): one forward and one backward Gauss-Seidel sweep on x with right
- * hand side r, in the given ordering (HPCGX_ORDER_*). */
+ * hand side r, in the given ordering (HPCGX_ORDER_*).  The workgroups of a
+ * lexicographic sweep wait for each other; a wait that lasts for seconds
+ * gives up and leaves a wrong x, which hpcgx_check_status reports. */
 int hpcgx_symgs(const hpcgx_problem *p, int level, int ordering,
                 const double *r, double *x, void *stream);
 
 /* replaces ComputeMG (ComputeMG.cpp:33-38 -> ComputeMG_ref.cpp:39-63): the
  * V-cycle from `level` down, x := M^-1 r (x is zeroed first). Uses the
- * problem's own coarse-level vectors. */
+ * problem's own coarse-level vectors.  hpcgx_check_status as for
+ * hpcgx_symgs. */
 int hpcgx_mg(hpcgx_problem *p, int level, int ordering, const double *r,
              double *x, void *stream);
 
@@ -401,6 +404,9 @@ int hpcgx_cg_fleet(hpcgx_problem *p, int ordering, const double *b, double *x, i
  *                      where at most half of the free memory holds it), or
  *                      one launch per hyperplane of the schedule
  *                      (default 1; the same bits)
+ *   "lex_polls"        polls after which a wait of such a sweep gives up
+ *                      (0..2^22, default 2^22: seconds; see
+ *                      hpcgx_check_status)
  *   "block_nt"         1/0: the block PCG's vector kernels (r.z, the p and
  *                      r updates) use non-temporal loads and stores on
  *                      multivectors of 2^24 or more values (default 1; the
@@ -516,8 +522,11 @@ int hpcgx_autotune(hpcgx_problem *p, int ordering, int iterations, char *report,
                    int report_len);
 
 /* No counterpart in the reference: waits for `stream` and reports a
- * wavefront sweep whose dependency wait gave up (HPCGX_EHIP).  hpcgx_cg
- * performs the same check before returning. */
+ * lexicographic ("lex_panels") or wavefront ("wave") sweep of this problem
+ * whose dependency wait gave up since the last check (HPCGX_EHIP): the x of
+ * that sweep and of those after it is wrong.  The report clears the state.
+ * hpcgx_cg and hpcgx_cg_fleet perform the same check before returning;
+ * hpcgx_symgs and hpcgx_mg are asynchronous and cannot. */
 int hpcgx_check_status(hpcgx_problem *p, void *stream);
 
 /* ---- measurement ----------------------------------------------------------- */
