@@ -153,8 +153,8 @@ __global__ __launch_bounds__(kBlock) void k_lex_fill(
     const int64_t *__restrict__ pstart, int npanels, const int32_t *__restrict__ row,
     const int32_t *__restrict__ pos, const int32_t *__restrict__ iperm,
     const int32_t *__restrict__ col, const double *__restrict__ val,
-    const double *__restrict__ diag, const uint8_t *__restrict__ nnz_row,
-    double *__restrict__ lval, int32_t *__restrict__ lcol, int32_t *__restrict__ ldpos,
+    const double *__restrict__ diag, const uint8_t *__restrict__ dslot,
+    const uint8_t *__restrict__ nnz_row, double *__restrict__ lval, int32_t *__restrict__ lcol, int32_t *__restrict__ ldpos,
     int *bad) {
   const int64_t q = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
   if (q >= nrec) return;  // whole wavefronts
@@ -233,12 +233,12 @@ __global__ __launch_bounds__(kBlock) void k_lex_fill(
     }
   }
   if (!fits && live) {
+    ds = dslot[i];  // (not by its value, which may be 0 until it is replaced)
     for (int u = 0; u < kSlots; ++u) {
       const double v = val[(int64_t)u * n + i];
       int32_t c = pos[col[(int64_t)u * n + i]];
       // an unused slot's column need not be near: the row's own x there
       if (v == 0.0 && (c < lo || c >= hi)) c = k;
-      if (c == k && v != 0.0) ds = u;
       lval[lex_at(start, cnt, u, lane)] = v;
       lcol[at0 + (int64_t)u * cnt] = c;
     }
@@ -589,7 +589,7 @@ bool try_lex(Problem &P, Level &L, LexPlan &X, const std::vector<int64_t> &bound
   const int64_t wpb = kBlock / 64;
   k_lex_fill<<<(unsigned)((X.nrec + wpb - 1) / wpb), kBlock, 0, s>>>(
       X.nrec, n, X.recs, pof.as<int32_t>(), X.pstart, X.npanels, X.row, X.pos, L.iperm, L.col,
-      L.val, L.diag, L.nnz_row, X.val, X.col, X.dpos, bad.as<int>());
+      L.val, L.diag, L.dslot, L.nnz_row, X.val, X.col, X.dpos, bad.as<int>());
   HPCGX_LAUNCHED();
   int far = 0;
   HPCGX_HIP(hipMemcpyAsync(&far, bad.p, sizeof far, hipMemcpyDeviceToHost, s));
