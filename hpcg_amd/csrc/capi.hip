@@ -283,7 +283,6 @@ int hpcgx_replace_diagonal(hpcgx_problem *p, int level, const double *diag, void
     hpcgx::Level &L = level_of(p, level);
     hpcgx::launch_replace_diag(L, diag, S(stream));
     hpcgx::replace_diag32(L, diag, S(stream));
-    hpcgx::lex_replace_diag(L, diag, S(stream));
   });
 }
 

@@ -138,6 +138,7 @@ struct LexPlan {
   double *val = nullptr;      // [28 n] chunk by chunk, two slots side by side; then the diagonal
   int32_t *col = nullptr;     // [27 n] positions
   int32_t *dpos = nullptr;    // [n] slot of the diagonal
+  unsigned *taken = nullptr;  // the Level::diag_gen whose diagonal the copy holds
   double *x = nullptr, *r = nullptr;  // [n] x and r in this order
   unsigned *prog = nullptr;   // ticket and progress counters, forward then backward
   hipEvent_t done = nullptr;  // the last sweep's end (its scratch is free again)
@@ -162,6 +163,7 @@ struct Level {
   int32_t *col = nullptr;   // [kSlots * n] device-order column ids
   double *val = nullptr;    // [kSlots * n]
   double *diag = nullptr;   // [n]
+  unsigned *diag_gen = nullptr;  // replacements of the diagonal so far, counted on the device
   uint8_t *dslot = nullptr; // [n] slot of the diagonal entry
   uint8_t *nnz_row = nullptr; // [n] stored entries per row
   int32_t *perm = nullptr;  // natural row -> device row
@@ -533,7 +535,6 @@ bool launch_tail32(const Problem &P, int l, const float *r, float *x, hipStream_
 bool launch_symgs_turn(const Problem &P, const Level &L, int64_t begin, int64_t end,
                        const double *r, double *x, hipStream_t s, double *dpart, bool zero_x);
 bool launch_symgs_lex(Problem &P, int l, const double *r, double *x, hipStream_t s);
-void lex_replace_diag(Level &L, const double *d, hipStream_t s);
 void launch_symgs_list(const Level &L, const int32_t *rows, int64_t count,
                        const double *r, double *x, hipStream_t s);
 // The colour step of a forward sweep whose x was zero when the sweep began

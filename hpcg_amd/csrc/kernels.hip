@@ -980,8 +980,9 @@ __global__ __launch_bounds__(kBlock) void k_prolong(
 
 __global__ __launch_bounds__(kBlock) void k_replace_diag(
     int64_t n, const uint8_t *__restrict__ dslot, const double *__restrict__ d,
-    double *__restrict__ diag, double *__restrict__ val) {
+    double *__restrict__ diag, double *__restrict__ val, unsigned *gen) {
   const int64_t i = gtid();
+  if (i == 0) ++*gen;
   if (i < n) {
     const double v = d[i];
     diag[i] = v;
@@ -2206,7 +2207,7 @@ void launch_symgs_wave(Problem &P, const Level &L, int dir, const double *r,
 
 void launch_replace_diag(Level &L, const double *d, hipStream_t s) {
   k_replace_diag<<<grid_for(L.n), kBlock, 0, s>>>(L.n, L.dslot, d, L.diag,
-                                                  L.val);
+                                                  L.val, L.diag_gen);
   HPCGX_LAUNCHED();
 }
 

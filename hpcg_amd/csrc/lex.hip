@@ -250,36 +250,35 @@ __global__ __launch_bounds__(kBlock) void k_lex_fill(
   if (lane == 0) recs[q].general = fits ? 0u : 1u;
 }
 
-// A new diagonal (device order) into the copy: slot ldpos of each row and the
-// diagonal's own.
-__global__ __launch_bounds__(kBlock) void k_lex_diag(int64_t nrec,
-                                                     const LexRec *__restrict__ recs,
-                                                     const int32_t *__restrict__ row,
-                                                     const int32_t *__restrict__ ldpos,
-                                                     const double *__restrict__ d, double *lval) {
-  const int64_t q = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-  if (q >= nrec) return;
-  const int lane = threadIdx.x & 63, cnt = recs[q].cnt;
-  if (lane >= cnt) return;
-  const int32_t start = recs[q].start, k = start + lane;
-  const double v = d[row[k]];
-  lval[lex_at(start, cnt, ldpos[k], lane)] = v;
-  lval[lex_at(start, cnt, kSlots, lane)] = v;
-}
-
 __global__ __launch_bounds__(kBlock) void k_lex_zero(int64_t n, double *x) {
   const int64_t i = gtid();
   if (i < n) x[i] = 0.0;
 }
 
-// x and r into the sweep's order; clears both sweeps' progress counters.
-__global__ __launch_bounds__(kBlock) void k_lex_in(int64_t n, const int32_t *__restrict__ row,
-                                                   const double *__restrict__ r,
-                                                   const double *__restrict__ x,
-                                                   double *__restrict__ lr,
-                                                   double *__restrict__ lx, unsigned *prog,
-                                                   int64_t nprog) {
+// x and r into the sweep's order; clears both sweeps' progress counters.  Where
+// the level's diagonal has been replaced since the copy took its own (*taken is
+// behind *gen, both counted on the device, so that a replacement replayed from
+// a graph counts too), it goes into the copy first: slot ldpos of each row and
+// the diagonal's own.
+__global__ __launch_bounds__(kBlock) void k_lex_in(
+    int64_t n, const int32_t *__restrict__ row, const double *__restrict__ r,
+    const double *__restrict__ x, double *__restrict__ lr, double *__restrict__ lx,
+    unsigned *prog, int64_t nprog, const unsigned *gen, const unsigned *taken, int64_t nrec,
+    const LexRec *__restrict__ recs, const int32_t *__restrict__ ldpos,
+    const double *__restrict__ diag, double *__restrict__ lval) {
   const int64_t k = gtid();
+  if (*gen != *taken) {
+    const int lane = threadIdx.x & 63;
+    const int64_t waves = (int64_t)gridDim.x * (kBlock / 64);
+    for (int64_t q = k / 64; q < nrec; q += waves) {
+      const int cnt = recs[q].cnt;
+      const int32_t start = recs[q].start;
+      if (lane >= cnt) continue;
+      const double v = diag[row[start + lane]];
+      lval[lex_at(start, cnt, ldpos[start + lane], lane)] = v;
+      lval[lex_at(start, cnt, kSlots, lane)] = v;
+    }
+  }
   if (k < nprog) prog[k] = 0u;
   if (k >= n) return;
   const int32_t i = row[k];
@@ -289,8 +288,10 @@ __global__ __launch_bounds__(kBlock) void k_lex_in(int64_t n, const int32_t *__r
 
 __global__ __launch_bounds__(kBlock) void k_lex_out(int64_t n, const int32_t *__restrict__ pos,
                                                     const double *__restrict__ lx,
-                                                    double *__restrict__ x) {
+                                                    double *__restrict__ x, const unsigned *gen,
+                                                    unsigned *taken) {
   const int64_t i = gtid();
+  if (i == 0) *taken = *gen;
   if (i < n) x[i] = lx[pos[i]];
 }
 
@@ -582,6 +583,8 @@ bool try_lex(Problem &P, Level &L, LexPlan &X, const std::vector<int64_t> &bound
                            hipMemcpyHostToDevice, s));
   HPCGX_HIP(hipMemcpyAsync(X.pstart, pstart.data(), sizeof(int64_t) * pstart.size(),
                            hipMemcpyHostToDevice, s));
+  X.taken = X.mem.alloc<unsigned>(1);
+  HPCGX_HIP(hipMemcpyAsync(X.taken, L.diag_gen, sizeof(unsigned), hipMemcpyDeviceToDevice, s));
   Buf pof(sizeof(int32_t) * panel_of.size()), bad(sizeof(int));
   HPCGX_HIP(hipMemcpyAsync(pof.p, panel_of.data(), sizeof(int32_t) * panel_of.size(),
                            hipMemcpyHostToDevice, s));
@@ -677,7 +680,9 @@ bool launch_symgs_lex(Problem &P, int l, const double *r, double *x, hipStream_t
   }
   const int64_t n = L.n;
   k_lex_in<<<grid_for(std::max(n, 2 * X.nprog)), kBlock, 0, s>>>(n, X.row, r, x, X.r, X.x, X.prog,
-                                                                 2 * X.nprog);
+                                                                 2 * X.nprog, L.diag_gen, X.taken,
+                                                                 X.nrec, X.recs, X.dpos, L.diag,
+                                                                 X.val);
   HPCGX_LAUNCHED();
   const dim3 g(X.npanels), b(64 * X.waves);
 #define HPCGX_LEX(ST, DIR)                                                                       \
@@ -692,19 +697,10 @@ bool launch_symgs_lex(Problem &P, int l, const double *r, double *x, hipStream_t
   }
 #undef HPCGX_LEX
   HPCGX_LAUNCHED();
-  k_lex_out<<<grid_for(n), kBlock, 0, s>>>(n, X.pos, X.x, x);
+  k_lex_out<<<grid_for(n), kBlock, 0, s>>>(n, X.pos, X.x, x, L.diag_gen, X.taken);
   HPCGX_LAUNCHED();
   if (!own) HPCGX_HIP(hipEventRecord(X.done, s));
   return true;
-}
-
-void lex_replace_diag(Level &L, const double *d, hipStream_t s) {
-  LexPlan &X = L.lex;
-  if (!X.ready) return;
-  const int64_t wpb = kBlock / 64;
-  k_lex_diag<<<(unsigned)((X.nrec + wpb - 1) / wpb), kBlock, 0, s>>>(X.nrec, X.recs, X.row, X.dpos,
-                                                                     d, X.val);
-  HPCGX_LAUNCHED();
 }
 
 }  // namespace hpcgx

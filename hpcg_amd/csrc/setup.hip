@@ -897,6 +897,8 @@ void finalize_level(Problem &P, int l, NaturalLevel &N, int flags,
   L.col = P.arena.alloc<int32_t>((size_t)kSlots * n);
   L.val = P.arena.alloc<double>((size_t)kSlots * n);
   L.diag = P.arena.alloc<double>(n);
+  L.diag_gen = P.arena.alloc<unsigned>(1);
+  HPCGX_HIP(hipMemsetAsync(L.diag_gen, 0, sizeof(unsigned), s));
   L.dslot = P.arena.alloc<uint8_t>(n);
   L.nnz_row = P.arena.alloc<uint8_t>(n);
   k_permute_ell<<<grid_for(n), kBlock, 0, s>>>(n, L.iperm, L.perm, N.col, N.val,

@@ -39,3 +39,43 @@ def test_diagonal_zero_when_copied(dims, every):
     a, b = sweeps(P)
     assert a.isfinite().all() and torch.equal(a, b)
     P.close()
+
+
+def test_captured_replacements():
+    """A replacement captured before the copy exists, and one captured after,
+    each replayed with new values between sweeps; and one by the CG's own graph."""
+    import hpcg_amd
+    import torch
+    P = hpcg_amd.Problem.generate(24, 40, 16, nlevels=2)
+    d = [P.copy_diagonal(l) for l in range(2)]
+    new = [v.clone() for v in d]
+    graphs = []
+    for when in range(2):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for l in range(2):
+                P.replace_diagonal(new[l], l)
+        graphs.append(graph)
+        for k in range(3):
+            for graph in graphs:
+                for l in range(2):
+                    new[l].copy_(d[l] * (1.0 + 0.1 * (3 * when + k + 1)))
+                graph.replay()
+                for l in range(2):
+                    a, b = sweeps(P, l, seed=k)
+                    assert a.isfinite().all() and torch.equal(a, b), (when, k, l)
+    outs = []
+    r = torch.ones(P.nrow(0), dtype=torch.float64, device="cuda")
+    for panels in (1, 0):
+        P.tune("lex_panels", panels)
+        for l in range(2):
+            P.replace_diagonal(d[l], l)
+        x = [torch.zeros_like(r) for _ in range(2)]
+        P.cg(r, x[0], max_iter=3, ordering="lexicographic", graph=True)
+        for l in range(2):
+            P.replace_diagonal(d[l] * 1.5, l)
+        P.cg(r, x[1], max_iter=3, ordering="lexicographic", graph=True)
+        outs.append(x)
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    assert not torch.equal(outs[0][0], outs[0][1])
+    P.close()
