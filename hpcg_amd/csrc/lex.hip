@@ -83,13 +83,18 @@ __device__ inline unsigned pload(const unsigned *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// key[natural row] = panel * nsched + hyperplane; panel p holds the natural
-// rows [bound[p], bound[p + 1])
+// Panel p holds the natural rows [bound[p], bound[p + 1]).  FIND: the first and
+// last hyperplane of each panel, span[2 p] and span[2 p + 1].  Else
+// key[natural row] = first[panel] + hyperplane: the panel's own hyperplanes
+// only, as a panel meets few of a long grid's.
+template <bool FIND>
 __global__ __launch_bounds__(kBlock) void k_lex_key(int64_t n, int nsched, int npanels,
                                                     const int64_t *__restrict__ bound,
                                                     const int64_t *__restrict__ level_ptr,
                                                     const int32_t *__restrict__ level_rows,
                                                     const int32_t *__restrict__ iperm,
+                                                    int32_t *span,
+                                                    const int32_t *__restrict__ first,
                                                     int32_t *__restrict__ key) {
   const int64_t k = gtid();
   if (k >= n) return;
@@ -104,7 +109,12 @@ __global__ __launch_bounds__(kBlock) void k_lex_key(int64_t n, int nsched, int n
     const int mid = (a + b + 1) / 2;
     if (bound[mid] <= g) a = mid; else b = mid - 1;
   }
-  key[g] = a * nsched + lo;
+  if (FIND) {
+    if (span[2 * a] > lo) atomicMin(&span[2 * a], lo);
+    if (span[2 * a + 1] < lo) atomicMax(&span[2 * a + 1], lo);
+  } else {
+    key[g] = first[a] + lo;
+  }
 }
 
 // row[k] = device row of position k, pos[device row] = k
@@ -501,22 +511,48 @@ bool try_lex(Problem &P, Level &L, LexPlan &X, const std::vector<int64_t> &bound
              hipStream_t s) {
   const int64_t n = L.n;
   const int64_t np = (int64_t)bound.size() - 1;
-  if (np * L.nsched >= (int64_t)1 << 30) return false;
-  std::vector<int64_t> kp;  // positions of (panel, hyperplane) keys
+  std::vector<int32_t> span(2 * np);   // first and last hyperplane of a panel
+  std::vector<int32_t> first(np + 1);  // key of hyperplane 0 of a panel; last: all keys
+  std::vector<int64_t> kp;             // positions of (panel, hyperplane) keys
   X.row = X.mem.alloc<int32_t>(n);
   X.pos = X.mem.alloc<int32_t>(n);
   {
     Buf key(sizeof(int32_t) * n), order(sizeof(int32_t) * n),
-        lptr(sizeof(int64_t) * (L.nsched + 1)), bnd(sizeof(int64_t) * bound.size());
+        lptr(sizeof(int64_t) * (L.nsched + 1)), bnd(sizeof(int64_t) * bound.size()),
+        spn(sizeof(int32_t) * span.size()), fst(sizeof(int32_t) * first.size());
+    for (int64_t p = 0; p < np; ++p) {
+      span[2 * p] = L.nsched;
+      span[2 * p + 1] = -1;
+    }
+    HPCGX_HIP(hipMemcpyAsync(spn.p, span.data(), sizeof(int32_t) * span.size(),
+                             hipMemcpyHostToDevice, s));
     HPCGX_HIP(hipMemcpyAsync(bnd.p, bound.data(), sizeof(int64_t) * bound.size(),
                              hipMemcpyHostToDevice, s));
     HPCGX_HIP(hipMemcpyAsync(lptr.p, L.level_ptr.data(), sizeof(int64_t) * (L.nsched + 1),
                              hipMemcpyHostToDevice, s));
-    k_lex_key<<<grid_for(n), kBlock, 0, s>>>(n, L.nsched, (int)np, bnd.as<int64_t>(),
-                                             lptr.as<int64_t>(), L.level_rows, L.iperm,
-                                             key.as<int32_t>());
-    HPCGX_LAUNCHED();
-    kp = sort_rows_by_key(n, key.as<int32_t>(), (int)(np * L.nsched), order.as<int32_t>(), s);
+    auto keys = [&](auto kernel) {
+      kernel<<<grid_for(n), kBlock, 0, s>>>(n, L.nsched, (int)np, bnd.as<int64_t>(),
+                                            lptr.as<int64_t>(), L.level_rows, L.iperm,
+                                            spn.as<int32_t>(), fst.as<int32_t>(),
+                                            key.as<int32_t>());
+      HPCGX_LAUNCHED();
+    };
+    keys(k_lex_key<true>);
+    HPCGX_HIP(hipMemcpyAsync(span.data(), spn.p, sizeof(int32_t) * span.size(),
+                             hipMemcpyDeviceToHost, s));
+    HPCGX_HIP(hipStreamSynchronize(s));
+    // a grid's planes meet at most 2 n hyperplanes together
+    int64_t nkeys = 0;
+    for (int64_t p = 0; p < np; ++p) {
+      first[p] = (int32_t)(nkeys - span[2 * p]);
+      nkeys += span[2 * p + 1] - span[2 * p] + 1;
+      if (nkeys > 4 * n) return false;
+    }
+    first[np] = (int32_t)nkeys;
+    HPCGX_HIP(hipMemcpyAsync(fst.p, first.data(), sizeof(int32_t) * first.size(),
+                             hipMemcpyHostToDevice, s));
+    keys(k_lex_key<false>);
+    kp = sort_rows_by_key(n, key.as<int32_t>(), (int)nkeys, order.as<int32_t>(), s);
     k_lex_rows<<<grid_for(n), kBlock, 0, s>>>(n, order.as<int32_t>(), L.perm, X.row, X.pos);
     HPCGX_LAUNCHED();
     HPCGX_HIP(hipStreamSynchronize(s));
@@ -529,10 +565,10 @@ bool try_lex(Problem &P, Level &L, LexPlan &X, const std::vector<int64_t> &bound
   std::vector<int64_t> pstart;
   std::vector<LexRec> recs;
   for (int64_t p = 0; p < np; ++p) {
-    pstart.push_back(kp[p * L.nsched]);
-    for (int lv = 0; lv < L.nsched; ++lv) {
-      const int64_t e = kp[p * L.nsched + lv + 1];
-      for (int64_t b = kp[p * L.nsched + lv]; b < e;) {
+    pstart.push_back(kp[first[p] + span[2 * p]]);
+    for (int lv = span[2 * p]; lv <= span[2 * p + 1]; ++lv) {
+      const int64_t e = kp[first[p] + lv + 1];
+      for (int64_t b = kp[first[p] + lv]; b < e;) {
         level.push_back(lv);
         for (int w = 0; w < W; ++w) {
           LexRec r = {};
