@@ -136,7 +136,7 @@ struct LexPlan {
   int32_t *row = nullptr;     // [n] device row of a position
   int32_t *pos = nullptr;     // [n] position of a device row
   double *val = nullptr;      // [28 n] chunk by chunk, two slots side by side; then the diagonal
-  int32_t *col = nullptr;     // [27 n] positions
+  int32_t *col = nullptr;     // [27 n] positions, where some chunk is general
   int32_t *dpos = nullptr;    // [n] slot of the diagonal
   unsigned *taken = nullptr;  // the Level::diag_gen whose diagonal the copy holds
   double *x = nullptr, *r = nullptr;  // [n] x and r in this order

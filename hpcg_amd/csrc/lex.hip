@@ -147,6 +147,19 @@ __device__ inline int wave_max(int v) {
   return v;
 }
 
+// A chunk of a plan: rows [start, start + cnt) of a panel that holds [pb, pe);
+// its and its neighbour panels' rows are [lo, hi).
+struct LexChunk {
+  int32_t start, cnt, pb, pe, lo, hi;
+};
+__device__ inline LexChunk lex_chunk(int64_t q, const LexRec *recs, const int32_t *panel_of,
+                                     const int64_t *pstart, int npanels) {
+  const int p = panel_of[q];
+  const int32_t pb = (int32_t)pstart[p], pe = (int32_t)pstart[p + 1];
+  return LexChunk{recs[q].start, recs[q].cnt, pb, pe, p > 0 ? (int32_t)pstart[p - 1] : pb,
+                  p + 1 < npanels ? (int32_t)pstart[p + 2] : pe};
+}
+
 // Copies one chunk's rows (one wavefront).  Where it can, the chunk's slots
 // are aligned by natural column offset (repeated wavefront minimum of each
 // row's next offset, as k_tile_layout does) into five groups that keep the
@@ -156,32 +169,28 @@ __device__ inline int wave_max(int v) {
 // (rows of a hyperplane and their neighbours are consecutive in this order).  A row without the slot's offset gets the value 0 there.  Chunks
 // that do not fit (offsets that do not ascend, stored zeros, more offsets or
 // other couplings, rows further back than the ring of fresh x holds) keep the
-// device slots and 32-bit columns.  *bad is set when a column lies further
-// away than the next panel.
+// device slots and 32-bit columns (k_lex_cols).  Bit 0 of *found is set when a
+// column lies further away than the next panel, bit 1 when a chunk does not fit.
 __global__ __launch_bounds__(kBlock) void k_lex_fill(
     int64_t nrec, int64_t n, LexRec *recs, const int32_t *__restrict__ panel_of,
     const int64_t *__restrict__ pstart, int npanels, const int32_t *__restrict__ row,
     const int32_t *__restrict__ pos, const int32_t *__restrict__ iperm,
     const int32_t *__restrict__ col, const double *__restrict__ val,
     const double *__restrict__ diag, const uint8_t *__restrict__ dslot,
-    const uint8_t *__restrict__ nnz_row, double *__restrict__ lval, int32_t *__restrict__ lcol, int32_t *__restrict__ ldpos,
-    int *bad) {
+    const uint8_t *__restrict__ nnz_row, double *__restrict__ lval, int32_t *__restrict__ ldpos,
+    int *found) {
   const int64_t q = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
   if (q >= nrec) return;  // whole wavefronts
-  const int cnt = recs[q].cnt;
+  const LexChunk C = lex_chunk(q, recs, panel_of, pstart, npanels);
+  const int cnt = C.cnt;
   const int lane = threadIdx.x & 63;
-  const int32_t start = recs[q].start;
+  const int32_t start = C.start, pb = C.pb, pe = C.pe;
   if (lane < kSlots) recs[q].base[lane] = (uint32_t)(start + kLexEdge) << 3;
   if (cnt == 0) return;
-  const int pn = panel_of[q];
-  const int32_t pb = (int32_t)pstart[pn], pe = (int32_t)pstart[pn + 1];
-  const int32_t lo = pn > 0 ? (int32_t)pstart[pn - 1] : pb;
-  const int32_t hi = pn + 1 < npanels ? (int32_t)pstart[pn + 2] : pe;
   const bool live = lane < cnt;
   const int32_t k = start + (live ? lane : 0);
   const int64_t i = row[k];
   const int32_t g = iperm[i];
-  const int64_t at0 = (int64_t)start * kSlots + lane;
   // the row's entries, in slot order: ascending offsets and no stored zeros?
   int m = 0, last = INT_MIN, ds = 0;
   bool plain = true, far = false;
@@ -191,11 +200,11 @@ __global__ __launch_bounds__(kBlock) void k_lex_fill(
     const int o = iperm[cd] - g;
     const int32_t c = pos[cd];
     plain = plain && (m == 0 || o > last);
-    far = far || c < lo || c >= hi;
+    far = far || c < C.lo || c >= C.hi;
     last = o;
     ++m;
   }
-  if (live && far) atomicOr(bad, 1);
+  if (live && far) atomicOr(found, 1);
   plain = plain && m == nnz_row[i];
   bool fits = __ballot(live && !plain) == 0ull;
   // two passes over the chunk's distinct offsets: count each group's, then
@@ -244,20 +253,38 @@ __global__ __launch_bounds__(kBlock) void k_lex_fill(
   }
   if (!fits && live) {
     ds = dslot[i];  // (not by its value, which may be 0 until it is replaced)
-    for (int u = 0; u < kSlots; ++u) {
-      const double v = val[(int64_t)u * n + i];
-      int32_t c = pos[col[(int64_t)u * n + i]];
-      // an unused slot's column need not be near: the row's own x there
-      if (v == 0.0 && (c < lo || c >= hi)) c = k;
-      lval[lex_at(start, cnt, u, lane)] = v;
-      lcol[at0 + (int64_t)u * cnt] = c;
-    }
+    for (int u = 0; u < kSlots; ++u)
+      lval[lex_at(start, cnt, u, lane)] = val[(int64_t)u * n + i];
   }
   if (live) {
     lval[lex_at(start, cnt, kSlots, lane)] = diag[i];
     ldpos[k] = ds;
   }
-  if (lane == 0) recs[q].general = fits ? 0u : 1u;
+  if (lane == 0) {
+    recs[q].general = fits ? 0u : 1u;
+    if (!fits) atomicOr(found, 2);
+  }
+}
+
+// The 32-bit columns of the chunks that k_lex_fill marked general.
+__global__ __launch_bounds__(kBlock) void k_lex_cols(
+    int64_t nrec, int64_t n, const LexRec *recs, const int32_t *__restrict__ panel_of,
+    const int64_t *__restrict__ pstart, int npanels, const int32_t *__restrict__ row,
+    const int32_t *__restrict__ pos, const int32_t *__restrict__ col,
+    const double *__restrict__ val, int32_t *__restrict__ lcol) {
+  const int64_t q = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  if (q >= nrec) return;
+  const LexChunk C = lex_chunk(q, recs, panel_of, pstart, npanels);
+  const int lane = threadIdx.x & 63;
+  if (!recs[q].general || lane >= C.cnt) return;
+  const int32_t k = C.start + lane;
+  const int64_t i = row[k];
+  for (int u = 0; u < kSlots; ++u) {
+    int32_t c = pos[col[(int64_t)u * n + i]];
+    // an unused slot's column need not be near: the row's own x there
+    if (val[(int64_t)u * n + i] == 0.0 && (c < C.lo || c >= C.hi)) c = k;
+    lcol[(int64_t)C.start * kSlots + (int64_t)u * C.cnt + lane] = c;
+  }
 }
 
 __global__ __launch_bounds__(kBlock) void k_lex_zero(int64_t n, double *x) {
@@ -505,9 +532,16 @@ struct Buf {  // device buffer freed on scope exit
   template <class T> T *as() const { return static_cast<T *>(p); }
 };
 
-// The plan with panels of natural rows [bound[p], bound[p + 1]); false when
-// some row couples further than to the next panel.
-bool try_lex(Problem &P, Level &L, LexPlan &X, const std::vector<int64_t> &bound,
+// What the copy takes: values, x, r and three row ids, a record for each
+// wavefront and step, and 32-bit columns where a chunk needs them.
+double lex_bytes(int64_t n, int64_t nrec, bool cols) {
+  return (double)n * (8.0 * (kLexStore + 2) + 4.0 * (3 + (cols ? kSlots : 0))) +
+         (double)nrec * sizeof(LexRec);
+}
+
+// The plan with panels of natural rows [bound[p], bound[p + 1]), in at most
+// `room` bytes; false when some row couples further than to the next panel.
+bool try_lex(Problem &P, Level &L, LexPlan &X, const std::vector<int64_t> &bound, double room,
              hipStream_t s) {
   const int64_t n = L.n;
   const int64_t np = (int64_t)bound.size() - 1;
@@ -601,11 +635,11 @@ bool try_lex(Problem &P, Level &L, LexPlan &X, const std::vector<int64_t> &bound
   X.npanels = (int)np;
   X.waves = W;
   X.nrec = (int64_t)recs.size();
+  if (lex_bytes(n, X.nrec, false) > room) return false;
   X.recs = X.mem.alloc<LexRec>(recs.size());
   X.sptr = X.mem.alloc<int32_t>(sptr.size());
   X.pstart = X.mem.alloc<int64_t>(pstart.size());
   X.val = X.mem.alloc<double>((size_t)kLexStore * n);
-  X.col = X.mem.alloc<int32_t>((size_t)kSlots * n);
   X.dpos = X.mem.alloc<int32_t>(n);
   X.x = X.mem.alloc<double>(n + 2 * kLexEdge) + kLexEdge;
   k_lex_zero<<<grid_for(n + 2 * kLexEdge), kBlock, 0, s>>>(n + 2 * kLexEdge, X.x - kLexEdge);
@@ -621,19 +655,30 @@ bool try_lex(Problem &P, Level &L, LexPlan &X, const std::vector<int64_t> &bound
                            hipMemcpyHostToDevice, s));
   X.taken = X.mem.alloc<unsigned>(1);
   HPCGX_HIP(hipMemcpyAsync(X.taken, L.diag_gen, sizeof(unsigned), hipMemcpyDeviceToDevice, s));
-  Buf pof(sizeof(int32_t) * panel_of.size()), bad(sizeof(int));
+  Buf pof(sizeof(int32_t) * panel_of.size()), flags(sizeof(int));
   HPCGX_HIP(hipMemcpyAsync(pof.p, panel_of.data(), sizeof(int32_t) * panel_of.size(),
                            hipMemcpyHostToDevice, s));
-  HPCGX_HIP(hipMemsetAsync(bad.p, 0, sizeof(int), s));
+  HPCGX_HIP(hipMemsetAsync(flags.p, 0, sizeof(int), s));
   const int64_t wpb = kBlock / 64;
-  k_lex_fill<<<(unsigned)((X.nrec + wpb - 1) / wpb), kBlock, 0, s>>>(
-      X.nrec, n, X.recs, pof.as<int32_t>(), X.pstart, X.npanels, X.row, X.pos, L.iperm, L.col,
-      L.val, L.diag, L.dslot, L.nnz_row, X.val, X.col, X.dpos, bad.as<int>());
+  const unsigned g = (unsigned)((X.nrec + wpb - 1) / wpb);
+  k_lex_fill<<<g, kBlock, 0, s>>>(X.nrec, n, X.recs, pof.as<int32_t>(), X.pstart, X.npanels,
+                                  X.row, X.pos, L.iperm, L.col, L.val, L.diag, L.dslot, L.nnz_row,
+                                  X.val, X.dpos, flags.as<int>());
   HPCGX_LAUNCHED();
-  int far = 0;
-  HPCGX_HIP(hipMemcpyAsync(&far, bad.p, sizeof far, hipMemcpyDeviceToHost, s));
+  int found = 0;
+  HPCGX_HIP(hipMemcpyAsync(&found, flags.p, sizeof found, hipMemcpyDeviceToHost, s));
   HPCGX_HIP(hipStreamSynchronize(s));
-  return far == 0;
+  if (found & 1) return false;
+  X.col = nullptr;
+  if (found & 2) {
+    if (lex_bytes(n, X.nrec, true) > room) return false;
+    X.col = X.mem.alloc<int32_t>((size_t)kSlots * n);
+    k_lex_cols<<<g, kBlock, 0, s>>>(X.nrec, n, X.recs, pof.as<int32_t>(), X.pstart, X.npanels,
+                                    X.row, X.pos, L.col, L.val, X.col);
+    HPCGX_LAUNCHED();
+    HPCGX_HIP(hipStreamSynchronize(s));
+  }
+  return true;
 }
 
 // Panels: the planes of the grids the rows come from, where known.  Else one
@@ -647,13 +692,14 @@ void build_lex(Problem &P, int l, hipStream_t s) {
   LexPlan &X = L.lex;
   X.tried = true;
   const int64_t n = L.n;
-  // a copy takes 27 * 12 + 32 bytes a row; at most half of what is free
+  // at most half of what is free
   size_t avail = 0, total = 0;
   if (hipMemGetInfo(&avail, &total) != hipSuccess) {
     (void)hipGetLastError();
     return;
   }
-  if ((double)n * (12.0 * kSlots + 48.0) > 0.5 * (double)avail) return;
+  const double room = 0.5 * (double)avail;
+  if (lex_bytes(n, 0, false) > room) return;
   std::vector<std::vector<int64_t>> tries;
   std::vector<int64_t> planes{0};
   for (const GridPart &g : grid_parts(P, l))
@@ -671,7 +717,7 @@ void build_lex(Problem &P, int l, hipStream_t s) {
   }
   for (const auto &bound : tries) {
     try {
-      if (try_lex(P, L, X, bound, s)) {
+      if (try_lex(P, L, X, bound, room, s)) {
         X.ready = true;
         return;
       }

@@ -400,9 +400,12 @@ int hpcgx_cg_fleet(hpcgx_problem *p, int ordering, const double *b, double *x, i
  *   "lex_panels"       1/0: FP64 sweeps in the reference's row order run as
  *                      one launch per direction over panels of rows, from a
  *                      copy of the level's matrix in that order built at
- *                      the first such sweep (about 360 bytes a row; only
- *                      where at most half of the free memory holds it), or
- *                      one launch per hyperplane of the schedule
+ *                      the first such sweep (252 bytes a row and 128 for
+ *                      each 64 rows or fewer of a panel's hyperplane; 108
+ *                      bytes a row more where the sparsity needs 32-bit
+ *                      columns; only where at most half of the free memory
+ *                      holds it), or one launch per hyperplane of the
+ *                      schedule
  *                      (default 1; the same bits)
  *   "lex_polls"        polls after which a wait of such a sweep gives up
  *                      (0..2^22, default 2^22: seconds; see

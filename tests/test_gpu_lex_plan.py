@@ -53,3 +53,20 @@ def test_long_grids_same_bits(dims):
     a, b = both(P)
     assert torch.equal(a, b)
     P.close()
+
+
+@pytest.mark.parametrize("dims", [(64, 48, 32), (130, 64, 20)])
+def test_copy_bytes(dims):
+    """No 32-bit columns (108 bytes a row) where the rows' offsets are regular."""
+    import hpcg_amd
+    P = hpcg_amd.Problem.generate(*dims, nlevels=1)
+    n = P.nrow(0)
+    r, x = random_pair(n)
+    before = P.memory_use()
+    P.symgs(r, x, ordering="lexicographic")
+    P.check()
+    # 28 values, x, r, three row ids; a 128-byte record per wavefront and step
+    # (at most one step per two rows of these planes' shortest hyperplanes)
+    grown = (P.memory_use() - before) / n
+    assert 252 <= grown < 252 + 32, grown
+    P.close()
