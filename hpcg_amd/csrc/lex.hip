@@ -170,7 +170,8 @@ __device__ inline LexChunk lex_chunk(int64_t q, const LexRec *recs, const int32_
 // that do not fit (offsets that do not ascend, stored zeros, more offsets or
 // other couplings, rows further back than the ring of fresh x holds) keep the
 // device slots and 32-bit columns (k_lex_cols).  Bit 0 of *found is set when a
-// column lies further away than the next panel, bit 1 when a chunk does not fit.
+// column lies further away than the next panel, bit 1 when a chunk does not fit;
+// joint[p] when panels p - 1 and p couple.
 __global__ __launch_bounds__(kBlock) void k_lex_fill(
     int64_t nrec, int64_t n, LexRec *recs, const int32_t *__restrict__ panel_of,
     const int64_t *__restrict__ pstart, int npanels, const int32_t *__restrict__ row,
@@ -178,7 +179,7 @@ __global__ __launch_bounds__(kBlock) void k_lex_fill(
     const int32_t *__restrict__ col, const double *__restrict__ val,
     const double *__restrict__ diag, const uint8_t *__restrict__ dslot,
     const uint8_t *__restrict__ nnz_row, double *__restrict__ lval, int32_t *__restrict__ ldpos,
-    int *found) {
+    int *found, int *joint) {
   const int64_t q = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
   if (q >= nrec) return;  // whole wavefronts
   const LexChunk C = lex_chunk(q, recs, panel_of, pstart, npanels);
@@ -193,7 +194,7 @@ __global__ __launch_bounds__(kBlock) void k_lex_fill(
   const int32_t g = iperm[i];
   // the row's entries, in slot order: ascending offsets and no stored zeros?
   int m = 0, last = INT_MIN, ds = 0;
-  bool plain = true, far = false;
+  bool plain = true, far = false, before = false, after = false;
   for (int j = 0; j < kSlots; ++j) {
     if (val[(int64_t)j * n + i] == 0.0) continue;
     const int32_t cd = col[(int64_t)j * n + i];
@@ -201,10 +202,14 @@ __global__ __launch_bounds__(kBlock) void k_lex_fill(
     const int32_t c = pos[cd];
     plain = plain && (m == 0 || o > last);
     far = far || c < C.lo || c >= C.hi;
+    before = before || c < pb;
+    after = after || c >= pe;
     last = o;
     ++m;
   }
   if (live && far) atomicOr(found, 1);
+  if (__ballot(live && before) && lane == 0) joint[panel_of[q]] = 1;
+  if (__ballot(live && after) && lane == 0) joint[panel_of[q] + 1] = 1;
   plain = plain && m == nnz_row[i];
   bool fits = __ballot(live && !plain) == 0ull;
   // two passes over the chunk's distinct offsets: count each group's, then
@@ -264,6 +269,18 @@ __global__ __launch_bounds__(kBlock) void k_lex_fill(
     recs[q].general = fits ? 0u : 1u;
     if (!fits) atomicOr(found, 2);
   }
+}
+
+// No waiting where two panels do not couple (the last plane of one problem of a
+// fleet and the first of the next).
+__global__ __launch_bounds__(kBlock) void k_lex_apart(int64_t nrec, LexRec *recs,
+                                                      const int32_t *__restrict__ panel_of,
+                                                      const int *__restrict__ joint) {
+  const int64_t q = gtid();
+  if (q >= nrec) return;
+  const int p = panel_of[q];
+  if (!joint[p]) recs[q].need[0] = 0;
+  if (!joint[p + 1]) recs[q].need[1] = 0;
 }
 
 // The 32-bit columns of the chunks that k_lex_fill marked general.
@@ -655,15 +672,19 @@ bool try_lex(Problem &P, Level &L, LexPlan &X, const std::vector<int64_t> &bound
                            hipMemcpyHostToDevice, s));
   X.taken = X.mem.alloc<unsigned>(1);
   HPCGX_HIP(hipMemcpyAsync(X.taken, L.diag_gen, sizeof(unsigned), hipMemcpyDeviceToDevice, s));
-  Buf pof(sizeof(int32_t) * panel_of.size()), flags(sizeof(int));
+  // (flags: what k_lex_fill found, then its joint)
+  Buf pof(sizeof(int32_t) * panel_of.size()), flags(sizeof(int) * (np + 2));
   HPCGX_HIP(hipMemcpyAsync(pof.p, panel_of.data(), sizeof(int32_t) * panel_of.size(),
                            hipMemcpyHostToDevice, s));
-  HPCGX_HIP(hipMemsetAsync(flags.p, 0, sizeof(int), s));
+  HPCGX_HIP(hipMemsetAsync(flags.p, 0, sizeof(int) * (np + 2), s));
   const int64_t wpb = kBlock / 64;
   const unsigned g = (unsigned)((X.nrec + wpb - 1) / wpb);
   k_lex_fill<<<g, kBlock, 0, s>>>(X.nrec, n, X.recs, pof.as<int32_t>(), X.pstart, X.npanels,
                                   X.row, X.pos, L.iperm, L.col, L.val, L.diag, L.dslot, L.nnz_row,
-                                  X.val, X.dpos, flags.as<int>());
+                                  X.val, X.dpos, flags.as<int>(), flags.as<int>() + 1);
+  HPCGX_LAUNCHED();
+  k_lex_apart<<<grid_for(X.nrec), kBlock, 0, s>>>(X.nrec, X.recs, pof.as<int32_t>(),
+                                                  flags.as<int>() + 1);
   HPCGX_LAUNCHED();
   int found = 0;
   HPCGX_HIP(hipMemcpyAsync(&found, flags.p, sizeof found, hipMemcpyDeviceToHost, s));

@@ -78,3 +78,21 @@ def test_lex_polls_reported_by_host_surface():
     r = subprocess.run([CHECK], capture_output=True, text=True, timeout=100)
     print(r.stdout, r.stderr, flush=True)
     assert r.returncode == 0
+
+
+def test_fleet_problems_do_not_wait_for_each_other():
+    """One plane a problem: no panel couples to another, so no wait is left to
+    give up, even under a limit of 0 polls."""
+    import hpcg_amd
+    import torch
+    P = hpcg_amd.Problem.generate_fleet(((24, 16, 1), (8, 40, 1), (70, 9, 1)) * 8, nlevels=1)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(9)
+    r = torch.rand(P.nrow(0), generator=g, dtype=torch.float64, device="cuda") - 0.5
+    x = torch.zeros_like(r)
+    assert limited(P, lambda: P.symgs(r, x, ordering="lexicographic")) is None
+    P.tune("lex_panels", 0)
+    y = torch.zeros_like(r)
+    P.symgs(r, y, ordering="lexicographic")
+    assert torch.equal(x, y)
+    P.close()
