@@ -751,6 +751,15 @@ void build_lex(Problem &P, int l, hipStream_t s) {
   }
 }
 
+// The copy's allocations, copies and waits would end a capture of other work
+// under way on another stream (by any thread, in the global mode): this thread
+// leaves that rule while it builds, and touches no captured stream.
+struct BesideCaptures {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  BesideCaptures() { HPCGX_HIP(hipThreadExchangeStreamCaptureMode(&mode)); }
+  ~BesideCaptures() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 bool capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &st) != hipSuccess) {
@@ -772,7 +781,10 @@ bool launch_symgs_lex(Problem &P, int l, const double *r, double *x, hipStream_t
   // iterations run inside calls that own the problem's vectors anyway.
   const bool own = s && (s == P.graph.cap || s == P.fleet.graph.cap);
   if (!own && capturing(s)) return false;
-  if (!X.tried && !own) build_lex(P, l, s);
+  if (!X.tried && !own) {
+    const BesideCaptures relaxed;
+    build_lex(P, l, s);
+  }
   if (!X.ready) return false;
   // one scratch per level: a sweep on another stream follows the last one
   if (!own) {

@@ -70,3 +70,49 @@ def test_copy_bytes(dims):
     grown = (P.memory_use() - before) / n
     assert 252 <= grown < 252 + 32, grown
     P.close()
+
+
+@pytest.mark.parametrize("thread", [False, True])
+def test_first_sweep_beside_a_capture(thread):
+    """The first sweep allocates its copy; a capture on another stream, by this
+    thread or another, stays valid and the copy is built."""
+    import threading
+
+    import hpcg_amd
+    import torch
+    P = hpcg_amd.Problem.generate(24, 16, 12, nlevels=1)
+    n = P.nrow(0)
+    r, x = random_pair(n)
+    y = torch.zeros_like(x)
+    side = torch.cuda.Stream()
+    before = P.memory_use()
+    z, fails = x.clone(), []
+
+    def sweep():
+        try:
+            with torch.cuda.stream(side):
+                P.symgs(r, z, ordering="lexicographic")
+        except Exception as e:  # (reported by the test's own thread)
+            fails.append(e)
+
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y.copy_(x)
+        if thread:
+            t = threading.Thread(target=sweep)
+            t.start()
+            t.join()
+        else:
+            sweep()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert not fails, fails
+    P.check()
+    assert torch.equal(x, y)
+    assert P.memory_use() - before >= 252 * n
+    P.tune("lex_panels", 0)
+    w = x.clone()
+    P.symgs(r, w, ordering="lexicographic")
+    assert torch.equal(z, w)
+    P.close()
