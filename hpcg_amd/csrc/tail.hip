@@ -27,6 +27,7 @@
 // 0.6 us of dependent LDS reads, 27 subtractions, a division and the barrier;
 // a step over 512 rows streamed from L2 1.8 us (27 loads of 512 bytes for each
 // of 8 wavefronts); and 2 us of first loads a level and sweep.
+#include <atomic>
 #include <climits>
 
 #include "internal.hpp"
@@ -258,6 +259,21 @@ __global__ __launch_bounds__(64 * kTailWaves) void k_tail(const TailArgs<V, T> A
     A.x[(int64_t)i * A.stride + blockIdx.x] = lds[A.lev[0].xo + i];
 }
 
+// Lets a kernel ask for kTailLds on the current device, once.  The limit belongs
+// to the function, for every problem and thread: with each launch's own size,
+// one thread could lower it between another's setting and launch.
+template <class V, class T>
+void allow_lds() {
+  static std::atomic<uint64_t> done{0};  // devices
+  int dev = 0;
+  HPCGX_HIP(hipGetDevice(&dev));
+  const uint64_t bit = dev < 64 ? (uint64_t)1 << dev : 0;
+  if (done.load() & bit) return;
+  HPCGX_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_tail<V, T>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTailLds));
+  done.fetch_or(bit);
+}
+
 template <class V, class T, class F>
 bool tail(const Problem &P, int l0, int columns, const T *r, T *x, double *rz,
           const double *r64, hipStream_t s, F &&fields) {
@@ -293,9 +309,7 @@ bool tail(const Problem &P, int l0, int columns, const T *r, T *x, double *rz,
   }
   const size_t bytes = sizeof(T) * (size_t)at;
   if (bytes > kTailLds) return false;
-  if (bytes > 32768)  // (what any kernel may ask for; a setting of the current device)
-    HPCGX_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_tail<V, T>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+  if (bytes > 32768) allow_lds<V, T>();  // (what any kernel may ask for)
   k_tail<V, T><<<(unsigned)columns, 64 * kTailWaves, bytes, s>>>(A);
   HPCGX_LAUNCHED();
   return true;
