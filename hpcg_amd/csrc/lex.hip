@@ -47,6 +47,7 @@ namespace {
 constexpr int kLexWaves = 4;               // wavefronts per workgroup, at most
 constexpr int kLexPad = 32;                // progress counters 128 bytes apart
 constexpr int64_t kLexRows = 256;          // see build_lex
+constexpr int64_t kLexWide = 6;            // see try_lex
 constexpr int kLexAhead = 1;               // steps the matrix loads run ahead
 constexpr int kLexIn = 4, kLexOut = 9;     // slots of the own and of a neighbour panel
 static_assert(2 * kLexOut + 2 * kLexIn + 1 == kSlots, "slot groups");
@@ -649,6 +650,16 @@ bool try_lex(Problem &P, Level &L, LexPlan &X, const std::vector<int64_t> &bound
         recs[st * W + w].need[1] = p + 1 < np ? (int32_t)(sptr[p + 2] - b) : 0;
     }
   }
+  // A panel is one workgroup's, 256 rows a step at most, and rows whose fresh
+  // neighbours lie beyond the ring of x (hyperplanes of over 570 rows a panel)
+  // take about 4.9 us a step; a launch of a hyperplane of hundreds to thousands
+  // of rows takes 27 to 34 us, spread over the chip.  So a panel of more than
+  // six steps a hyperplane is slower, ms a sweep, panels / launches: one plane
+  // of 2048^2 159 / 337, of 4096^2 (5.7 steps) 679 / 731, of 6000^2 (8.3) 1483 /
+  // 1175, of 8192^2 (11) 2735 / 1573.
+  int64_t longest = 0;
+  for (int64_t p = 0; p < np; ++p) longest = std::max<int64_t>(longest, sptr[p + 1] - sptr[p]);
+  if (longest > kLexWide * L.nsched) throw Error(HPCGX_EUNSUP, "hyperplanes too wide for panels");
   X.npanels = (int)np;
   X.waves = W;
   X.nrec = (int64_t)recs.size();
@@ -743,7 +754,7 @@ void build_lex(Problem &P, int l, hipStream_t s) {
         return;
       }
       X.mem.clear();
-    } catch (const std::exception &) {  // no room for the copy: one launch per hyperplane
+    } catch (const std::exception &) {  // too wide, or no room: one launch per hyperplane
       (void)hipGetLastError();
       X.mem.clear();
       return;
@@ -774,7 +785,9 @@ bool capturing(hipStream_t s) {
 bool launch_symgs_lex(Problem &P, int l, const double *r, double *x, hipStream_t s) {
   Level &L = P.L[l];
   LexPlan &X = L.lex;
-  if (!P.use_lex || L.n < 2 || L.n >= ((int64_t)1 << 29) - 2 * kLexEdge)
+  // (two hyperplanes or fewer are no more launches than this path's four: 22 us
+  // against 29)
+  if (!P.use_lex || L.nsched < 3 || L.n >= ((int64_t)1 << 29) - 2 * kLexEdge)
     return false;
   // Under a caller's capture the copy cannot be built, and its scratch would
   // be used at replays this call cannot order; the problem's own captured

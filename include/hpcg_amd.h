@@ -404,8 +404,9 @@ int hpcgx_cg_fleet(hpcgx_problem *p, int ordering, const double *b, double *x, i
  *                      each 64 rows or fewer of a panel's hyperplane; 108
  *                      bytes a row more where the sparsity needs 32-bit
  *                      columns; only where at most half of the free memory
- *                      holds it), or one launch per hyperplane of the
- *                      schedule
+ *                      holds it, and not for planes of more than about
+ *                      4200 x 4200 points), or one launch per hyperplane of
+ *                      the schedule
  *                      (default 1; the same bits)
  *   "lex_polls"        polls after which a wait of such a sweep gives up
  *                      (0..2^22, default 2^22: seconds; see

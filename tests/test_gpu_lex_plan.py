@@ -116,3 +116,18 @@ def test_first_sweep_beside_a_capture(thread):
     P.symgs(r, w, ordering="lexicographic")
     assert torch.equal(z, w)
     P.close()
+
+
+@pytest.mark.parametrize("dims,panels", [((512, 512, 1), True), ((4500, 4500, 1), False),
+                                         ((1, 1, 2), False), ((1, 1, 3), True)])
+def test_rule_for_panels(dims, panels):
+    """A plane so wide that one workgroup takes longer over a hyperplane than a
+    launch, and a level of two hyperplanes, keep one launch per hyperplane."""
+    import hpcg_amd
+    P = hpcg_amd.Problem.generate(*dims, nlevels=1)
+    r, x = random_pair(P.nrow(0))
+    before = P.memory_use()
+    P.symgs(r, x, ordering="lexicographic")
+    P.check()
+    assert (P.memory_use() > before) == panels
+    P.close()
