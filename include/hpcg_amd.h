@@ -444,18 +444,18 @@ int hpcgx_cg_fleet(hpcgx_problem *p, int ordering, const double *b, double *x, i
  *                      residual recompute) (default 1; the same x and
  *                      residuals)
  *   "gs_block"         threads per workgroup of the finest level's FP64
- *                      colour steps of more than 3 * 2^20 rows (and of its
+ *                      colour steps of more than 6 * 2^20 rows (and of its
  *                      zero-x steps): 64, 128, 256 or 512 (default 256);
  *                      smaller steps run with all of a row's loads in flight
  *                      at a fixed shape
  *   "gs_waves"         1/0: the finest level's FP64 colour steps of more than
- *                      3 * 2^20 rows run under register caps that allow 7
+ *                      6 * 2^20 rows run under register caps that allow 7
  *                      waves per SIMD (default 1); 0 leaves the register
  *                      count to the compiler
  *   "x_pairs"          0-15: on tiles whose offset words are all affine and
  *                      whose slot 3m + 2 has the base one above slot 3m's
  *                      (all m), the finest level's kernels (FP64 colour
- *                      steps: those of more than 3 * 2^20 rows) take slot 3m +
+ *                      steps: those of more than 6 * 2^20 rows) take slot 3m +
  *                      2's x values from slot 3m's moved one lane
  *                      (cross-lane permute) instead of a second gather.
  *                      Bit 0: the FP64 colour steps without r.z partials
