@@ -574,6 +574,7 @@ int hpcgx_autotune(hpcgx_problem *p, int ordering, int iterations, char *report,
     struct Knob {
       const char *key;
       std::vector<double> values;
+      bool live = true;  // some launch of this problem depends on it
     };
     bool any_c16 = false;
     for (int l = 0; l < P.nlevels; ++l) any_c16 = any_c16 || P.L[l].c16;
@@ -588,9 +589,14 @@ int hpcgx_autotune(hpcgx_problem *p, int ordering, int iterations, char *report,
     knobs.push_back({"spmv_order", {0, 1}});
     knobs.push_back({"xcd_remap", {0, 1}});
     if (P.L[0].c16) {  // the finest colour steps' shape: workgroup size, register cap
+      const hpcgx::Level &A = P.L[0];
+      bool capped = false;  // full steps other than with all loads in flight
+      for (int c = 0; c < A.ncolors; ++c)
+        capped = capped || A.color_ptr[c + 1] - A.color_ptr[c] > hpcgx::kDeepRows;
       knobs.push_back({"gs_block", {256, 128, 512, 64}});
-      knobs.push_back({"gs_waves", {1, 0}});
-      knobs.push_back({"x_pairs", {3, 0}});  // applies at 256 threads with the caps
+      knobs.push_back({"gs_waves", {1, 0}, capped});
+      // applies at 256 threads with the caps, and to a streamed matrix's SpMV
+      knobs.push_back({"x_pairs", {3, 0}, capped || A.stream});
     }
     std::string log;
     char line[160];
@@ -610,7 +616,7 @@ int hpcgx_autotune(hpcgx_problem *p, int ordering, int iterations, char *report,
         std::snprintf(line, sizeof line, "%s=%g: %.4f ms/iteration\n", k.key, k.values[q],
                       tmin[q] * 1e3);
         log += line;
-        if (tmin[q] < best_t) {
+        if (tmin[q] < best_t && (k.live || q == 0)) {  // (else equal code: the default)
           best_t = tmin[q];
           best_v = k.values[q];
         }

@@ -483,6 +483,9 @@ inline Col16 col16_of(const Problem &P, const Level &L, int64_t begin = 0) {
 // Windows of 4 and 16 measure the same in FP64, 446 and 468 in FP32 at 256^3;
 // each die's own eighth of the rows (xcd_block) is slower than windows.
 constexpr int64_t kWin = 8;
+// The largest FP64 colour step that runs with all of a row's loads in flight
+// (kernels.hip's gs_row_deep).
+constexpr int64_t kDeepRows = (int64_t)6 << 20;
 __device__ inline int64_t window_block(int64_t b, int64_t G) {
   const int64_t q = b % (8 * kWin), w = b - q;
   return w + 8 * kWin <= G ? w + (q % 8) * kWin + q / 8 : b;

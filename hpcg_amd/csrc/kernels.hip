@@ -399,12 +399,11 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
 // the diagonal array (as in the zero-x step): 8 bytes a row for 27 compares
 // and selects.
 //
-// kDeepRows, the largest step that runs so, is where the two cross (us a step,
+// kDeepRows (internal.hpp) is where the two cross (us a step,
 // k_gs_range16 / this, the medians of several allocations from 3.5M rows on):
 // 32768 rows 7.7 / 4.6, 137280 12.8 / 10.1, 262144 20.5 / 16.2, 884736 50.0 /
 // 45.4, 2.1M 107.3 / 101, 3.55M 189 / 170, 4.7M 266 / 258, 8.9M 474 / 487,
 // 16.8M 921 / 923.
-constexpr int64_t kDeepRows = (int64_t)6 << 20;
 template <bool STREAM>
 __device__ inline double gs_row_deep(const Col16 &C, int64_t i, int64_t n,
                                      const int32_t *__restrict__ col,

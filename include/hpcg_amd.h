@@ -519,7 +519,8 @@ int hpcgx_tune(hpcgx_problem *p, const char *key, double value);
  * "xcd_remap", and, where the finest level has narrow column ids, "gs_block", "gs_waves" and
  * "x_pairs"; a fleet times hpcgx_cg_fleet and tunes "fleet_blocks" in place of
  * "spmv_dot_blocks"), keeping the fastest value of each.  Each knob's candidates are timed
- * in two interleaved rounds and keep their faster time.  Writes one line per candidate (that
+ * in two interleaved rounds and keep their faster time; where no launch of this problem depends
+ * on a knob (gs_waves, x_pairs: see there) its default stays.  Writes one line per candidate (that
  * time) and per choice into `report` (may be NULL).  Uses the default stream; synchronous.
  * Changing "spmv_dot_blocks" changes the dots' summation order. */
 int hpcgx_autotune(hpcgx_problem *p, int ordering, int iterations, char *report,
