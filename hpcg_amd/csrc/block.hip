@@ -384,8 +384,9 @@ __device__ __attribute__((always_inline)) inline void bgs32_row_zero_live(
 // LIVE: the live slots only (bgs32_row_zero_live), else every slot (bgs32_row_zero)
 template <bool STREAM, int S, bool LIVE = false>
 __global__ __launch_bounds__(kBlock) void k_bgs32_rows_zero(
-    int64_t begin, int64_t end, int64_t n, Col16 C, const uint32_t *__restrict__ vc, const int32_t *__restrict__ col,
-    const half_t *__restrict__ val16, const float *__restrict__ diag32,
+    int64_t begin, int64_t end, int64_t n, Col16 C, const uint32_t *__restrict__ vc,
+    const int32_t *__restrict__ col, const half_t *__restrict__ val16,
+    const float *__restrict__ diag32,
     const float *__restrict__ R, float *X) {
   constexpr int W = S / 4;
   const int64_t g = window_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;

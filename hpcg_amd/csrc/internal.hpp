@@ -524,8 +524,6 @@ void launch_spmv(const Problem &P, const Level &L, const double *x, double *y,
 // path only).
 void launch_symgs_rows(const Problem &P, const Level &L, int64_t begin, int64_t end,
                        const double *r, double *x, hipStream_t s, double *dpart = nullptr);
-// Reference-order symmetric sweep by panels (lex.hip); false (nothing
-// launched) where it does not apply.
 // The multicolour V-cycle from level l down in one launch (tail.hip), rz as
 // symgs; false (nothing launched) where the levels are too large for it.
 bool launch_tail(const Problem &P, int l, const double *r, double *x, hipStream_t s, double *rz);
@@ -537,6 +535,8 @@ bool launch_tail32(const Problem &P, int l, const float *r, float *x, hipStream_
 // where the level has no narrow ids.
 bool launch_symgs_turn(const Problem &P, const Level &L, int64_t begin, int64_t end,
                        const double *r, double *x, hipStream_t s, double *dpart, bool zero_x);
+// Reference-order symmetric sweep by panels (lex.hip); false (nothing
+// launched) where it does not apply.
 bool launch_symgs_lex(Problem &P, int l, const double *r, double *x, hipStream_t s);
 void launch_symgs_list(const Level &L, const int32_t *rows, int64_t count,
                        const double *r, double *x, hipStream_t s);
@@ -603,8 +603,9 @@ void launch_update_p32(int64_t n, const float *z, double *p, const double *scala
 void launch_update_p(int64_t n, const double *z, double *p,
                      const double *scalars, hipStream_t s, bool stream);
 // r = b - A x on the finest level L with r32 = (float)r (unless null; with it,
-// from FP16 values where they are exact) and r.r (into the scalars) in one pass over the row chunks; false (nothing launched) where
-// the chunk partials do not cover L
+// from FP16 values where they are exact) and r.r (into the scalars) in one pass
+// over the row chunks; false (nothing launched) where the chunk partials do not
+// cover L
 bool launch_residual_fused(Problem &P, const Level &L, const double *b, const double *x,
                            double *r, float *r32, hipStream_t s);
 void launch_residual0(Problem &P, int64_t n, const double *b, const double *Ap,

@@ -353,8 +353,9 @@ __global__ __launch_bounds__(kBlock) void k_gs_range(
 
 // k_gs_range with narrow column ids (begin is a colour's first row).  BS
 // threads per workgroup; W: the waves-per-EU floor given to the compiler
-// (7 caps it at 72 VGPRs; 1 leaves it free, 94 registers).  The finest level's workgroup size and cap are
-// tuning knobs ("gs_block", "gs_waves"); other levels use kBlock and 7.
+// (7 caps it at 72 VGPRs; 1 leaves it free, 94 registers).  The finest level's
+// workgroup size and cap are tuning knobs ("gs_block", "gs_waves"); other levels
+// use kBlock and 7.
 template <bool STREAM, bool FINEST, int BS, int W, bool PAIRS = false>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_gs_range16(
     int64_t begin, int64_t end, int64_t n, Col16 C, const int32_t *__restrict__ col,
@@ -649,7 +650,8 @@ template <bool STREAM, bool ZERO, bool RZ>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_gs_turn(
     int64_t begin, int64_t end, int64_t n, Col16 C, const int32_t *__restrict__ col,
     const double *__restrict__ val, const double *__restrict__ diag,
-    const uint8_t *__restrict__ dslot, const double *__restrict__ r, double *x, double *__restrict__ dpart) {
+    const uint8_t *__restrict__ dslot, const double *__restrict__ r, double *x,
+    double *__restrict__ dpart) {
   const int64_t i = begin + window_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   double s = 0.0;
   if (i < end) {
@@ -757,7 +759,8 @@ __device__ inline void gs_row_zero_live(const Col16 &C, int64_t begin, int64_t i
 template <bool STREAM, bool FINEST, int BS, bool LIVE = false>
 __global__ __launch_bounds__(BS) void k_gs_zero16(
     int64_t begin, int64_t end, int64_t n, Col16 C, const int32_t *__restrict__ col,
-    const double *__restrict__ val, const double *__restrict__ diag, const double *__restrict__ r, double *x, bool xcd) {
+    const double *__restrict__ val, const double *__restrict__ diag,
+    const double *__restrict__ r, double *x, bool xcd) {
   const int64_t i = begin + xcd_window(xcd, true) * BS + threadIdx.x;
   if (i >= end) return;
   if (LIVE)

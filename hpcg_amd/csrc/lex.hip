@@ -167,8 +167,9 @@ __device__ inline LexChunk lex_chunk(int64_t q, const LexRec *recs, const int32_
 // ascending order: kLexOut slots for the panel before, kLexIn for lower rows
 // of its own panel, the diagonal, kLexIn for upper rows, kLexOut for the panel
 // after; a slot's column must be one base plus the row's place in the chunk
-// (rows of a hyperplane and their neighbours are consecutive in this order).  A row without the slot's offset gets the value 0 there.  Chunks
-// that do not fit (offsets that do not ascend, stored zeros, more offsets or
+// (rows of a hyperplane and their neighbours are consecutive in this order).  A
+// row without the slot's offset gets the value 0 there.  Chunks that do not fit
+// (offsets that do not ascend, stored zeros, more offsets or
 // other couplings, rows further back than the ring of fresh x holds) keep the
 // device slots and 32-bit columns (k_lex_cols).  Bit 0 of *found is set when a
 // column lies further away than the next panel, bit 1 when a chunk does not fit;
@@ -815,7 +816,8 @@ bool launch_symgs_lex(Problem &P, int l, const double *r, double *x, hipStream_t
   const dim3 g(X.npanels), b(64 * X.waves);
 #define HPCGX_LEX(ST, DIR)                                                                       \
   k_lex_sweep<ST, DIR><<<g, b, 0, s>>>(X.npanels, X.waves, X.recs, X.sptr, X.pstart, X.val,      \
-                                       X.col, X.r, X.x, X.prog + DIR * X.nprog, P.lex_polls, P.wave_err)
+                                       X.col, X.r, X.x, X.prog + DIR * X.nprog, P.lex_polls,     \
+                                       P.wave_err)
   if (L.stream) {
     HPCGX_LEX(true, 0);
     HPCGX_LEX(true, 1);

@@ -135,7 +135,8 @@ __global__ __launch_bounds__(64 * kTailWaves) void k_tail(const TailArgs<V, T> A
   }
   for (int l = 0; l < A.nlev; ++l)
     for (int i = threadIdx.x; i < A.lev[l].n; i += 64 * kTailWaves) lds[A.lev[l].xo + i] = (T)0;
-  for (int i = threadIdx.x; i < A.lev[0].n; i += 64 * kTailWaves) lds[A.lev[0].ro + i] = A.r[(int64_t)i * A.stride + blockIdx.x];
+  for (int i = threadIdx.x; i < A.lev[0].n; i += 64 * kTailWaves)
+    lds[A.lev[0].ro + i] = A.r[(int64_t)i * A.stride + blockIdx.x];
   lds_barrier();
 
   // down the levels and up again
@@ -255,7 +256,7 @@ __global__ __launch_bounds__(64 * kTailWaves) void k_tail(const TailArgs<V, T> A
       lds_barrier();
     }
   }
-  for (int i = threadIdx.x; i < A.lev[0].n; i += 64 * kTailWaves) 
+  for (int i = threadIdx.x; i < A.lev[0].n; i += 64 * kTailWaves)
     A.x[(int64_t)i * A.stride + blockIdx.x] = lds[A.lev[0].xo + i];
 }
 

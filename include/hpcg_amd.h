@@ -91,7 +91,10 @@ typedef struct {
   int64_t ncoarse;       /* rows of the next level (0 on coarsest) */
   int wave;              /* 1: multicolour sweeps run as a wavefront */
   int nslabs;            /* slabs of the wavefront schedule */
-  int col16;             /* 1: narrow column ids (tile base + offset) built */
+  int col16;             /* 1: narrow column ids (tile base + offset) built, in tiles that
+                          * start at multiples of 64 rows.  0 does not mean none: levels of
+                          * 4096 rows and more hold them in any case, and the two counts
+                          * below are theirs */
   int64_t wide_tiles;    /* tiles of 64 rows that keep 32-bit column ids */
   int64_t byte_tiles;    /* tiles of 64 rows with 8-bit column offsets */
 } hpcgx_level_info;
@@ -358,7 +361,10 @@ int hpcgx_cg_fleet(hpcgx_problem *p, int ordering, const double *b, double *x, i
  *   "wave_min_rows"    levels with at least this many rows get a wavefront
  *                      schedule (default 2^23)
  *   "wave_slab_factor" slab width in units of the matrix bandwidth (>= 1)
- *   "xcd_remap"        1/0: map workgroups to XCD-contiguous row ranges
+ *   "xcd_remap"        1/0: map workgroups to XCD-contiguous row ranges, or
+ *                      in order or in windows, whichever measured faster for
+ *                      the kernel (default 0; FP64 colour steps of at most
+ *                      6 * 2^20 rows run in windows either way)
  *   "pair_rows"        1/0: colour steps with two adjacent rows per thread
  *                      (16-byte matrix loads)
  *   "stream_min_bytes" matrices larger than this are read with non-temporal
