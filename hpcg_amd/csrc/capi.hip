@@ -102,6 +102,9 @@ void alloc_solver_state(hpcgx::Problem &P) {
   P.nrz_partials = (n + hpcgx::kTile - 1) / hpcgx::kTile + 64;  // one per wavefront of rows
   P.rz_part = P.arena.alloc<double>(P.nrz_partials);
   P.dot_parts = P.arena.alloc<double>(hpcgx::kDotParts);
+  // what is allocated from here on (mixed and block state) comes before the
+  // copies of the reference-order sweeps, which can do without
+  P.arena.reclaim = [&P] { return hpcgx::lex_drop(P); };
 }
 
 // shared tail of both setup paths: schedules, reordering, links

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <functional>
 #include <new>
 #include <stdexcept>
 #include <string>
@@ -87,11 +88,17 @@ int guard(F &&f) {
 struct DeviceArena {
   std::vector<void *> ptrs;
   double bytes = 0.0;
+  std::function<bool()> reclaim;  // gives back memory that can be done without, if any
   template <class T>
   T *alloc(size_t count) {
     void *p = nullptr;
     if (count == 0) count = 1;
-    HPCGX_HIP(hipMalloc(&p, count * sizeof(T)));
+    hipError_t e = hipMalloc(&p, count * sizeof(T));
+    if (e == hipErrorOutOfMemory && reclaim && reclaim()) {
+      (void)hipGetLastError();
+      e = hipMalloc(&p, count * sizeof(T));
+    }
+    HPCGX_HIP(e);
     ptrs.push_back(p);
     bytes += double(count) * sizeof(T);
     return static_cast<T *>(p);
@@ -538,6 +545,9 @@ bool launch_symgs_turn(const Problem &P, const Level &L, int64_t begin, int64_t 
 // Reference-order symmetric sweep by panels (lex.hip); false (nothing
 // launched) where it does not apply.
 bool launch_symgs_lex(Problem &P, int l, const double *r, double *x, hipStream_t s);
+// Frees the copies of the levels that such sweeps have built (the next sweep
+// builds one again where there is room); false where there are none.
+bool lex_drop(Problem &P);
 void launch_symgs_list(const Level &L, const int32_t *rows, int64_t count,
                        const double *r, double *x, hipStream_t s);
 // The colour step of a forward sweep whose x was zero when the sweep began

@@ -783,6 +783,24 @@ bool capturing(hipStream_t s) {
 
 }  // namespace
 
+bool lex_drop(Problem &P) {
+  bool any = false;
+  for (int l = 0; l < P.nlevels; ++l) {
+    LexPlan &X = P.L[l].lex;
+    if (!X.ready) continue;
+    // (captured iterations run inside calls that wait for them)
+    if (X.done) HPCGX_HIP(hipEventSynchronize(X.done));
+    X.mem.clear();
+    X.ready = X.tried = false;
+    any = true;
+  }
+  if (any) {
+    P.graph.reset();
+    P.fleet.graph.reset();
+  }
+  return any;
+}
+
 bool launch_symgs_lex(Problem &P, int l, const double *r, double *x, hipStream_t s) {
   Level &L = P.L[l];
   LexPlan &X = L.lex;

@@ -406,13 +406,14 @@ int hpcgx_cg_fleet(hpcgx_problem *p, int ordering, const double *b, double *x, i
  *   "lex_panels"       1/0: FP64 sweeps in the reference's row order run as
  *                      one launch per direction over panels of rows, from a
  *                      copy of the level's matrix in that order built at
- *                      the first such sweep (252 bytes a row and 128 for
- *                      each 64 rows or fewer of a panel's hyperplane; 108
- *                      bytes a row more where the sparsity needs 32-bit
- *                      columns; only where at most half of the free memory
- *                      holds it, and not for planes of more than about
- *                      4200 x 4200 points), or one launch per hyperplane of
- *                      the schedule
+ *                      the first such sweep, or one launch per hyperplane of
+ *                      the schedule.  The copy takes 252 bytes a row, 128 for
+ *                      each 64 rows or fewer of a panel's hyperplane and,
+ *                      where the sparsity needs 32-bit columns, 108 bytes a
+ *                      row more.  It is built only where at most half of the
+ *                      free memory holds it, and not for planes of more than
+ *                      about 4200 x 4200 points, and is given back when the
+ *                      problem's mixed or block state finds no room
  *                      (default 1; the same bits)
  *   "lex_polls"        polls after which a wait of such a sweep gives up
  *                      (0..2^22, default 2^22: seconds; see
