@@ -197,6 +197,34 @@ __device__ __attribute__((always_inline)) inline void row_terms(
   }
 }
 
+// y += the terms of row i over 32-bit columns, of X's rows below `below`.
+template <int S, class T, class H, int V>
+__device__ __attribute__((always_inline)) inline void row_again(
+    T (&y)[V], T sign, int64_t below, int64_t i, int o, int64_t n,
+    const int32_t *__restrict__ col, const H *__restrict__ val, const T *X) {
+#pragma unroll 1
+  for (int j = 0; j < kSlots; ++j) {
+    const int32_t c = col[(int64_t)j * n + i];
+    const T a = (T)val[(int64_t)j * n + i];
+#pragma unroll
+    for (int k = 0; k < V; ++k) y[k] += sign * (a * (c < below ? X[(int64_t)c * S + o + k] : (T)0));
+  }
+}
+
+// Stores a colour step's result, mixed.hip's gs32_keep for each column.
+template <int S>
+__device__ __attribute__((always_inline)) inline void bgs32_keep(
+    float (&z)[4], int64_t below, int64_t i, int o, int64_t n, const int32_t *__restrict__ col,
+    const half_t *__restrict__ val16, float d, const float *__restrict__ R, float *X) {
+  if (spoilt(z)) {
+    ldv<4>(R + i * S + o, z);
+    row_again<S>(z, -1.0f, below, i, o, n, col, val16, X);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) z[k] = z[k] / d;
+  }
+  stv<4>(X + i * S + o, z);
+}
+
 // Row i, columns [o, o + 4): mixed.hip's gs32_row for each column.  Always
 // inlined: with the x-sharing kernels calling it too the compiler made it a
 // function of its own, and a call per row took the colour step from 99 to
@@ -219,7 +247,7 @@ __device__ __attribute__((always_inline)) inline void bgs32_row(int64_t i, int o
   const float d = diag32[i];
 #pragma unroll
   for (int k = 0; k < V; ++k) sum[k] = sum[k] / d;
-  stv<V>(X + i * S + o, sum);
+  bgs32_keep<S>(sum, n, i, o, n, col, val16, d, R, X);
 }
 
 // ---- the first forward sweep of a block V-cycle level from X = 0 ----------
@@ -290,7 +318,7 @@ __device__ __attribute__((always_inline)) inline void bgs32_row_zero(
   const float d = diag32[i];
 #pragma unroll
   for (int k = 0; k < V; ++k) sum[k] = sum[k] / d;
-  stv<V>(X + i * S + o, sum);
+  bgs32_keep<S>(sum, begin, i, o, n, col, val16, d, R, X);
 }
 
 // bgs32_row_zero over the live slots only (tune key "zero_live"): kRecLive's
@@ -376,7 +404,7 @@ __device__ __attribute__((always_inline)) inline void bgs32_row_zero_live(
   const float d = diag32[i];
 #pragma unroll
   for (int k = 0; k < V; ++k) sum[k] = sum[k] / d;
-  stv<V>(X + i * S + o, sum);
+  bgs32_keep<S>(sum, begin, i, o, n, col, val16, d, R, X);
 }
 
 // A colour step of the first forward sweep from X = 0, rows [begin, end)
@@ -414,10 +442,10 @@ __device__ inline bool bpairs_tile(const Col16 &C, int t) { return C.pairs(C.fla
 // the compiler hoists every triple's loads above the lane moves and needs
 // some 180 registers.
 template <bool STREAM, int S>
-__device__ __attribute__((always_inline)) inline void bgs32_row_pairs(int64_t i, int o, int64_t n, const Col16 &C,
-                                       const uint32_t *__restrict__ vc,
-                                       const float *__restrict__ diag32,
-                                       const float *__restrict__ R, float *X) {
+__device__ __attribute__((always_inline)) inline void bgs32_row_pairs(
+    int64_t i, int o, int64_t n, const Col16 &C, const uint32_t *__restrict__ vc,
+    const int32_t *__restrict__ col, const half_t *__restrict__ val16,
+    const float *__restrict__ diag32, const float *__restrict__ R, float *X) {
   constexpr int V = 4, W = S / 4, ROWS = 64 / W;
   const int t = C.tile(i);
   const int32_t *__restrict__ base = C.bases(t);
@@ -452,7 +480,7 @@ __device__ __attribute__((always_inline)) inline void bgs32_row_pairs(int64_t i,
   const float d = diag32[i];
 #pragma unroll
   for (int k = 0; k < V; ++k) sum[k] = sum[k] / d;
-  stv<V>(X + i * S + o, sum);
+  bgs32_keep<S>(sum, n, i, o, n, col, val16, d, R, X);
 }
 
 // One colour step, rows [begin, end) (begin a colour's first row when C16).
@@ -472,7 +500,7 @@ void k_bgs32_rows(int64_t begin, int64_t end, int64_t n, Col16 C, const uint32_t
     // the wavefront's first row; all its 64 / W rows present (uniform)
     const int64_t i0 = begin + (g & ~(int64_t)63) / W;
     if (i0 + 64 / W <= end && bpairs_tile(C, C.tile(i0))) {
-      bgs32_row_pairs<STREAM, S>(i, (int)(g % W) * 4, n, C, vc, diag32, R, X);
+      bgs32_row_pairs<STREAM, S>(i, (int)(g % W) * 4, n, C, vc, col, val16, diag32, R, X);
       return;
     }
   }
@@ -506,6 +534,13 @@ __global__ __launch_bounds__(kBlock) void k_bresid_restrict32_rows(
   ldv<V>(XF + f * S + o, xv);
 #pragma unroll
   for (int k = 0; k < V; ++k) a[k] += d * xv[k];
+  if (spoilt(a)) {
+#pragma unroll
+    for (int k = 0; k < V; ++k) a[k] = 0.0f;
+    row_again<S>(a, 1.0f, n, f, o, n, col, val16, XF);
+#pragma unroll
+    for (int k = 0; k < V; ++k) a[k] += d * XF[f * S + o + k];
+  }
   float rf[V];
   ldv<V>(RF + f * S + o, rf);
 #pragma unroll
@@ -561,6 +596,11 @@ __device__ inline void bspmv_row(int64_t i, int o, int64_t n, const Col16 &C,
 #pragma unroll
                                  for (int k = 0; k < V; ++k) y[k] += a * xv[k];
                                });
+    if (spoilt(y)) {
+#pragma unroll
+      for (int k = 0; k < V; ++k) y[k] = 0.0;
+      row_again<S>(y, 1.0, n, i, o, n, col, val, X);
+    }
   } else {
 #pragma unroll
     for (int j = 0; j < kSlots; ++j) {

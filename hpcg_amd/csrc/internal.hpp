@@ -222,8 +222,8 @@ struct Level {
   //   kTile16: base[j] + col16[j * n + i]
   //   kTile32: col[j * n + i] (more than 27 distinct offsets, or a slot
   //            spanning more than 65535 columns)
-  // `col` holds the 32-bit ids of every tile, col16 those of every 8- and
-  // 16-bit tile.  Tile t's record, trec[t * kBaseStride ..], one 128-byte line
+  // `col` holds the 32-bit ids of every tile, the row itself in a slot that it
+  // does not use; col16 the narrow ones of every 8- and 16-bit tile.  Tile t's record, trec[t * kBaseStride ..], one 128-byte line
   // that a wavefront reads with a few scalar loads: the 27 bases, then
   // kRecFlags (class | affine bits << 8 | pairs << 16) and kRecLive.  One line
   // for everything matters on small levels, whose steps are a chain of memory
@@ -496,6 +496,28 @@ constexpr int64_t kDeepRows = (int64_t)6 << 20;
 __device__ inline int64_t window_block(int64_t b, int64_t G) {
   const int64_t q = b % (8 * kWin), w = b - q;
   return w + 8 * kWin <= G ? w + (q % 8) * kWin + q / 8 : b;
+}
+
+// In a slot that a row does not use, the narrow column ids (and the panels of
+// lex.hip) make it multiply some other row's x by 0, which is NaN where that x is
+// not finite.  So the results of a wavefront's rows stand if they are finite;
+// otherwise its rows are summed again without those products (the 32-bit columns
+// of unused slots are the row itself), and a NaN or an infinity reaches only rows
+// that couple to it.
+// (True for a whole wavefront, so that the branch is one of its own, out of line.)
+constexpr int kNotFinite = 0x207;  // classes of v_cmp_class: NaNs and infinities
+__device__ inline bool not_finite(double v) { return __builtin_amdgcn_class(v, kNotFinite); }
+__device__ inline bool not_finite(float v) { return __builtin_amdgcn_classf(v, kNotFinite); }
+template <class T>
+__device__ inline bool spoilt(T v) {
+  return __builtin_expect(__ballot(not_finite(v)) != 0ull, 0);
+}
+template <class T, int V>
+__device__ inline bool spoilt(const T (&v)[V]) {
+  bool bad = false;
+#pragma unroll
+  for (int k = 0; k < V; ++k) bad = bad || not_finite(v[k]);
+  return __builtin_expect(__ballot(bad) != 0ull, 0);
 }
 
 // Offset word g of row i (the place-th of its tile) on a kTile8 tile: loaded,

@@ -210,6 +210,34 @@ __device__ inline double gs_row(int64_t i, int64_t n,
   return sum / d;
 }
 
+// What the narrow rows below fall back to (spoilt): the row summed again from the
+// 32-bit columns.  Loops of one slot, to hold few registers.
+__device__ inline double row_dot_again(const int32_t *__restrict__ col,
+                                       const double *__restrict__ val,
+                                       const double *__restrict__ x, int64_t n, int64_t i) {
+  double sum = 0.0;
+#pragma unroll 1
+  for (int j = 0; j < kSlots; ++j) sum += val[(int64_t)j * n + i] * x[col[(int64_t)j * n + i]];
+  return sum;
+}
+
+// The new x_i, from its own value xi and, of x, only what lies below `below`
+// (0 for the rest).
+__device__ inline double gs_again(const int32_t *__restrict__ col, const double *__restrict__ val,
+                                  const double *__restrict__ r, const double *x, double xi,
+                                  int64_t below, int64_t n, int64_t i) {
+  double sum = r[i], d = 0.0;
+#pragma unroll 1
+  for (int j = 0; j < kSlots; ++j) {
+    const double v = val[(int64_t)j * n + i];
+    const int32_t c = col[(int64_t)j * n + i];
+    sum -= v * (c == i ? xi : c < below ? x[c] : 0.0);
+    if (c == i && v != 0.0) d = v;
+  }
+  sum += xi * d;
+  return sum / d;
+}
+
 // Narrow column ids (Level::trec).  The caller's wavefront lies in one tile,
 // so the tile id and its record are uniform (read through the scalar cache).
 // narrow_row() calls f(j, k, c) for every slot j in order, with k = j*n + i
@@ -294,12 +322,12 @@ __device__ inline double row_dot16(const Col16 &C, const int32_t *__restrict__ c
     affine_pairs_row(C, t, n, i, x, [&](int, int64_t k, int32_t, double xc) {
       sum += mload<STREAM>(val + k) * xc;
     });
-    return sum;
+  } else {
+    narrow_row<STREAM>(C, t, flags, n, i, [&](int, int64_t k, int32_t c) {
+      sum += mload<STREAM>(val + k) * x[c];
+    });
   }
-  narrow_row<STREAM>(C, t, flags, n, i, [&](int, int64_t k, int32_t c) {
-    sum += mload<STREAM>(val + k) * x[c];
-  });
-  return sum;
+  return spoilt(sum) ? row_dot_again(col, val, x, n, i) : sum;
 }
 
 template <bool STREAM, bool PAIRS = false>
@@ -323,18 +351,18 @@ __device__ inline double gs_row16(const Col16 &C, int64_t i, int64_t n,
       }
     });
     sum += xi * d;
-    x[i] = sum / d;
-    return sum / d;
   } else {
     narrow_row<STREAM>(C, t, flags, n, i, [&](int, int64_t k, int32_t c) {
       const double v = mload<STREAM>(val + k);
       sum -= v * x[c];
       if (c == i && v != 0.0) d = v;
     });
+    sum += x[i] * d;
   }
-  sum += x[i] * d;
-  x[i] = sum / d;
-  return sum / d;
+  double z = sum / d;
+  if (spoilt(z)) z = gs_again(col, val, r, x, x[i], n, n, i);
+  x[i] = z;
+  return z;
 }
 
 // All rows of one colour (a contiguous device-order range) at once: rows of
@@ -445,7 +473,8 @@ __device__ inline double gs_row_deep(const Col16 &C, int64_t i, int64_t n,
 #pragma unroll
   for (int j = 0; j < kSlots; ++j) sum -= v[j] * xs[j];
   sum += xi * d;
-  const double z = sum / d;
+  double z = sum / d;
+  if (spoilt(z)) z = gs_again(col, val, r, x, x[i], n, n, i);
   x[i] = z;
   return z;
 }
@@ -569,7 +598,9 @@ __device__ inline void gs_row_zero(const Col16 &C, uint32_t zm, int64_t begin, i
   }
   const double d = mload<STREAM>(diag + i);
   sum += 0.0 * d;
-  x[i] = sum / d;
+  double z = sum / d;
+  if (spoilt(z)) z = gs_again(col, val, r, x, 0.0, begin, n, i);
+  x[i] = z;
 }
 
 // The turn of a symmetric sweep: the last colour's forward step and the first
@@ -641,8 +672,14 @@ __device__ inline double gs_row_turn(const Col16 &C, int64_t begin, int64_t i, i
 #pragma unroll
   for (int j = 0; j < kSlots; ++j) sum -= j == ds ? zd : xs[j];
   sum += zd;
-  x[i] = sum / d;
-  return sum / d;
+  double z2 = sum / d;
+  if (spoilt(z2)) {
+    const int64_t below = ZERO ? begin : n;
+    z2 = gs_again(col, val, r, x, ZERO ? 0.0 : x[i], below, n, i);
+    z2 = gs_again(col, val, r, x, z2, below, n, i);
+  }
+  x[i] = z2;
+  return z2;
 }
 
 // RZ: also the r.z partials of the backward step, as k_gs_rz16.
@@ -752,7 +789,9 @@ __device__ inline void gs_row_zero_live(const Col16 &C, int64_t begin, int64_t i
     sum = zero_live_sum<STREAM, 3, CH>(C, zm, t, tb, lane, xlim, n, col, val, x, sum);
   const double d = mload<STREAM>(diag + i);
   sum += 0.0 * d;
-  x[i] = sum / d;
+  double z = sum / d;
+  if (spoilt(z)) z = gs_again(col, val, r, x, 0.0, begin, n, i);
+  x[i] = z;
 }
 
 // LIVE: the live slots only (gs_row_zero_live), else every slot (gs_row_zero)
@@ -1182,12 +1221,11 @@ __global__ __launch_bounds__(kBlock) void k_spmv_dot_c(
 // Row i of A p in FP64 from the FP16 off-diagonal values (packed words)
 // and the FP64 diagonal, in slot order; 32-bit tiles read the FP64 matrix.
 template <bool STREAM>
-__device__ inline double row_dot_h(const Col16 &C, const uint32_t *__restrict__ vc,
-                                   const uint8_t *__restrict__ dslot,
-                                   const double *__restrict__ diag,
-                                   const int32_t *__restrict__ col,
-                                   const double *__restrict__ val,
-                                   const double *__restrict__ p, int64_t n, int64_t i) {
+__device__ inline double h_sum(const Col16 &C, const uint32_t *__restrict__ vc,
+                               const uint8_t *__restrict__ dslot,
+                               const double *__restrict__ diag, const int32_t *__restrict__ col,
+                               const double *__restrict__ val, const double *__restrict__ p,
+                               int64_t n, int64_t i) {
   const int t = C.tile(i);
   if ((C.flags(t) & 3u) == kTile32) return row_dot<STREAM>(col, val, p, n, i);
   const int32_t *__restrict__ base = C.bases(t);
@@ -1204,22 +1242,32 @@ __device__ inline double row_dot_h(const Col16 &C, const uint32_t *__restrict__ 
   return y;
 }
 
+template <bool STREAM>
+__device__ inline double row_dot_h(const Col16 &C, const uint32_t *__restrict__ vc,
+                                   const uint8_t *__restrict__ dslot,
+                                   const double *__restrict__ diag,
+                                   const int32_t *__restrict__ col,
+                                   const double *__restrict__ val,
+                                   const double *__restrict__ p, int64_t n, int64_t i) {
+  const double y = h_sum<STREAM>(C, vc, dslot, diag, col, val, p, n, i);
+  return spoilt(y) ? row_dot_again(col, val, p, n, i) : y;
+}
+
 // row_dot_h on an 8-bit tile from the FP16 value pairs (vp, kPairWords words)
 // and the 8-bit offsets (none loaded where the tile's words are affine):
 // the same FP16 values, columns and slot order, 2 to 3 bytes per slot in
 // place of 4.  Other tiles take row_dot_h.
 template <bool STREAM>
-__device__ inline double row_dot_hp(const Col16 &C, const uint32_t *__restrict__ vp,
-                                    const uint32_t *__restrict__ vc,
-                                    const uint8_t *__restrict__ dslot,
-                                    const double *__restrict__ diag,
-                                    const int32_t *__restrict__ col,
-                                    const double *__restrict__ val,
-                                    const double *__restrict__ p, int64_t n, int64_t i,
-                                    int64_t end) {
+__device__ inline double hp_sum(const Col16 &C, const uint32_t *__restrict__ vp,
+                                const uint32_t *__restrict__ vc,
+                                const uint8_t *__restrict__ dslot,
+                                const double *__restrict__ diag,
+                                const int32_t *__restrict__ col,
+                                const double *__restrict__ val, const double *__restrict__ p,
+                                int64_t n, int64_t i, int64_t end) {
   const int t = C.tile(i);
   const uint32_t flags = C.flags(t);
-  if (C.cls(flags) != kTile8) return row_dot_h<STREAM>(C, vc, dslot, diag, col, val, p, n, i);
+  if (C.cls(flags) != kTile8) return h_sum<STREAM>(C, vc, dslot, diag, col, val, p, n, i);
   const int32_t *__restrict__ base = C.bases(t);
   const unsigned words = C.words(flags);
   const int place = C.place(i);
@@ -1278,6 +1326,19 @@ __device__ inline double row_dot_hp(const Col16 &C, const uint32_t *__restrict__
     y += a * p[c];
   }
   return y;
+}
+
+template <bool STREAM>
+__device__ inline double row_dot_hp(const Col16 &C, const uint32_t *__restrict__ vp,
+                                    const uint32_t *__restrict__ vc,
+                                    const uint8_t *__restrict__ dslot,
+                                    const double *__restrict__ diag,
+                                    const int32_t *__restrict__ col,
+                                    const double *__restrict__ val,
+                                    const double *__restrict__ p, int64_t n, int64_t i,
+                                    int64_t end) {
+  const double y = hp_sum<STREAM>(C, vp, vc, dslot, diag, col, val, p, n, i, end);
+  return spoilt(y) ? row_dot_again(col, val, p, n, i) : y;
 }
 
 // k_spmv_dot_h with one workgroup per row chunk; partials as k_spmv_dot_c.

@@ -483,12 +483,22 @@ __global__ __launch_bounds__(64 * kLexWaves) void k_lex_sweep(
       for (int j = 0; j < kLexIn; ++j)
         fresh[j] = *reinterpret_cast<const double *>(reinterpret_cast<const char *>(ring) +
                                                      G.f[j]);
+      auto xj = [&](int j) {
+        return j >= kFresh && j < kFresh + kLexIn ? fresh[j - kFresh] : j == kDiag ? M.o : G.x[j];
+      };
       double sum = M.r;
 #pragma unroll
-      for (int j = 0; j < kSlots; ++j)
-        sum -= M.v[j / 2][j % 2] * (j >= kFresh && j < kFresh + kLexIn ? fresh[j - kFresh]
-                         : j == kDiag                       ? M.o
-                                                            : G.x[j]);
+      for (int j = 0; j < kSlots; ++j) sum -= M.v[j / 2][j % 2] * xj(j);
+      // without the slots that the row does not use (such rows store no zeros);
+      // from registers: loads here would make every later step wait for them
+      if (__builtin_expect(__ballot(__builtin_amdgcn_class(sum, kNotFinite)) != 0ull, 0)) {
+        sum = M.r;
+#pragma unroll
+        for (int j = 0; j < kSlots; ++j) {
+          const double v = M.v[j / 2][j % 2];
+          sum -= v * (j != kDiag && v == 0.0 ? 0.0 : xj(j));
+        }
+      }
       finish(S, sum, M.o, M.v[kSlots / 2][1]);
     } else {
       const uint32_t ln = lane_of(S);

@@ -122,6 +122,39 @@ __device__ inline float row_dot32(int64_t i, int64_t n,
   return s;
 }
 
+// kernels.hip's gs_again and row_dot_again in FP32, where the narrow row's result
+// is spoilt; gs32_keep stores it.
+__device__ inline float gs32_keep(float v, int64_t below, int64_t i, int64_t n,
+                                  const int32_t *__restrict__ col,
+                                  const half_t *__restrict__ val16,
+                                  const float *__restrict__ diag32,
+                                  const float *__restrict__ r, float *x) {
+  if (spoilt(v)) {
+    float sum = r[i];
+#pragma unroll 1
+    for (int j = 0; j < kSlots; ++j) {
+      const int32_t c = col[(int64_t)j * n + i];
+      sum -= (float)val16[(int64_t)j * n + i] * (c < below ? x[c] : 0.0f);
+    }
+    v = sum / diag32[i];
+  }
+  x[i] = v;
+  return v;
+}
+
+__device__ inline float row_dot32_keep(float s, int64_t i, int64_t n,
+                                       const int32_t *__restrict__ col,
+                                       const half_t *__restrict__ val16,
+                                       const float *__restrict__ diag32,
+                                       const float *__restrict__ x) {
+  if (!spoilt(s)) return s;
+  s = 0.0f;
+#pragma unroll 1
+  for (int j = 0; j < kSlots; ++j)
+    s += (float)val16[(int64_t)j * n + i] * x[col[(int64_t)j * n + i]];
+  return s + diag32[i] * x[i];
+}
+
 // Narrow column ids (Level::trec): the caller's wavefront lies in one tile.
 //
 // Entry of a narrow tile packed in one 32-bit word (Level::vc):
@@ -148,9 +181,7 @@ __device__ inline float gs32_row16(const Col16 &C, const uint32_t *__restrict__ 
     const int32_t c = base[j] + (int32_t)(w >> 16);
     sum -= (float)vc_val(w) * x[c];
   }
-  const float v = sum / diag32[i];
-  x[i] = v;
-  return v;
+  return gs32_keep(sum / diag32[i], n, i, n, col, val16, diag32, r, x);
 }
 
 template <bool STREAM>
@@ -170,7 +201,7 @@ __device__ inline float row_dot32_16(const Col16 &C, const uint32_t *__restrict_
     s += (float)vc_val(w) * x[c];
   }
   s += diag32[i] * x[i];
-  return s;
+  return row_dot32_keep(s, i, n, col, val16, diag32, x);
 }
 
 // Whether row i's wavefront can share x windows between slots 3m and 3m + 2:
@@ -213,9 +244,7 @@ __device__ inline float gs32_row8(const Col16 &C, const uint32_t *__restrict__ v
       const half_t a = __builtin_bit_cast(half_t, (uint16_t)(pv[j / 2] >> (16 * (j % 2))));
       sum -= (float)a * xs[j];
     }
-    const float v = sum / di;
-    x[i] = v;
-    return v;
+    return gs32_keep(sum / di, n, i, n, col, val16, diag32, r, x);
   }
 #pragma unroll
   for (int g = 0; g < kSlotWords; ++g) o8[g] = off8_word<STREAM>(C.off8, words, g, n, i, pos);
@@ -249,9 +278,7 @@ __device__ inline float gs32_row8(const Col16 &C, const uint32_t *__restrict__ v
       sum -= (float)a * x[c];
     }
   }
-  const float v = sum / diag32[i];
-  x[i] = v;
-  return v;
+  return gs32_keep(sum / diag32[i], n, i, n, col, val16, diag32, r, x);
 }
 
 // row_dot32_16 on an 8-bit tile from the FP16 value pairs (gs32_row8's
@@ -282,7 +309,7 @@ __device__ inline float row_dot32_8(const Col16 &C, const uint32_t *__restrict__
     s += (float)a * x[c];
   }
   s += diag32[i] * x[i];
-  return s;
+  return row_dot32_keep(s, i, n, col, val16, diag32, x);
 }
 
 // The first forward sweep of an FP32 V-cycle level from x = 0: the FP32
@@ -370,7 +397,7 @@ __device__ inline void gs32_row_zero(const Col16 &C, uint32_t zm, int64_t begin,
       sum -= (float)a * buf_f32(buf_view(x, live ? xlim : 0u), (uint32_t)c * 4u);
     }
   }
-  x[i] = sum / diag32[i];
+  gs32_keep(sum / diag32[i], begin, i, n, col, val16, diag32, r, x);
 }
 
 // gs32_row_zero over the live slots only (tune key "zero_live"): kRecLive's
@@ -475,7 +502,7 @@ __device__ inline void gs32_row_zero_live(const Col16 &C, int64_t begin,
     sum = zero_live_sum32<STREAM, 1, CH>(C, zm, t, tb, lane, xlim, n, vp, vc, col, val16, x, sum);
   else
     sum = zero_live_sum32<STREAM, 0, CH>(C, zm, t, tb, lane, xlim, n, vp, vc, col, val16, x, sum);
-  x[i] = sum / diag32[i];
+  gs32_keep(sum / diag32[i], begin, i, n, col, val16, diag32, r, x);
 }
 
 // v16p[w*n + i] = bits of val16[(2w)*n + i] | bits of val16[(2w+1)*n + i] << 16

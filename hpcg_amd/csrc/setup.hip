@@ -356,7 +356,8 @@ __global__ __launch_bounds__(kBlock) void k_tile_rows(int64_t T, int ncolors,
 //     overwritten before it is read); a row without an entry in a slot gets
 //     the value 0 and a valid column: where the slot's entries all lie at one
 //     base plus their row's place in the tile, the column at that place too
-//     (the slot is then affine), else one already in the slot's range.  The
+//     (the slot is then affine), else one already in the slot's range; its
+//     32-bit column is the row itself.  The
 //     slot's base is its smallest column.  The tile's class: 8-bit offsets if
 //     every slot spans at most 255 columns, 16-bit if at most 65535, else (or
 //     with more than 27 distinct offsets) 32-bit ids only.
@@ -434,7 +435,8 @@ __global__ __launch_bounds__(kBlock) void k_tile_layout(
     if (used && hi - lo > 255) narrow8 = false;
     const int32_t base = used || window ? lo : first;
     if (row) {
-      col[(int64_t)u * n + i] = cc;
+      // (the row itself where it has no entry: see spoilt, internal.hpp)
+      col[(int64_t)u * n + i] = has ? c : (int32_t)i;
       val[(int64_t)u * n + i] = has ? v : 0.0;
       col16[(int64_t)u * n + i] = (uint16_t)(cc - base);
       o8[u / 4] |= ((uint32_t)(cc - base) & 0xffu) << (8 * (u % 4));

@@ -216,8 +216,19 @@ __global__ __launch_bounds__(64 * kTailWaves) void k_tail(const TailArgs<V, T> A
         const T xi = x[i];
         sum = terms<V, T>(sum, v, [&](int j) { return x[cj[j]]; });
         if (F64) sum += xi * d;
-        const T z = sum / d;
+        T z = sum / d;
         if (row) x[i] = z;
+        if (spoilt(sum)) {  // (after the store, which the next step waits for)
+          sum = ri;
+#pragma unroll 1
+          for (int j = 0; j < kSlots; ++j) {
+            const int32_t c = L.col[(int64_t)j * L.n + i];
+            sum -= (T)L.val[(int64_t)j * L.n + i] * (c == i ? xi : x[c]);
+          }
+          if (F64) sum += xi * d;
+          z = sum / d;
+          if (row) x[i] = z;
+        }
         if (s >= rz_from) {
           double p = 0.0;
           if (row) p = F64 ? (double)(ri * z) : A.r64[i] * (double)z;
