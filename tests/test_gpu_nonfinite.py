@@ -98,20 +98,26 @@ def sweeps(P, r, x):
     z = torch.empty_like(y)
     P.mg32(r.float(), z, ordering="multicolor")
     out += [y, z]
-    R = torch.stack([r, r * 0.5, x, r - x], dim=1).float().contiguous()
-    Z = torch.empty_like(R)
-    P.mg32_block(R, Z, ordering="multicolor")
+    for s in (2, 4, 8):
+        R = torch.stack([r, r * 0.5, x, r - x] * 2, dim=1)[:, :s].float().contiguous()
+        Z = torch.empty_like(R)
+        P.mg32_block(R, Z, ordering="multicolor")
+        out.append(Z)
     P.check()
-    return out + [Z]
+    return out
 
 
-@pytest.mark.parametrize("zero_live", [11, 4, 0])
+@pytest.mark.parametrize("knobs", [{"zero_live": 11}, {"zero_live": 4}, {"zero_live": 0},
+                                   {"col8": 0}, {"affine8": 0}, {"fp16_pairs": 0}, {"turn": 0},
+                                   {"zero_guess": 0},
+                                   {"x_pairs": 15, "block_pairs": 1, "stream_min_bytes": 0}])
 @pytest.mark.parametrize("dims,levels", [((16, 16, 16), 2), ((32, 32, 32), 3), ((33, 31, 29), 1),
                                          ((36, 20, 28), 3), ((64, 64, 8), 2)])
-def test_sweeps_as_by_32bit_columns(hp, dims, levels, zero_live):
+def test_sweeps_as_by_32bit_columns(hp, dims, levels, knobs):
     import torch
     P = hp.Problem.generate(*dims, nlevels=levels)
-    P.tune("zero_live", zero_live)
+    for key, value in knobs.items():
+        P.tune(key, value)
     n = P.nrow(0)
     g = torch.Generator(device="cuda")
     g.manual_seed(7)
