@@ -26,8 +26,9 @@
 // offset, so that both the stored entries and the gathered x of a wavefront
 // are consecutive.  x and r are permuted into the same order for the sweep.
 //
-// Measured (MI355X, one V-cycle in reference order): 256^3 439.2 -> 23.9 ms,
-// 64x48x32 21.7 -> 2.56 ms.  What bounds it now is the chain of hyperplanes:
+// Measured (MI355X, one V-cycle in reference order): 256^3 439.2 -> 24.4 ms,
+// 64x48x32 21.7 -> 2.54 ms (the first, which builds the copy, 155 and 5.1 ms).
+// What bounds it now is the chain of hyperplanes:
 // about 1.1 us a step (one wavefront a panel) to 1.5 us (two), for gathers
 // behind the barrier, 27 dependent subtractions and a division, over
 // (hyperplanes of a panel) + 7 (panels - 1) steps: each panel starts four

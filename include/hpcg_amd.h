@@ -485,7 +485,9 @@ int hpcgx_cg_fleet(hpcgx_problem *p, int ordering, const double *b, double *x, i
  *                      colour in one launch (FP64), or one of them where the
  *                      second repeats the first (FP32, whose update does not
  *                      read the row's own x).  hpcgx_kernel_timing does not
- *                      log that launch (default 1; the same bits)
+ *                      log that launch (default 1; the same bits, but for an
+ *                      FP32 x that overflows: the second update would make
+ *                      its infinity a NaN)
  *   "block_pairs"      1/0: the block PCG's finest colour steps at s = 8,
  *                      on tiles where "x_pairs" applies, take slot 3m + 2's
  *                      neighbour rows from slot 3m's moved one row (2
