@@ -211,10 +211,14 @@ __device__ inline double gs_row(int64_t i, int64_t n,
 }
 
 // What the narrow rows below fall back to (spoilt): the row summed again from the
-// 32-bit columns.  Loops of one slot, to hold few registers.
+// 32-bit columns.  Loops of one slot, to hold few registers, and the row passes
+// through an empty asm: else its addresses are formed before the fast sum and
+// stay in registers, of which the capped steps then spill six (512^3 without
+// x_pairs, one level, four iterations: 83.4 to 84.3 ms, 85.1 to 85.7 with them).
 __device__ inline double row_dot_again(const int32_t *__restrict__ col,
                                        const double *__restrict__ val,
                                        const double *__restrict__ x, int64_t n, int64_t i) {
+  asm volatile("" : "+v"(i));
   double sum = 0.0;
 #pragma unroll 1
   for (int j = 0; j < kSlots; ++j) sum += val[(int64_t)j * n + i] * x[col[(int64_t)j * n + i]];
@@ -226,6 +230,7 @@ __device__ inline double row_dot_again(const int32_t *__restrict__ col,
 __device__ inline double gs_again(const int32_t *__restrict__ col, const double *__restrict__ val,
                                   const double *__restrict__ r, const double *x, double xi,
                                   int64_t below, int64_t n, int64_t i) {
+  asm volatile("" : "+v"(i));
   double sum = r[i], d = 0.0;
 #pragma unroll 1
   for (int j = 0; j < kSlots; ++j) {
